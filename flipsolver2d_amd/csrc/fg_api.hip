@@ -334,8 +334,11 @@ void carve(fg_scene* s, Carver& cv)
     h.sid = cv.take<int32_t>(C);
     h.pcount = cv.take<int32_t>(C);
     h.marker = cv.take<int32_t>(C);
-    h.lsFlags = cv.take<int32_t>(kMaxBands);
-    h.lsTile = cv.take<uint8_t>(2 * cdiv(s->I, kBfsTile) * cdiv(s->J, kBfsTile));
+    const int64_t bfs_tiles = cdiv(s->I, kBfsTile) * cdiv(s->J, kBfsTile);
+    h.lsFlags = cv.take<int32_t>(kMaxBands + 1);
+    h.lsTile = cv.take<uint8_t>(bfs_tiles);
+    h.lsStamp = cv.take<int32_t>(bfs_tiles);
+    h.lsQueue = cv.take<int32_t>(2 * bfs_tiles);
     h.u = cv.take<float>(FU);
     h.su = cv.take<float>(FU);
     h.uf = cv.take<float>(FU);
@@ -629,7 +632,7 @@ __global__ void k_gather_scalars(const SceneDev* scenes, int n, SceneScalars* ou
 // Group-wide flags for the host's polls:
 //   out[0]: some scene's solve has not met its FP64 tolerance
 //   out[1]: some scene's inner PCG is still iterating
-//   out[2]: some scene's level-set band `band` reached its last level
+//   out[2]: some scene's level-set band `band` reached its last level (it queued tiles for the next)
 __global__ void k_group_flags(const SceneDev* scenes, int n, int band, int32_t* out)
 {
     __shared__ int any[3];
@@ -644,7 +647,7 @@ __global__ void k_group_flags(const SceneDev* scenes, int n, int band, int32_t* 
                 any[0] = 1;
                 if (!sc->inner_done) any[1] = 1;
             }
-        } else if (s.lsFlags[band]) {
+        } else if (s.lsFlags[band + 1]) {
             any[2] = 1;
         }
     }

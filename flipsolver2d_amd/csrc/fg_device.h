@@ -168,9 +168,10 @@ struct SceneDev {
     int32_t* sid;
     int32_t* pcount;
     int32_t* marker;        // level-set BFS levels
-    int32_t* lsFlags;       // [kMaxBands] band reached its last level
-    uint8_t* lsTile;        // [2][BFS tiles] by band parity: the tile reached its band's last level
-                            // (band 0 reads the tiles holding a known cell)
+    int32_t* lsFlags;       // [kMaxBands + 1]: tiles that band b-1 queued for band b (it reached its last level there)
+    uint8_t* lsTile;        // [BFS tiles]: the tile holds a known cell
+    int32_t* lsStamp;       // [BFS tiles]: the last band the tile was queued for
+    int32_t* lsQueue;       // [2][BFS tiles] by band parity: the band's tiles
     // faces: working (P2G/project), saved (extrapolated, pre-force), final
     float *u, *v, *su, *sv, *uf, *vf;
     uint8_t *uval, *vval, *uvalS, *vvalS, *uvalF, *vvalF;

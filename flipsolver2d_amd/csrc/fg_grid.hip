@@ -4,6 +4,8 @@
 // I x (J+1) (FlipSolver2dLib/staggeredvelocitygrid.cpp:6-14).  One thread
 // per cell; blocks of a launch are remapped so each XCD gets a contiguous
 // band of rows.
+#include <algorithm>
+
 #include "fg_kernels.h"
 
 namespace fg {
@@ -411,262 +413,282 @@ __global__ void __launch_bounds__(kBlock) k_sdf_exact(const SceneDev* scenes)
 // ---------------------------------------------------------------------------
 constexpr int kTile = 32;
 static_assert(kTile == kBfsTile, "the host sizes the BFS launches and tile flags by kBfsTile");
-constexpr int16_t kNone = 0x7fff;     // outside the grid
-constexpr int16_t kUnreached = 0x7ffe;
 
-// Levels are expanded as row bitmasks (the region is at most 64 cells
-// wide): one wave holds one region row per lane, dilates the frontier of
-// level L with shifts and lane shuffles, and removes the reached set, so the
-// expansion costs a few instructions per row and level and needs no
-// barrier.  The value pass then visits only the cells of each level.
+// A lane's value from the lane below / above it, 0 past the wave's ends (a
+// DPP move over the whole wave, no LDS permute).
+__device__ __forceinline__ unsigned long long lane_below(unsigned long long v)
+{
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, 0x138, 0xf, 0xf, true);          // wave_shr:1
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), 0x138, 0xf, 0xf, true);
+    return ((unsigned long long)hi << 32) | lo;
+}
+__device__ __forceinline__ unsigned long long lane_above(unsigned long long v)
+{
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, 0x130, 0xf, 0xf, true);          // wave_shl:1
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), 0x130, 0xf, 0xf, true);
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// One band in one tile (any tile: the block's, or one of a queue).  A working
+// tile is a latency chain (few tiles work at a time, one to a CU), so
+// everything that does not depend on a value is taken out of the level loop:
+//   rows      a wave loads whole region rows (lane = column), so the rows'
+//             bitmasks (known, level L0) are ballots of the loads;
+//   expansion lane = region row (the region is at most 64 cells wide): the
+//             frontier of each level by shifts and whole-wave DPP moves, no
+//             barrier.  Every wave does it, so no wave waits for another's;
+//             wave w lists the cells of the levels st = w (mod 4): row,
+//             column and the 8-bit mask of the neighbours of a lower level
+//             (bits of the set reached one level before).  A row of up to
+//             kShortRow cells is its lane's, a longer one the whole wave's
+//             (lane = column);
+//   values    level by level, a thread a cell: its list entry (read a level
+//             ahead), eight neighbours' values, the FP64 sum of the masked
+//             ones, the store to LDS and to global memory; one barrier.
+// In the block at 1024^2 a full 16-level band takes 23,000 cycles (load and
+// row masks 6,000, expansion and lists 6,000, values 8,000-12,000), 33,000
+// with each level's cells searched in the row masks inside the level loop
+// and the quotient by a division.
+constexpr int kShortRow = 6;   // a vertical or slanted front leaves one or two cells a row; 6 bounds the lanes' loop
 template <int H, bool LEVELSET, bool OUT = false>
-__device__ void bfs_band(const float* gin, const uint8_t* vin, const int32_t* mkin, float* gout, uint8_t* vout,
-                         int32_t* mkout, int si, int sj, int L0, int* more, uint8_t* tile_more)
+__device__ bool bfs_band(int tile, const float* gin, const uint8_t* vin, const int32_t* mkin, float* gout, uint8_t* vout,
+                         int32_t* mkout, int si, int sj, int L0)
 {
     constexpr int R = kTile + 2 * H;
     static_assert(R <= 64, "a region row must fit one 64-bit mask");
-    // LDS row strides chosen so that the cells of a region column (a level's
-    // vertical side, visited by consecutive threads) fall in different banks:
-    // an odd number of words per row, for the floats and for the int16
-    // markers (two to a word)
-    constexpr int RS = R + 1;
-    constexpr int RSM = ((R + 2) / 2) % 2 == 1 ? R + 2 : R + 4;
-    constexpr int T = 16;   // threads as a 16 x 16 layout for the load and store passes
-    __shared__ int16_t mk[R * RSM];
-    __shared__ float val[R * RS];
-    __shared__ unsigned long long front[H + 1][R];   // front[s]: region cells at level L0 + s
-    __shared__ unsigned long long open_s[R];
-    __shared__ int16_t pre[H + 1][64];                // row offsets of level L0+s's cells
-    __shared__ int16_t tot[H + 1];
-    __shared__ int top_s;
-    const int tx = threadIdx.x & (T - 1), ty = threadIdx.x >> 4;
+    constexpr int RS = R + 1;             // odd row stride: a region column falls in different banks
+    constexpr int NW = kBlock / 64;       // waves
+    static_assert(NW == 4, "four levels a step of the expansion, one a wave");
+    constexpr int NR = (R + NW - 1) / NW; // region rows a wave loads
+    typedef unsigned long long mask_t;
+    __shared__ float vbuf[(R + 2) * RS + 2];   // a margin of one cell: neighbours of border cells are read, never used
+    __shared__ mask_t known_s[64], front_s[64], done_s[64];   // by row: known, level L0, reached by the last level
+    __shared__ int2 level_s[NW * ((H + NW - 1) / NW) + 1];    // by level: first list entry and count
+    __shared__ int cursor;
+    __shared__ uint32_t list[R * R + kBlock];  // cells by level: neighbour mask << 12 | row << 6 | column
+    __shared__ double inv[9];                  // 1 / count
+    float* const val = vbuf + RS + 1;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tilesJ = (sj + kTile - 1) / kTile;
-    const int tile = blockIdx.x;
     const int ti = tile / tilesJ, tj = tile - (tile / tilesJ) * tilesJ;
     const int gi0 = ti * kTile - H, gj0 = tj * kTile - H;
-    // the region: every load of the thread issued before any is used
-    // (clamped indices, the loads unconditional; each value is pinned by an
-    // empty asm after all of them, so none is sunk into a later branch)
-    // Extrapolation (!LEVELSET) loads the halo's values only if the tile has
-    // work: a tile with no unknown cell, or no known one within reach, is
-    // copied, and needs the region's validity bytes and its own values alone.
-    constexpr int NA = (R + T - 1) / T;
-    float xr[NA][NA];
-    int lr[NA][NA];
-    bool okr[NA][NA];
+    const int gj = gj0 + lane;
+    const bool colok = lane < R && gj >= 0 && gj < sj;
+    const int gjc = min(max(gj, 0), sj - 1);
+    const bool incol = lane >= H && lane < H + kTile;
+    // the rows: every load of the thread issued before any is used (clamped
+    // indices; each value is pinned by an empty asm after all of them, so
+    // none is sunk into a later branch).  Extrapolation (!LEVELSET) loads
+    // the halo's values only if the tile has work: a tile with no unknown
+    // cell, or no known one within reach, is copied, and needs the region's
+    // validity bytes and its own values alone.
+    float xr[NR];
+    int lr[NR];
 #pragma unroll
-    for (int a = 0; a < NA; a++)
-#pragma unroll
-        for (int b = 0; b < NA; b++) {
-            const int ri = ty + a * T, rj = tx + b * T;
-            const int gi = gi0 + ri, gj = gj0 + rj;
-            okr[a][b] = ri < R && rj < R && gi >= 0 && gi < si && gj >= 0 && gj < sj;
-            const size_t g = (size_t)min(max(gi, 0), si - 1) * sj + min(max(gj, 0), sj - 1);
-            const bool inner = ri >= H && ri < H + kTile && rj >= H && rj < H + kTile;
-            xr[a][b] = (LEVELSET || inner) ? gbl<const float>(gin)[g] : 0.f;
-            if (LEVELSET) lr[a][b] = gbl<const int32_t>(mkin)[g];
-            else lr[a][b] = (int)gbl<const uint8_t>(vin)[g];
-        }
-#pragma unroll
-    for (int a = 0; a < NA; a++)
-#pragma unroll
-        for (int b = 0; b < NA; b++) {
-            asm volatile("" : "+v"(xr[a][b]), "+v"(lr[a][b]));
-            xr[a][b] = okr[a][b] ? xr[a][b] : 0.f;
-            lr[a][b] = okr[a][b] ? lr[a][b] : -1;
-        }
-    bool has_front = false, has_open = false;
-#pragma unroll
-    for (int a = 0; a < NA; a++)
-#pragma unroll
-        for (int b = 0; b < NA; b++) {
-            const int ri = ty + a * T, rj = tx + b * T;
-            if (ri >= R || rj >= R) continue;
-            int16_t m = kNone;
-            if (lr[a][b] >= 0) {
-                if (LEVELSET) m = lr[a][b] <= L0 ? (int16_t)lr[a][b] : kUnreached;
-                else m = lr[a][b] ? 0 : kUnreached;
-            }
-            has_front |= m == L0;
-            has_open |= m == kUnreached;
-            mk[ri * RSM + rj] = m;
-            val[ri * RS + rj] = xr[a][b];
-        }
-    // a tile cell reaches level L0+s only through a level-L0 cell within
-    // distance s <= H, i.e. inside this region
-    const bool work = __syncthreads_or(has_front) && __syncthreads_or(has_open);
-    if (!LEVELSET && work) {   // the halo's values (the barriers below order these stores)
-        float hv[NA][NA];
-#pragma unroll
-        for (int a = 0; a < NA; a++)
-#pragma unroll
-            for (int b = 0; b < NA; b++) {
-                const int ri = ty + a * T, rj = tx + b * T;
-                const bool inner = ri >= H && ri < H + kTile && rj >= H && rj < H + kTile;
-                const int gi = gi0 + ri, gj = gj0 + rj;
-                const size_t g = (size_t)min(max(gi, 0), si - 1) * sj + min(max(gj, 0), sj - 1);
-                hv[a][b] = (okr[a][b] && !inner) ? gbl<const float>(gin)[g] : 0.f;
-            }
-#pragma unroll
-        for (int a = 0; a < NA; a++)
-#pragma unroll
-            for (int b = 0; b < NA; b++) {
-                const int ri = ty + a * T, rj = tx + b * T;
-                const bool inner = ri >= H && ri < H + kTile && rj >= H && rj < H + kTile;
-                if (ri < R && rj < R && !inner) val[ri * RS + rj] = hv[a][b];
-            }
+    for (int a = 0; a < NR; a++) {
+        const int ri = w + a * NW, gi = gi0 + ri;
+        const size_t g = (size_t)min(max(gi, 0), si - 1) * sj + gjc;
+        const bool inner = incol && ri >= H && ri < H + kTile;
+        xr[a] = (LEVELSET || inner) ? gbl<const float>(gin)[g] : 0.f;
+        if (LEVELSET) lr[a] = gbl<const int32_t>(mkin)[g];
+        else lr[a] = (int)gbl<const uint8_t>(vin)[g];
     }
+#pragma unroll
+    for (int a = 0; a < NR; a++) asm volatile("" : "+v"(xr[a]), "+v"(lr[a]));
+    if (threadIdx.x < 9) inv[threadIdx.x] = threadIdx.x ? 1.0 / (double)threadIdx.x : 0.0;
+    if (threadIdx.x == 9) cursor = 0;
+    if (threadIdx.x < NW * ((H + NW - 1) / NW) + 1) level_s[threadIdx.x] = make_int2(0, 0);
+    if (w == 0 && lane >= R) known_s[lane] = front_s[lane] = 0;   // rows past the region
+#pragma unroll
+    for (int a = 0; a < NR; a++) {
+        const int ri = w + a * NW, gi = gi0 + ri;
+        if (ri >= R) break;
+        const bool known = colok && gi >= 0 && gi < si && (LEVELSET ? lr[a] <= L0 : lr[a] != 0);
+        const mask_t mk = __ballot(known), mf = LEVELSET ? __ballot(known && lr[a] == L0) : mk;
+        if (lane == 0) {
+            known_s[ri] = mk;
+            front_s[ri] = mf;
+        }
+        if (lane < R) val[ri * RS + lane] = xr[a];
+    }
+    __syncthreads();
+    mask_t got = known_s[lane], f = front_s[lane];
+    // the open cells of this lane's row: inside the region and the grid, not known
+    const mask_t cols = __ballot(colok);
+    mask_t open = (lane < R && gi0 + lane >= 0 && gi0 + lane < si) ? cols & ~got : 0ull;
+    // a tile cell reaches level L0+s only through a level-L0 cell within
+    // distance s <= H, i.e. inside this region (every wave sees the same rows)
+    const bool work = __any(f != 0) && __any(open != 0);
     if (!work) {
         if (!LEVELSET) {
-            for (int li = ty; li < kTile; li += T)
-                for (int lj = tx; lj < kTile; lj += T) {
-                    const int gi = ti * kTile + li, gj = tj * kTile + lj;
-                    if (gi >= si || gj >= sj) continue;
-                    const size_t g = (size_t)gi * sj + gj;
-                    const int r = (li + H) * RS + (lj + H), rm = (li + H) * RSM + (lj + H);
-                    gout[g] = val[r];
-                    vout[g] = mk[rm] != kUnreached;
-                }
-        } else if (threadIdx.x == 0) {
-            *tile_more = 0;
-        }
-        return;
-    }
-    // row masks of the open (unreached) cells and of level L0, one ballot
-    // per region row (4 waves, consecutive LDS addresses)
-    {
-        const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-        for (int r = w; r < R; r += kBlock / 64) {
-            const int16_t m = lane < R ? mk[r * RSM + lane] : kNone;
-            const unsigned long long o = __ballot(m == kUnreached);
-            const unsigned long long f = __ballot(m == (int16_t)L0);
-            if (lane == 0) {
-                open_s[r] = o;
-                front[0][r] = f;
-            }
-        }
-    }
-    __syncthreads();
-    // expand levels L0+1 .. L0+H: wave 0, lane = region row; per level also
-    // the row offsets of its cells
-    if (threadIdx.x < 64) {
-        const int r = threadIdx.x;
-        unsigned long long open = r < R ? open_s[r] : 0ull, f = r < R ? front[0][r] : 0ull;
-        int top = 0;
-        for (int st = 1; st <= H; st++) {
-            const unsigned long long d = f | (f << 1) | (f >> 1);
-            const unsigned long long up = __shfl_up(d, 1, 64), dn = __shfl_down(d, 1, 64);
-            unsigned long long nf = d;
-            if (r > 0) nf |= up;
-            if (r < R - 1) nf |= dn;
-            nf &= open;
-            if (r >= R) nf = 0;
-            open &= ~nf;
-            if (r < R) front[st][r] = nf;
-            // exclusive scan of the row counts by bit slices: one ballot per
-            // bit of the count (<= 64), no lane shuffles
-            const int cnt = __popcll(nf);
-            const unsigned long long below = (1ull << r) - 1ull;
-            int excl = 0, total = 0;
 #pragma unroll
-            for (int b = 0; b < 7; b++) {
-                const unsigned long long m = __ballot((cnt >> b) & 1);
-                excl += __popcll(m & below) << b;
-                total += __popcll(m) << b;
+            for (int a = 0; a < NR; a++) {
+                const int ri = w + a * NW, gi = gi0 + ri;
+                if (!incol || ri < H || ri >= H + kTile || gi >= si || gj >= sj) continue;
+                const size_t g = (size_t)gi * sj + gj;
+                gbl(gout)[g] = xr[a];
+                gbl(vout)[g] = lr[a] != 0;
             }
-            pre[st][r] = (int16_t)excl;
-            if (r == 0) tot[st] = (int16_t)total;
-            f = nf;
-            if (!__any(nf != 0ull)) break;
-            top = st;
         }
-        if (r == 0) top_s = top;
+        return false;
+    }
+    float hv[NR];
+    if (!LEVELSET) {   // the halo's values, in flight over the expansion
+#pragma unroll
+        for (int a = 0; a < NR; a++) {
+            const int ri = w + a * NW, gi = gi0 + ri;
+            const size_t g = (size_t)min(max(gi, 0), si - 1) * sj + gjc;
+            const bool inner = incol && ri >= H && ri < H + kTile;
+            hv[a] = inner ? 0.f : gbl<const float>(gin)[g];
+        }
+    }
+    // expand levels L0+1 .. L0+H, four a step; wave w lists level w of the
+    // step (0: the fourth)
+    mask_t last = 0;   // level L0+H's cells of this lane's row
+    for (int g = 0; g < (H + NW - 1) / NW; g++) {
+        mask_t m = 0, before = 0;   // this wave's level, and the set reached before it
+#pragma unroll
+        for (int q = 1; q <= NW; q++) {
+            if (w == (q & (NW - 1))) before = got;
+            const mask_t d = f | (f << 1) | (f >> 1);
+            f = (d | lane_below(d) | lane_above(d)) & open;
+            if ((H & (NW - 1)) && g * NW + q > H) f = 0;
+            open &= ~f;
+            got |= f;
+            if (w == (q & (NW - 1))) m = f;
+        }
+        if (g * NW + NW == H) last = f;
+        const int st = g * NW + (w ? w : NW);
+        if (!__any(m != 0)) {
+            if (!__any(f != 0)) break;
+            continue;
+        }
+        // exclusive scan of the row counts by bit slices: one ballot per bit
+        // of the count (<= 64), no lane shuffles
+        const int cnt = __popcll(m);
+        int excl = 0;
+#pragma unroll
+        for (int b = 0; b < 7; b++) {
+            const mask_t s = __ballot((cnt >> b) & 1);
+            excl += __builtin_amdgcn_mbcnt_hi((uint32_t)(s >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)s, 0)) << b;
+        }
+        const int total = __builtin_amdgcn_readlane(excl + cnt, 63);
+        int first = 0;
+        if (lane == 0) {
+            first = atomicAdd(&cursor, total);
+            level_s[st] = make_int2(first, total);
+        }
+        const mask_t r0 = lane_below(before), r2 = lane_above(before);
+        first = __builtin_amdgcn_readfirstlane(first);
+        // neighbour bits in getNeighborhood order: the row above, left, right, the row below
+        auto three = [](mask_t r, int j) { return (uint32_t)((j > 0 ? r >> (j - 1) : r << 1) & 7ull); };
+        auto entry = [&](mask_t a, mask_t b, mask_t c, int i, int j) {
+            const uint32_t b1 = three(b, j);
+            const uint32_t nb = three(a, j) | ((b1 & 1u) << 3) | ((b1 & 4u) << 2) | (three(c, j) << 5);
+            return (nb << 12) | ((uint32_t)i << 6) | (uint32_t)j;
+        };
+        mask_t rest = cnt <= kShortRow ? m : 0ull;
+        for (int k = first + excl; __any(rest != 0); k++) {
+            if (rest != 0) {
+                const int j = __ffsll((long long)rest) - 1;
+                rest &= rest - 1;
+                list[k] = entry(r0, before, r2, lane, j);
+            }
+        }
+        for (mask_t longs = __ballot(cnt > kShortRow); longs; longs &= longs - 1) {
+            const int i = __ffsll((long long)longs) - 1;
+            auto row = [&](mask_t v) {
+                return ((mask_t)(uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), i) << 32) |
+                       (uint32_t)__builtin_amdgcn_readlane((int)v, i);
+            };
+            const mask_t mi = row(m);
+            const uint32_t e = entry(row(r0), row(before), row(r2), i, lane);
+            const int k = first + __builtin_amdgcn_readlane(excl, i) +
+                          __builtin_amdgcn_mbcnt_hi((uint32_t)(mi >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mi, 0));
+            if ((mi >> lane) & 1) list[k] = e;
+        }
+        if (!__any(f != 0)) break;
+    }
+    if (!LEVELSET) {
+        if (w == 0) done_s[lane] = got;
+#pragma unroll
+        for (int a = 0; a < NR; a++) {
+            const int ri = w + a * NW;
+            const bool inner = incol && ri >= H && ri < H + kTile;
+            if (ri < R && lane < R && !inner) val[ri * RS + lane] = hv[a];
+        }
     }
     __syncthreads();
-    const int top = top_s;
-    // values, level by level: the cells of a level spread over all threads
-    // (cell t of the level: the row whose offset range holds t, then the
-    // (t - offset)-th set bit of that row's mask)
-    for (int st = 1; st <= top; st++) {
+    if (!LEVELSET) {   // the tile's cells that no level reaches: known or out of reach
+#pragma unroll
+        for (int a = 0; a < NR; a++) {
+            const int ri = w + a * NW, gi = gi0 + ri;
+            if (!incol || ri < H || ri >= H + kTile || gi >= si || gj >= sj) continue;
+            const bool known = lr[a] != 0;
+            if (!known && ((done_s[ri] >> lane) & 1)) continue;   // the level loop writes it
+            const size_t g = (size_t)gi * sj + gj;
+            gbl(gout)[g] = xr[a];
+            gbl(vout)[g] = known;
+        }
+    }
+    // values, level by level; lane st of every wave holds level st's range
+    const int2 range = level_s[min(lane, NW * ((H + NW - 1) / NW))];
+    int off = __builtin_amdgcn_readlane(range.x, 1), n = __builtin_amdgcn_readlane(range.y, 1);
+    uint32_t ent = list[off + threadIdx.x];   // past the level's last entry: not used
+    for (int st = 1; st <= H && n > 0; st++) {
         const int L = L0 + st;
-        const int n = tot[st];
-        for (int t = threadIdx.x; t < n; t += kBlock) {
-            int lo = 0, hi = 63;
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (pre[st][mid] <= t) lo = mid;
-                else hi = mid - 1;
-            }
-            const int ri = lo;
-            int k = t - pre[st][ri];
-            unsigned long long m = front[st][ri];
-            int rj = 0;
-#pragma unroll
-            for (int w = 32; w >= 1; w >>= 1) {
-                const unsigned long long low = m & ((1ull << w) - 1ull);
-                const int c = __popcll(low);
-                if (k >= c) {
-                    k -= c;
-                    m >>= w;
-                    rj += w;
-                } else {
-                    m = low;
-                }
-            }
-            // the 8 neighbours in getNeighborhood order, loads first
-            int16_t qm[8];
+        const int noff = st < H ? __builtin_amdgcn_readlane(range.x, st + 1) : 0;
+        const int nn = st < H ? __builtin_amdgcn_readlane(range.y, st + 1) : 0;
+        const uint32_t nent = list[noff + threadIdx.x];   // the next level's, a barrier ahead
+        auto cell = [&](uint32_t ent) {
+            const int ri = (ent >> 6) & 63, rj = ent & 63, c = ri * RS + rj;
             float qv[8];
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const int di = (e < 3) ? -1 : (e < 5 ? 0 : 1);
                 const int dj = (e < 3) ? e - 1 : (e < 5 ? (e == 3 ? -1 : 1) : e - 6);
-                const int qi = ri + di, qj = rj + dj;
-                const bool ok = qi >= 0 && qi < R && qj >= 0 && qj < R;
-                qm[e] = ok ? mk[qi * RSM + qj] : kNone;
-                qv[e] = ok ? val[qi * RS + qj] : 0.f;
+                qv[e] = val[c + di * RS + dj];
             }
+            const int count = __popc(ent >> 12);
+            const double rc = inv[count];   // 1 / count rounded to nearest
+            // a neighbour that is not of a lower level adds +0: the sum
+            // starts at +0 and is never -0, so it is left as it was
             double avg = 0;
-            int count = 0;
 #pragma unroll
             for (int e = 0; e < 8; e++)
-                if (qm[e] < L) {
-                    avg += (double)qv[e];
-                    count++;
-                }
-            if (LEVELSET && OUT) val[ri * RS + rj] = (float)(avg / count + 1.f);
-            else if (LEVELSET) val[ri * RS + rj] = (float)(avg / count - 1.f);
-            else val[ri * RS + rj] = (float)(avg / count);
-            mk[ri * RSM + rj] = (int16_t)L;   // same-level neighbours read L or unreached: not below L either way
-        }
-        __syncthreads();
-    }
-    // write the tile
-    bool reached_end = false;
-    for (int li = ty; li < kTile; li += T)
-        for (int lj = tx; lj < kTile; lj += T) {
-            const int gi = ti * kTile + li, gj = tj * kTile + lj;
-            if (gi >= si || gj >= sj) continue;
-            const int r = (li + H) * RS + (lj + H), rm = (li + H) * RSM + (lj + H);
-            const size_t g = (size_t)gi * sj + gj;
-            const int16_t m = mk[rm];
-            if (LEVELSET) {
-                if (m > L0 && m <= L0 + H) {
-                    gout[g] = val[r];
-                    mkout[g] = m;
-                    reached_end |= m == L0 + H;
-                }
-            } else {
-                gout[g] = val[r];
-                vout[g] = (m != kUnreached) ? 1 : 0;
+                avg += (double)__uint_as_float(__float_as_uint(qv[e]) & (0u - ((ent >> (12 + e)) & 1u)));
+            // avg / count, correctly rounded: a quotient within an ulp and
+            // one step with its exact remainder (Markstein's theorem: rc is
+            // the correctly rounded reciprocal; no underflow, avg is a sum
+            // of floats); an infinite or NaN sum stays as it is
+            const double q0 = avg * rc;
+            const double q1 = __builtin_fma(__builtin_fma(-(double)count, q0, avg), rc, q0);
+            const double q = finite_d(avg) ? q1 : avg;
+            float x;
+            if (LEVELSET && OUT) x = (float)(q + 1.f);
+            else if (LEVELSET) x = (float)(q - 1.f);
+            else x = (float)q;
+            val[c] = x;
+            const int li = ri - H, lj = rj - H;
+            if ((unsigned)li < (unsigned)kTile && (unsigned)lj < (unsigned)kTile) {   // an open cell: inside the grid
+                const size_t g = (size_t)(gi0 + ri) * sj + (gj0 + rj);
+                // global stores (a flat store counts as an LDS operation too,
+                // and the barrier would wait for it)
+                gbl(gout)[g] = x;
+                if (LEVELSET) gbl(mkout)[g] = L;
+                else gbl(vout)[g] = 1;
             }
-        }
-    if (LEVELSET) {
-        const bool any = __syncthreads_or(reached_end);
-        if (threadIdx.x == 0) {
-            *tile_more = any ? 1 : 0;
-            if (any) *more = 1;
-        }
+        };
+        if ((int)threadIdx.x < n) cell(ent);
+        for (int t = threadIdx.x + kBlock; t < n; t += kBlock) cell(list[off + t]);
+        __syncthreads();
+        off = noff;
+        n = nn;
+        ent = nent;
     }
+    // did the tile reach the band's last level?  (every wave holds the rows)
+    const mask_t inner = ((1ull << kTile) - 1ull) << H;
+    return __any(lane >= H && lane < H + kTile && (last & inner) != 0);
 }
 
 // Velocity extrapolation, radius 10 (StaggeredVelocityGrid::extrapolate,
@@ -684,7 +706,7 @@ __global__ void __launch_bounds__(kBlock) k_extrapolate(const SceneDev* scenes, 
     const uint8_t* vin = isU ? (which == 0 ? s.uval : s.uvalS) : (which == 0 ? s.vval : s.vvalS);
     float* gout = isU ? (which == 0 ? s.su : s.uf) : (which == 0 ? s.sv : s.vf);
     uint8_t* vout = isU ? (which == 0 ? s.uvalS : s.uvalF) : (which == 0 ? s.vvalS : s.vvalF);
-    bfs_band<11, false>(gin, vin, nullptr, gout, vout, nullptr, si, sj, 0, nullptr, nullptr);
+    bfs_band<11, false>(blockIdx.x, gin, vin, nullptr, gout, vout, nullptr, si, sj, 0);
 }
 
 // Markers (known cells: sdf > 0, level 0), one block per BFS tile, which
@@ -702,7 +724,7 @@ __global__ void __launch_bounds__(kBlock) k_levelset_init(const SceneDev* scenes
     const int tile = blockIdx.x;
     if (tile >= tiles) return;
     if (tile == 0)
-        for (int k = threadIdx.x; k < kMaxBands; k += kBlock) s.lsFlags[k] = 0;
+        for (int k = threadIdx.x; k <= kMaxBands; k += kBlock) s.lsFlags[k] = 0;
     const int ti = tile / tilesJ, tj = tile - ti * tilesJ;
     bool known = false;
     for (int q = threadIdx.x; q < kTile * kTile; q += kBlock) {
@@ -714,46 +736,57 @@ __global__ void __launch_bounds__(kBlock) k_levelset_init(const SceneDev* scenes
         s.marker[c] = k ? 0 : kMaxLevel;
         known |= k;
     }
-    if (__syncthreads_or(known) && threadIdx.x == 0) {
-        s.lsTile[tile] = 1;
-        if (!OUT) s.sc->sdf_known = 1;   // some cell is outside
-    } else if (threadIdx.x == 0) {
-        s.lsTile[tile] = 0;
+    const bool any = __syncthreads_or(known);
+    if (threadIdx.x == 0) {
+        s.lsTile[tile] = any ? 1 : 0;
+        s.lsStamp[tile] = 0;
+        if (any && !OUT) s.sc->sdf_known = 1;   // some cell is outside
     }
 }
 
-// One band of extrapolateLevelsetInside: levels L0+1 .. L0+16.  Runs only if
-// the previous band reached its last level somewhere (lsFlags[band - 1]);
-// records the bands that ran in sc->ls_bands.  A tile has work only if a
-// level-L0 cell lies within its 16-cell halo, i.e. in it or one of its eight
-// neighbours (the halo is narrower than a tile), and such a tile reached
-// L0 in the band before: the others only record that they did not reach
-// the band's end.
+// One band of extrapolateLevelsetInside: levels L0+1 .. L0+16; records the
+// bands that ran in sc->ls_bands.  A tile has work only if a level-L0 cell
+// lies within its 16-cell halo, i.e. in it or one of its eight neighbours
+// (the halo is narrower than a tile), and such a tile reached L0 in the band
+// before.  Band 0 looks at its neighbours' flags (a block a tile); from then
+// on a tile that reaches the band's last level queues itself and its
+// neighbours for the next band, once each (an atomic stamp a tile), and the
+// launch has at most kBandBlocks blocks a scene, which share the queue.  The
+// queue's order varies, the results do not: a tile's cells depend on levels
+// the launch before finished.
+// A band is bound by latency: one tile's chain of 16 levels (10 us in the
+// block) and the start of its blocks.  With a block a tile, each with the
+// kernel's LDS and most only to exit, the 1,024 blocks of a 1024^2 scene took
+// over 20 us to pass; its bands queue about 100-180 tiles.  Averages over the
+// 1024^2 NB-FLIP dam break's 649 bands of 3 frames: 31.8 us a launch with a
+// block a tile and the search inside the level loop, 14.8 us so.  256 blocks
+// are one a CU.
+constexpr int kBandBlocks = 256;
 template <bool OUT>
 __global__ void __launch_bounds__(kBlock) k_levelset_band(const SceneDev* scenes, int band)
 {
     const SceneDev& s = scenes[blockIdx.y];
     if (!s.active) return;
-    if (band > 0 && cst(s.lsFlags)[band - 1] == 0) return;   // written by the previous band's launch
     const int tilesI = (s.I + kTile - 1) / kTile, tilesJ = (s.J + kTile - 1) / kTile;
     const int tiles = tilesI * tilesJ;
-    const int tile = blockIdx.x;
-    if (tile >= tiles) return;
-    if (tile == 0 && threadIdx.x == 0) s.sc->ls_bands = band + 1;
-    const uint8_t* fin = s.lsTile + (band & 1) * tiles;
-    uint8_t* fout = s.lsTile + ((band + 1) & 1) * tiles;
-    const int ti = tile / tilesJ, tj = tile - ti * tilesJ;
-    bool near = false;
-    if (threadIdx.x < 9) {
-        const int ni = ti + threadIdx.x / 3 - 1, nj = tj + threadIdx.x % 3 - 1;
-        near = ni >= 0 && ni < tilesI && nj >= 0 && nj < tilesJ && fin[ni * tilesJ + nj] != 0;
+    int32_t* const queue = s.lsQueue + ((band + 1) & 1) * tiles;   // the next band's tiles
+    // band 0: this block's own tile; later: the tiles queued by the band before
+    const int n = band == 0 ? tiles : cst(s.lsFlags)[band];
+    if (blockIdx.x == 0 && threadIdx.x == 0 && n > 0) s.sc->ls_bands = band + 1;
+    for (int k = blockIdx.x; k < n; k += gridDim.x) {
+        const int tile = band == 0 ? k : cst(s.lsQueue + (band & 1) * tiles)[k];
+        const int ti = tile / tilesJ, tj = tile - ti * tilesJ;
+        const int ni = ti + (int)threadIdx.x / 3 - 1, nj = tj + (int)threadIdx.x % 3 - 1;
+        const bool nine = threadIdx.x < 9 && ni >= 0 && ni < tilesI && nj >= 0 && nj < tilesJ;
+        if (band == 0 && !__syncthreads_or(nine && s.lsTile[ni * tilesJ + nj] != 0)) continue;
+        const bool end = bfs_band<16, true, OUT>(tile, s.fsdf, nullptr, s.marker, s.fsdf, nullptr, s.marker, s.I, s.J,
+                                                 band * 16);
+        if (end && nine) {
+            const int t = ni * tilesJ + nj;
+            if (atomicExch(&s.lsStamp[t], band + 1) != band + 1) queue[atomicAdd(&s.lsFlags[band + 1], 1)] = t;
+        }
+        __syncthreads();   // the tile's LDS is free for the next one
     }
-    if (!__syncthreads_or(near)) {
-        if (threadIdx.x == 0) fout[tile] = 0;
-        return;
-    }
-    bfs_band<16, true, OUT>(s.fsdf, nullptr, s.marker, s.fsdf, nullptr, s.marker, s.I, s.J, band * 16,
-                            &s.lsFlags[band], &fout[tile]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1003,6 +1036,7 @@ void launch_levelset_init(dim3 g, hipStream_t st, const SceneDev* sc, bool outsi
 }
 void launch_levelset_band(dim3 g, hipStream_t st, const SceneDev* sc, int band, bool outside)
 {
+    if (band > 0) g.x = std::min<unsigned>(g.x, kBandBlocks);
     if (outside) fg_launch(k_levelset_band<true>, g, dim3(kBlock), st, sc, band);
     else fg_launch(k_levelset_band<false>, g, dim3(kBlock), st, sc, band);
 }
