@@ -284,19 +284,24 @@ void carve(fg_scene* s, Carver& cv)
         auto cells = [&](int l) { return (int64_t)M.lv[l].I * M.lv[l].J; };
         M.t = std::max(1, n - 1);
         for (int t = 1; t < n - 1; t++) {
-            int64_t sum = 0;
-            for (int l = t; l < n; l++) sum += cells(l);
-            if (cells(t) <= kMgCoarseTop && sum <= kMgCoarseCells) {
+            int64_t sum = 0, halo = 0;
+            for (int l = t; l < n; l++) {
+                sum += cells(l);
+                halo += (int64_t)(M.lv[l].I + 4) * (M.lv[l].J + 4);
+            }
+            if (cells(t) <= kMgCoarseTop && sum <= kMgCoarseCells && halo <= kMgCoarseHalo) {
                 M.t = t;
                 break;
             }
         }
-        int o = 0;
+        int o = 0, halo = 0;
         for (int l = M.t; l < n; l++) {
             M.roff[l] = o;
             o += (int)cells(l);
+            halo += (M.lv[l].I + 4) * (M.lv[l].J + 4);
         }
         M.tcells = o;
+        M.thalo = (halo + 3) & ~3;
         std::memcpy(M.canon, mg_canonical(), sizeof(M.canon));
         h.mg = cv.take<MgLevels>(1);
         int64_t all = 0;
@@ -799,6 +804,7 @@ struct Group {
     int mg_levels = 0;                  // most multigrid levels of a scene using the V-cycle
     int map_kinds = 0;                  // block-map kinds the solve uses (0 when maps are off)
     int64_t map_off[kMapKinds]{};       // offset of each kind's map in the lane's map buffer
+    int mg_halo = 0;                    // largest MgLevels::thalo (k_mg_coarse's LDS)
     int mg_top = 0;                     // largest first level of k_mg_coarse (levels below: one launch each)
     unsigned mg_grid[kMgMaxLevels]{};   // blocks per scene over level l, one cell per thread
     unsigned sym_grid[kMgMaxLevels]{};  // 16 x 16-row tiles per scene over level l (k_mg_sym)
@@ -918,6 +924,7 @@ int make_group(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const std::vec
         if (s->h.precond == kPrecondMG) {
             G.mg_levels = std::max(G.mg_levels, s->mgh.n);
             G.mg_top = std::max(G.mg_top, s->mgh.t);
+            G.mg_halo = std::max(G.mg_halo, s->mgh.thalo);
             for (int l = 1; l < s->mgh.n; l++) {
                 const unsigned b = (unsigned)cdiv((int64_t)s->mgh.lv[l].I * s->mgh.lv[l].J, kBlock);
                 G.mg_grid[l] = std::max(G.mg_grid[l], b);
@@ -1254,7 +1261,7 @@ void launch_vcycle(const Group& G, hipStream_t st, const SolveLaunch& S, int whi
     }
     {
         KProf kp(G, FG_K_MG_COARSE, true);
-        launch_mg_coarse(dim3(1, S.ny), st, S.d);
+        launch_mg_coarse(dim3(1, S.ny), st, S.d, G.mg_halo);
         kp.done(0);
     }
     if (G.fused) {

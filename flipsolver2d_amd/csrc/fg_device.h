@@ -51,6 +51,10 @@ constexpr int kMgRowStride = 32;         // floats per stored coefficient row: o
 constexpr int kMgCoarseThreads = 1024;
 constexpr int kMgCoarseTop = kMgCoarseThreads;
 constexpr int kMgCoarseCells = 2 * kMgCoarseThreads;
+// and, with a two-cell halo round each level, at most kMgCoarseHalo cells
+// (x and y of every level in 32 KB of LDS; only grids a few cells wide, with
+// mostly halo, reach it: 32 x 32 over 16 x 16 is 1,696)
+constexpr int kMgCoarseHalo = 4096;
 constexpr int kFixupLongCap = 512;       // longest cell the wave-cooperative id sort takes
 
 // Material codes and tests, FlipSolver2dLib/materialgrid.h:6-20.
@@ -109,6 +113,7 @@ struct MgLevels {
     int32_t n;        // levels; level n-1 is the bottom
     int32_t t;        // first level of k_mg_coarse (1 <= t <= n-1)
     int32_t tcells;   // cells of levels t .. n-1 together
+    int32_t thalo;    // the same with a two-cell halo round each level, up to a multiple of 4
     // offset of level l >= t among the cells of levels t .. n-1: in
     // k_mg_coarse's LDS, and of its dinv from lv[t].dinv (the levels' dinv
     // arrays are contiguous in level order)

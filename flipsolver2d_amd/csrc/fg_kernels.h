@@ -58,7 +58,8 @@ FG_DECLARE_LAUNCH(mg_symmark, int l, int nsym);
 FG_DECLARE_LAUNCH(mg_down0, const int2* map, int which);
 FG_DECLARE_LAUNCH(mg_resid, const int2* map, int l);
 FG_DECLARE_LAUNCH(mg_restrict, const int2* map, int l);
-FG_DECLARE_LAUNCH(mg_coarse);
+// max_halo: the largest MgLevels::thalo of the launch's scenes
+FG_DECLARE_LAUNCH(mg_coarse, int max_halo);
 FG_DECLARE_LAUNCH(mg_prolong, const int2* map, int l);
 FG_DECLARE_LAUNCH(mg_post, const int2* map, int l);
 FG_DECLARE_LAUNCH(mg_rr, const int2* map, int l);

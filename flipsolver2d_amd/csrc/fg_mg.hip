@@ -610,65 +610,69 @@ __global__ void __launch_bounds__(kBlock) k_mg_restrict(const SceneDev* scenes, 
 // there, then the up steps of k_mg_prolong and k_mg_post back to level t,
 // whose y it writes for the level above.  The arithmetic and its order are
 // those of the per-level kernels, so where t falls does not change z.
-// Thread c owns cell c of every level.  The block is latency-bound, so its
-// global loads come in two rounds: every level's dinv with level t's input
-// (its 4x4 patch of y_{t-1}), then the stored coefficient rows of the
-// thread's level-t and bottom cells, held in registers for the way down
-// and the way up.  LDS: every level's r and dinv (a cell is active exactly
-// where its dinv's bit pattern is nonzero) and one work array for the level
-// at hand: its residual y on the way down (dead once the coarser r is
-// made), its x on the way up.  On the way up each level's y overwrites its
-// r in place (a thread reads only its own cell's r there), where the finer
-// level reads it.  On the way down each level's x = r dinv is made once
-// into its own array before the residual reads 25 of them.  The bottom's
-// iterate has its own array with a two-cell zero halo, so its stencil needs
-// no bounds tests.
+// Thread c owns cell c of every level.  One CU runs the whole block, so it
+// is bound by instruction issue (16 waves on four SIMDs) and by latency:
+//   - global loads come in two rounds, every level's dinv with level t's
+//     input (its 4x4 patch of y_{t-1}) and the bottom's rows, then the
+//     stored coefficient rows of the thread's level-t cell; a level's 25
+//     coefficients stay in registers for the way down and the way up;
+//   - every level's x and y lie in LDS with a two-cell halo of zeros
+//     (dynamic LDS, MgLevels::thalo floats each, cleared while the first
+//     loads are in flight), so a stencil, a restriction and a prolongation
+//     read at fixed offsets from the cell, with no bounds tests or masks (a
+//     halo zero adds what the masked clamped value did);
+//   - the bottom's sweeps alternate between its x and y, the first from
+//     zero without its stencil.
+// Masked and clamped addresses for each of the 25 terms, and the bottom's
+// coefficients read from LDS in every sweep, took 13.8 us a launch at
+// 32 x 32 over 16 x 16 cells; this form 9.7 us (the 128^2 dam break).
 __device__ __forceinline__ bool mg_active(float dinv) { return __float_as_uint(dinv) != 0u; }
 
-// The 25 stored coefficients of row c, loaded together.
-__device__ __forceinline__ void coarse_row_load(gptr<const float> coef, int CL, int c, float (&a)[kMgStencil])
+// The 25 coefficients of an active level-l row (see row_dot).
+template <typename MT>
+__device__ __forceinline__ void coarse_row(const MT& M, int l, int c, float dinv_c, float (&a)[kMgStencil])
 {
-    (void)CL;
-    load_coef_row(coef, c, a);
+#pragma unroll
+    for (int k = 0; k < kMgStencil; k++) a[k] = M.canon[l][k];
+    if (dinv_c > 0.f) load_coef_row(gbl<const float>(M.lv[l].coef), c, a);
 }
 
-// row_dot with v_k = V(k) made as it is summed (same terms, same order):
-// the canonical stencil (LDS) on canonical rows (dinv < 0), else the
-// coefficients in a.
-template <typename F>
-__device__ __forceinline__ float coarse_row_dot(const float* cn, const float (&a)[kMgStencil], float dinv_c, F V)
+// sum_k a_k x_k over the 5x5 neighbourhood of x[home], rows w floats apart
+__device__ __forceinline__ float coarse_dot(const float (&a)[kMgStencil], const float* x, int home, int w)
 {
-    const bool stored = dinv_c > 0.f;
     float ax = 0.f;
 #pragma unroll
-    for (int k = 0; k < kMgStencil; k++) ax += (stored ? a[k] : cn[k]) * V(k);
+    for (int k = 0; k < kMgStencil; k++) ax += a[k] * x[home + (k / 5 - 2) * w + (k % 5 - 2)];
     return ax;
 }
 
 __global__ void __launch_bounds__(kMgCoarseThreads) k_mg_coarse(const SceneDev* scenes)
 {
     constexpr int NT = kMgCoarseThreads;
-    constexpr int W = kMgBottomMax + 4;
     static_assert(kMgBottomMax * kMgBottomMax <= NT, "one bottom cell per thread");
     static_assert(kMgCoarseTop <= NT, "one level-t cell per thread");
+    static_assert(kMgBottomSweeps % 2 == 0, "the bottom's last sweep writes its y");
     __shared__ float rs[kMgCoarseCells], ds[kMgCoarseCells];
-    __shared__ float tx[kMgCoarseTop], xw[kMgCoarseTop];
-    __shared__ float xb[2][W * W];
-    __shared__ float cns[kMgMaxLevels][kMgStencil];
-    constexpr int kBS = kMgBottomMax * kMgBottomMax + 1;   // the bottom's entry stride in LDS (max)
-    __shared__ float cbs[kMgStencil * kBS];   // bottom coefficients, entry-major
+    extern __shared__ float4 halo4[];
     const SceneDev& s = scenes[blockIdx.y];
     const auto& M = *cst(s.mg);
     const int t = M.t, nb = M.n - 1;
     if (!mg_iterating(s)) return;
     const int tid = threadIdx.x;
-    if (tid < kMgMaxLevels * kMgStencil) (&cns[0][0])[tid] = (&M.canon[0][0])[tid];
+    const int HT = M.thalo;   // a multiple of 4
+    float* const hx = reinterpret_cast<float*>(halo4);
+    float* const hy = hx + HT;
     const auto& T = M.lv[t];
+    const auto& B = M.lv[nb];
     const int TI = T.I, TJ = T.J, CT = TI * TJ;   // roff[t] = 0
     const bool tin = tid < CT;
     const int tc = tin ? tid : CT - 1;
     const int tci = tc / TJ, tcj = tc - tci * TJ;
-    // round 1: dinv of levels t .. n-1 (contiguous) and level t's input
+    const int CB = B.I * B.J, ob = M.roff[nb];   // CB <= kMgBottomMax^2 (the hierarchy stops there)
+    const bool bin = tid < CB;
+    // round 1: dinv of levels t .. n-1 (contiguous), level t's input, and the
+    // bottom's rows, whose sweeps read the stored coefficients of every row
+    float dt, cb[kMgStencil];
     {
         gptr<const float> dg = gbl<const float>(T.dinv);
         const int TC = M.tcells;
@@ -684,148 +688,123 @@ __global__ void __launch_bounds__(kMgCoarseThreads) k_mg_coarse(const SceneDev* 
             rt = gbl<const float>(M.lv[1].r)[tc];
         }
 #pragma unroll
+        for (int k = 0; k < kMgStencil; k++) cb[k] = 0.f;
+        if (bin) load_coef_row(gbl<const float>(B.coef), tid, cb);
+        for (int k = tid; k < HT / 2; k += NT) halo4[k] = make_float4(0.f, 0.f, 0.f, 0.f);   // hx and hy
+        __syncthreads();
+        dt = dv[0];   // level t's dinv of cell tc
+#pragma unroll
         for (int q = 0; q < Q; q++)
             if (tid + q * NT < TC) ds[tid + q * NT] = dv[q];
-        if (tin) rs[tc] = (t == 1 || mg_active(dv[0])) ? rt : 0.f;   // dv[0] = level t's dinv of cell tc
-    }
-    __syncthreads();
-    // round 2: the coefficients of this thread's level-t row where it reads
-    // stored ones (level t above the bottom), and the bottom's, whose sweeps
-    // read the stored coefficients of every row
-    const auto& B = M.lv[nb];
-    const int CB = B.I * B.J, ob = M.roff[nb];   // CB <= kMgBottomMax^2 (the hierarchy stops there)
-    const bool bin = tid < CB;
-    const int bc = bin ? tid : 0;
-    const float dct = tin ? ds[tc] : 0.f;
-    float ct[kMgStencil];
-#pragma unroll
-    for (int k = 0; k < kMgStencil; k++) ct[k] = 0.f;
-    if (tin && nb != t && dct > 0.f) coarse_row_load(gbl<const float>(T.coef), CT, tc, ct);
-    // the bottom's entry stride in LDS: a multiple of the 32 banks plus one,
-    // so that the copy below (consecutive threads: consecutive entries of a
-    // row) and a sweep (consecutive cells: one entry) are both conflict-free
-    const int SB = ((CB + 31) & ~31) + 1;
-    {   // the bottom's coefficient rows (contiguous) to LDS by the whole block,
-        // transposed to entry-major there
-        gptr<const float> bcoef = gbl<const float>(B.coef);
-        const int NBC = kMgRowStride * CB;
-        constexpr int QB = (kMgRowStride * kMgBottomMax * kMgBottomMax + NT - 1) / NT;
-        float v[QB];
-#pragma unroll
-        for (int q = 0; q < QB; q++) v[q] = bcoef[min(tid + q * NT, NBC - 1)];
-#pragma unroll
-        for (int q = 0; q < QB; q++) {
-            const int i = tid + q * NT, c = i / kMgRowStride, k = i % kMgRowStride;
-            if (i < NBC && k < kMgStencil) cbs[k * SB + c] = v[q];
+        if (tin) {
+            const float r = (t == 1 || mg_active(dt)) ? rt : 0.f;
+            rs[tc] = r;
+            if (t < nb) hx[(tci + 2) * (TJ + 4) + tcj + 2] = r * fabsf(dt);   // x = r dinv
         }
     }
-    for (int l = t; l < nb; l++) {   // down: x = r dinv, y = r - A x, r_{l+1} = R y
+    // round 2: this thread's level-t row
+    float ct[kMgStencil];
+    if (t < nb) coarse_row(M, t, tc, tin ? dt : 0.f, ct);
+    __syncthreads();
+    int ho = 0;   // level l's place in hx and hy
+    for (int l = t; l < nb; l++) {   // down: y = r - A x, r_{l+1} = R y, x_{l+1} = r_{l+1} dinv
         const auto& L = M.lv[l];
-        const int LI = L.I, LJ = L.J, CL = LI * LJ, o = M.roff[l];
-        if (tid < CL) xw[tid] = rs[o + tid] * fabsf(ds[o + tid]);   // x = r dinv
-        __syncthreads();
+        const int LJ = L.J, CL = L.I * LJ, o = M.roff[l], w = LJ + 4;
         if (tid < CL) {
-            const int c = tid;
-            const float dc = ds[o + c];
+            const float dc = ds[o + tid];
+            const int ci = tid / LJ, cj = tid - ci * LJ, home = ho + (ci + 2) * w + cj + 2;
             float y = 0.f;   // inactive row: r = 0 and no coefficients
             if (dc != 0.f) {
-                const int ci = c / LJ, cj = c - ci * LJ;
-                auto V = [&](int k) {
-                    const int ni = ci + k / 5 - 2, nj = cj + k % 5 - 2;
-                    const bool ok = ni >= 0 && ni < LI && nj >= 0 && nj < LJ;
-                    return xw[min(max(ni, 0), LI - 1) * LJ + min(max(nj, 0), LJ - 1)] * mask01(ok);
-                };
                 float ax;
                 if (l == t) {
-                    ax = coarse_row_dot(cns[l], ct, dc, V);
+                    ax = coarse_dot(ct, hx, home, w);
                 } else {
                     float a[kMgStencil];
-#pragma unroll
-                    for (int k = 0; k < kMgStencil; k++) a[k] = 0.f;
-                    if (dc > 0.f) coarse_row_load(gbl<const float>(L.coef), CL, c, a);
-                    ax = coarse_row_dot(cns[l], a, dc, V);
+                    coarse_row(M, l, tid, dc, a);
+                    ax = coarse_dot(a, hx, home, w);
                 }
-                y = rs[o + c] - ax;
+                y = rs[o + tid] - ax;
             }
-            tx[c] = y;
+            hy[home] = y;
         }
         __syncthreads();
         const auto& N = M.lv[l + 1];
-        const int NJ = N.J, NC = N.I * NJ, on = M.roff[l + 1];
-        if (tid < NC) {
-            const int c = tid, ci = c / NJ, cj = c - ci * NJ;
-            rs[on + c] = mg_active(ds[on + c]) ? restrict_at(static_cast<const float*>(tx), LI, LJ, ci, cj) : 0.f;
+        const int NJ = N.J, NC = N.I * NJ, on = M.roff[l + 1], hn = ho + (L.I + 4) * w;
+        if (tid < NC) {   // restrict_at on the halo
+            const int ci = tid / NJ, cj = tid - ci * NJ;
+            const float dn = ds[on + tid];
+            const float* const f = hy + ho + (2 * ci + 1) * w + 2 * cj + 1;   // fine cell (2 ci - 1, 2 cj - 1)
+            float acc = 0.f;
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+#pragma unroll
+                for (int b = 0; b < 4; b++) acc += (w1(a) * w1(b)) * f[a * w + b];
+            const float r = mg_active(dn) ? 0.25f * acc : 0.f;
+            rs[on + tid] = r;
+            if (l + 1 < nb) hx[hn + (ci + 2) * (NJ + 4) + cj + 2] = r * fabsf(dn);
         }
+        ho = hn;
         __syncthreads();
     }
     {   // bottom: y = kMgBottomSweeps sweeps of x += dinv (r - A x) from 0
-        const int ci = bc / B.J, cj = bc - ci * B.J;
-        const float dv = fabsf(ds[ob + bc]), rv = rs[ob + bc];
-        for (int k = tid; k < 2 * W * W; k += NT) (&xb[0][0])[k] = 0.f;
+        const int w = B.J + 4, ci = tid / B.J, cj = tid - ci * B.J, home = ho + (ci + 2) * w + cj + 2;
+        const float dv = bin ? fabsf(ds[ob + tid]) : 0.f, rv = bin ? rs[ob + tid] : 0.f;
+        float x = 0.f + dv * (rv - 0.f);
+        if (bin) hx[home] = x;
         __syncthreads();
-        const int home = (ci + 2) * W + (cj + 2);
-        int cur = 0;
-        for (int sw = 0; sw < kMgBottomSweeps; sw++) {
+#pragma unroll 1
+        for (int sw = 1; sw < kMgBottomSweeps; sw++) {
+            const float* const from = (sw & 1) ? hx : hy;
+            float* const to = (sw & 1) ? hy : hx;
             if (bin) {
-                float ax = 0.f;
-#pragma unroll
-                for (int k = 0; k < kMgStencil; k++)
-                    ax += cbs[k * SB + bc] * xb[cur][home + (k / 5 - 2) * W + (k % 5 - 2)];
-                xb[cur ^ 1][home] = xb[cur][home] + dv * (rv - ax);
+                x = x + dv * (rv - coarse_dot(cb, from, home, w));
+                to[home] = x;
             }
             __syncthreads();
-            cur ^= 1;
         }
-        if (bin) {
-            const float y = xb[cur][home];
-            rs[ob + bc] = y;
-            if (nb == t) gbl(B.y)[bc] = y;
-        }
-        __syncthreads();
+        if (bin && nb == t) gbl(B.y)[tid] = x;
     }
     for (int l = nb - 1; l >= t; l--) {   // up: x = r dinv + P y_{l+1}, y = x + dinv (r - A x)
         const auto& L = M.lv[l];
         const auto& N = M.lv[l + 1];
-        const int LI = L.I, LJ = L.J, CL = LI * LJ, o = M.roff[l];
-        const float* yn = rs + M.roff[l + 1];   // y_{l+1}, in place of r_{l+1}
+        const int LJ = L.J, CL = L.I * LJ, o = M.roff[l], w = LJ + 4, wn = N.J + 4;
+        const int hn = ho;
+        ho -= (L.I + 4) * w;
+        const int ci = tid / LJ, cj = tid - ci * LJ, home = ho + (ci + 2) * w + cj + 2;
+        const float dc = tid < CL ? ds[o + tid] : 0.f, rc = tid < CL ? rs[o + tid] : 0.f;
+        float x = 0.f;
         if (tid < CL) {
-            const int c = tid;
-            const float dc = ds[o + c];
-            float x = 0.f;
-            if (mg_active(dc)) {
-                const int ci = c / LJ, cj = c - ci * LJ;
-                x = rs[o + c] * fabsf(dc) + prolong_at(yn, N.I, N.J, ci, cj);
+            if (mg_active(dc)) {   // prolong_at on the halo
+                const int p0 = (ci >> 1) + 2, q0 = (cj >> 1) + 2;
+                const int p1 = (ci & 1) ? p0 + 1 : p0 - 1, q1 = (cj & 1) ? q0 + 1 : q0 - 1;
+                const float* const f = hy + hn;
+                float acc = 0.f;
+                acc += (0.75f * 0.75f) * f[p0 * wn + q0];
+                acc += (0.75f * 0.25f) * f[p0 * wn + q1];
+                acc += (0.25f * 0.75f) * f[p1 * wn + q0];
+                acc += (0.25f * 0.25f) * f[p1 * wn + q1];
+                x = rc * fabsf(dc) + acc;
             }
-            tx[c] = x;
+            hx[home] = x;
         }
         __syncthreads();
         if (tid < CL) {
-            const int c = tid;
-            const float dc = ds[o + c];
             float y = 0.f;   // inactive row: x = 0
             if (dc != 0.f) {
-                const int ci = c / LJ, cj = c - ci * LJ;
-                auto V = [&](int k) {
-                    const int ni = ci + k / 5 - 2, nj = cj + k % 5 - 2;
-                    const bool ok = ni >= 0 && ni < LI && nj >= 0 && nj < LJ;
-                    return tx[min(max(ni, 0), LI - 1) * LJ + min(max(nj, 0), LJ - 1)] * mask01(ok);
-                };
                 float ax;
                 if (l == t) {
-                    ax = coarse_row_dot(cns[l], ct, dc, V);
+                    ax = coarse_dot(ct, hx, home, w);
                 } else {
                     float a[kMgStencil];
-#pragma unroll
-                    for (int k = 0; k < kMgStencil; k++) a[k] = 0.f;
-                    if (dc > 0.f) coarse_row_load(gbl<const float>(L.coef), CL, c, a);
-                    ax = coarse_row_dot(cns[l], a, dc, V);
+                    coarse_row(M, l, tid, dc, a);
+                    ax = coarse_dot(a, hx, home, w);
                 }
-                y = tx[c] + fabsf(dc) * (rs[o + c] - ax);   // tx[c] = the centre term x_12
+                y = x + fabsf(dc) * (rc - ax);
             }
-            rs[o + c] = y;
-            if (l == t) gbl(L.y)[c] = y;
+            hy[home] = y;
+            if (l == t) gbl(L.y)[tid] = y;
         }
-        __syncthreads();
+        if (l > t) __syncthreads();
     }
 }
 
@@ -1252,8 +1231,8 @@ void launch_mg_up0(dim3 g, hipStream_t st, const SceneDev* sc, const int2* map, 
     else
         fg_launch(k_mg_up0_wide, g, dim3(kBlock), st, sc, map, which);
 }
-void launch_mg_coarse(dim3 g, hipStream_t st, const SceneDev* sc)
+void launch_mg_coarse(dim3 g, hipStream_t st, const SceneDev* sc, int max_halo)
 {
-    fg_launch(k_mg_coarse, g, dim3(kMgCoarseThreads), st, sc);
+    fg_launch_shm(k_mg_coarse, g, dim3(kMgCoarseThreads), 2 * sizeof(float) * max_halo, st, sc);
 }
 }  // namespace fg
