@@ -51,8 +51,9 @@ HBM_PEAK_GBS = 8000.0
 #   pcg_a      17 B per cell and iteration (stencil code 1, z 4, old
 #              direction 4; p 4, q = A' p 4)
 #   pcg_b      32 B per cell and iteration (r -= alpha q in FP32, x += alpha p
-#              in FP64)
-#   mg_down0   5 C + 5 C1 per V-cycle (code, r; level-1 activity, r1)
+#              in FP64); IPP solves only
+#   mg_down0   33 C + 5 C1 per iteration (code, r_old, q, p, x; r, x; level-1
+#              activity, r1), 5 C + 5 C1 for the V-cycle that starts a sweep
 #   mg_up0     9 C + 4 C1 per V-cycle (code, r, z; level-1 y)
 #   mg_resid   k_mg_rr of every level l between level 1 and the coarse
 #              block: 9 B per level-l cell (r, dinv; r_{l+1}) and the 100 B of
@@ -73,7 +74,7 @@ KERNEL_BYTES = {
     "sdf": ("K_SDF", 1.0, "bytes", ["k_sdf_materials"]),
     "pcg_a": ("K_PCG_A", 17.0, "cells", ["k_pcg_a"]),
     "pcg_b": ("K_PCG_B", 32.0, "cells", ["k_pcg_b"]),
-    "mg_down0": ("K_MG_DOWN0", 1.0, "bytes", ["k_mg_down0"]),
+    "mg_down0": ("K_MG_DOWN0", 1.0, "bytes", ["k_mg_step0", "k_mg_down0"]),
     "mg_up0": ("K_MG_UP0", 1.0, "bytes", ["k_mg_up0", "k_mg_up0_wide"]),
     "mg_resid": ("K_MG_RESID", 1.0, "bytes", ["k_mg_rr"]),
     "mg_pp": ("K_MG_PP", 1.0, "bytes", ["k_mg_pp"]),

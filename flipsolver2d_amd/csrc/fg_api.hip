@@ -801,6 +801,7 @@ struct Group {
     bool sources = false;               // some scene has SOURCE cells (afterTransfer, reseeding)
     bool nb = false;                    // NB-FLIP scenes (a group holds one solver class)
     bool visc = false;                  // some scene has viscosity enabled
+    bool ipp = false;                   // some scene's solve uses the IPP
     int mg_levels = 0;                  // most multigrid levels of a scene using the V-cycle
     int map_kinds = 0;                  // block-map kinds the solve uses (0 when maps are off)
     int64_t map_off[kMapKinds]{};       // offset of each kind's map in the lane's map buffer
@@ -936,6 +937,8 @@ int make_group(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const std::vec
                     G.pp_grid[l] = std::max(G.pp_grid[l], (unsigned)mg_tiles(s->mgh.lv[l].I, s->mgh.lv[l].J));
             }
             G.mg_grid_d0 = std::max(G.mg_grid_d0, (unsigned)mg_d0_tiles(s->mgh.lv[1].I, s->mgh.lv[1].J));
+        } else {
+            G.ipp = true;
         }
         s->h.pblocks = (int)std::max<int64_t>(1, cdiv(std::max<int64_t>(s->n_bound, 1), kBlock));
         const Geo gs = geometry(s);
@@ -1225,18 +1228,21 @@ struct KProf {
 // cache, and the window's prologue and barriers cost more.
 bool ring_window(const Group& G) { return G.n == 1 && G.sc[0]->pcg_chunk >= 4 * (int64_t)G.sc[0]->J; }
 
-// One V-cycle z = M r over the scenes of S whose solve uses it; which: the
-// residual buffer (0: cr, 1: cr2).  Level-l launches cover the scenes that
-// have level l; a kind with no blocks is not launched.
-void launch_vcycle(const Group& G, hipStream_t st, const SolveLaunch& S, int which)
+// One V-cycle z = M r over the scenes of S whose solve uses it; it < 0: of
+// the residual that starts a sweep (cr), else of iteration it's, whose step
+// its first launch takes.  Level-l launches cover the scenes that have level
+// l; a kind with no blocks is not launched.
+void launch_vcycle(const Group& G, hipStream_t st, const SolveLaunch& S, int it)
 {
+    const int which = it < 0 || (it & 1) ? 0 : 1;   // the residual's buffer: even iterations write cr2
     // levels 1 .. t-1 one launch per step, levels t .. n-1 in k_mg_coarse
     // (t per scene; the maps and grids hold a level's blocks only for the
     // scenes that launch it)
     const int top = G.mg_top;
     if (S.blocks[1]) {
         KProf kp(G, FG_K_MG_DOWN0, true);
-        launch_mg_down0(S.grid(1), st, S.d, S.map[1], which);
+        if (it < 0) launch_mg_down0(S.grid(1), st, S.d, S.map[1], 0);
+        else launch_mg_step0(S.grid(1), st, S.d, S.map[1], it);
         kp.done(0);
     }
     if (G.fused) {
@@ -1284,8 +1290,8 @@ void launch_vcycle(const Group& G, hipStream_t st, const SolveLaunch& S, int whi
     kp.done(0);
 }
 
-// One PCG iteration it: p, q = A'p and p.q; r, x; z = M r (the V-cycle, when
-// the group uses it).
+// One PCG iteration it: p, q = A'p and p.q; r, x; z = M r (IPP scenes: one
+// kernel; the others: the V-cycle, whose first launch makes r and x).
 void launch_iteration(const Group& G, hipStream_t st, const SolveLaunch& S, int it)
 {
     {
@@ -1293,15 +1299,14 @@ void launch_iteration(const Group& G, hipStream_t st, const SolveLaunch& S, int 
         launch_pcg_a(S.grid(0), st, S.d, S.map[0], it);
         kp.done(0);   // units: at the end of the solve
     }
-    {
+    if (G.ipp) {
         KProf kp(G, FG_K_PCG_B, true);
         launch_pcg_b(S.grid(0), st, S.d, S.map[0], it);
         kp.done(0);
     }
     if (G.mg_levels) {
-        // the new residual: iteration it writes cr2 for even it, cr for odd
         KProf kp(G, FG_K_VCYCLE);
-        launch_vcycle(G, st, S, (it & 1) ? 0 : 1);
+        launch_vcycle(G, st, S, it);
         kp.done(0);
     }
 }
@@ -1390,7 +1395,7 @@ int run_solve(Group& G, bool rhs_from_grid)
         if (count == 0) break;
         if (G.mg_levels) {
             KProf kp(G, FG_K_VCYCLE);
-            launch_vcycle(G, st, S, 0);
+            launch_vcycle(G, st, S, -1);
             kp.done(0);
         }
         int it = 0;
@@ -1422,8 +1427,10 @@ int run_solve(Group& G, bool rhs_from_grid)
     for (fg_scene* s : G.sc) {
         const SceneScalars& h = *s->hsc;
         add_work(G.L, timed, FG_K_PCG_A, (int64_t)h.total_iters * s->C);
-        add_work(G.L, timed, FG_K_PCG_B, (int64_t)h.total_iters * s->C);
-        if (s->h.precond != kPrecondMG) continue;
+        if (s->h.precond != kPrecondMG) {
+            add_work(G.L, timed, FG_K_PCG_B, (int64_t)h.total_iters * s->C);
+            continue;
+        }
         const int64_t cycles = (int64_t)h.total_iters + h.sweeps;   // one per iteration and per sweep start
         add_work(G.L, timed, FG_K_VCYCLE, cycles * s->C);
         const MgLevel& L1 = s->mgh.lv[1];
@@ -1449,7 +1456,8 @@ int run_solve(Group& G, bool rhs_from_grid)
             }
         }
         add_work(G.L, timed, FG_K_MG_COARSE, cycles * mg_coarse_bytes(s));
-        add_work(G.L, timed, FG_K_MG_DOWN0, cycles * (5 * s->C + 5 * C1));
+        add_work(G.L, timed, FG_K_MG_DOWN0, (int64_t)h.sweeps * 5 * s->C + (int64_t)h.total_iters * 33 * s->C +
+                                                cycles * 5 * C1);
         add_work(G.L, timed, FG_K_MG_UP0, cycles * (9 * s->C + 4 * C1));
     }
     // a scene whose solve saw NaN/Inf stopped iterating (its flags say so);

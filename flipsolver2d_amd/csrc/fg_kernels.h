@@ -56,6 +56,7 @@ FG_DECLARE_LAUNCH(mg_galerkin, int l);
 FG_DECLARE_LAUNCH(mg_sym, int l);
 FG_DECLARE_LAUNCH(mg_symmark, int l, int nsym);
 FG_DECLARE_LAUNCH(mg_down0, const int2* map, int which);
+FG_DECLARE_LAUNCH(mg_step0, const int2* map, int it);
 FG_DECLARE_LAUNCH(mg_resid, const int2* map, int l);
 FG_DECLARE_LAUNCH(mg_restrict, const int2* map, int l);
 // max_halo: the largest MgLevels::thalo of the launch's scenes

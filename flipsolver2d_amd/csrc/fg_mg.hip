@@ -472,8 +472,17 @@ __global__ void __launch_bounds__(kBlock) k_mg_symmark(const SceneDev* scenes, i
 // per fine cell of the supports, then each thread sums its cell's 16
 // weighted res0.  Each value is formed by the same expression as it would
 // be per coarse cell, so r1 does not depend on the tiling.
+// kStep: the PCG step that makes r, fused: alpha from the partials of p.q,
+// r = r_old - alpha q over the patch (its halo formed again by each of the
+// tiles that need it, from the same values), r and x += alpha p (FP64)
+// written for the tile's own 2 kD0Tile x 2 kD0Tile fine cells.  On its own
+// that step is a launch that moves 32 B a cell and whose r this one reads
+// back; together 33 B, 27 % more of r_old, q and the code for the halo, and
+// one launch of an iteration's latency chain less: 9.4 -> 6.5 us at 128^2,
+// 94 -> 83 us at 4096^2 (the two kernels, this one).
 constexpr int kD0R = 2 * kD0Tile + 4;
-__global__ void __launch_bounds__(kBlock) k_mg_down0(const SceneDev* scenes, const int2* map, int which)
+template <bool kStep>
+__device__ __forceinline__ void mg_down0_tile(const SceneDev* scenes, const int2* map, int arg)
 {
     static_assert(kD0Tile * kD0Tile == kBlock, "one level-1 cell per thread");
     __shared__ float xs[kD0R][kD0R + 1];   // x0
@@ -481,6 +490,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_down0(const SceneDev* scenes, con
     __shared__ uint8_t cs[kD0R][kD0R + 4];
     const SceneBlock sb = scene_block(map, true);
     const SceneDev& s = scenes[sb.scene];
+    cptr<SceneScalars> scr = cst(s.sc);
     const auto& L1 = cst(s.mg)->lv[1];
     const int I1 = L1.I, J1 = L1.J;
     const int tjn = (J1 + kD0Tile - 1) / kD0Tile;
@@ -490,29 +500,67 @@ __global__ void __launch_bounds__(kBlock) k_mg_down0(const SceneDev* scenes, con
     const int ti = sb.block / tjn, tj = sb.block - ti * tjn;
     const int I = s.I, J = s.J;
     const int fi0 = 2 * kD0Tile * ti - 2, fj0 = 2 * kD0Tile * tj - 2;   // the patch's first fine cell
-    gptr<const float> r = gbl<const float>(which ? s.cr2 : s.cr);
+    const int it = arg;
+    gptr<const float> r = gbl<const float>(kStep ? ((it & 1) ? s.cr2 : s.cr) : (arg ? s.cr2 : s.cr));
+    gptr<float> rnew = gbl((it & 1) ? s.cr : s.cr2);
+    gptr<const float> q = gbl<const float>(s.cw);
+    gptr<const float> p = gbl<const float>((it & 1) ? s.cs1 : s.cp);
+    gptr<double> x = gbl(s.x64);
     gptr<const uint8_t> code = gbl<const uint8_t>(s.stencil);
     {   // code, r and x0 of the patch (outside the grid: code 0, r 0)
         constexpr int Q = (kD0R * kD0R + kBlock - 1) / kBlock;
         uint8_t kq[Q];
-        float vq[Q];
+        float vq[Q], qq[Q], pq[Q];
+        double xq[Q];
 #pragma unroll
         for (int u = 0; u < Q; u++) {
-            const int q = min((int)threadIdx.x + u * kBlock, kD0R * kD0R - 1);
-            const int fi = fi0 + q / kD0R, fj = fj0 + q % kD0R;
-            const int f = min(max(fi, 0), I - 1) * J + min(max(fj, 0), J - 1);   // clamped, not selected
+            const int k = min((int)threadIdx.x + u * kBlock, kD0R * kD0R - 1);
+            const int a = k / kD0R, b = k % kD0R;
+            const int f = min(max(fi0 + a, 0), I - 1) * J + min(max(fj0 + b, 0), J - 1);   // clamped, not selected
             kq[u] = code[f];
             vq[u] = r[f];
+            if constexpr (kStep) {
+                qq[u] = q[f];
+                // x and p are the own cells' alone: a halo lane loads an own cell's
+                const int g = min(max(fi0 + min(max(a, 2), kD0R - 3), 0), I - 1) * J +
+                              min(max(fj0 + min(max(b, 2), kD0R - 3), 0), J - 1);
+                xq[u] = x[g];
+                pq[u] = p[g];
+            }
+        }
+        float alpha = 0.f;
+        if constexpr (kStep) {
+            double t[1];
+            sum_partials<1>(s, kSlotPQ, s.pcg_blocks, t);
+            const bool lead = sb.block == 0 && threadIdx.x == 0;
+            if (!(t[0] > 0.0) || !finite_d(t[0])) {   // breakdown: end this sweep (every block sees it)
+                if (lead) s.sc->inner_done = 1;
+                return;
+            }
+            alpha = (float)(scr->gamma[it & 1] / t[0]);
+            if (lead) {
+                s.sc->inner_iters = it + 1;
+                s.sc->total_iters += 1;
+            }
         }
 #pragma unroll
         for (int u = 0; u < Q; u++) {
-            const int q = threadIdx.x + u * kBlock;
-            if (q >= kD0R * kD0R) break;
-            const int a = q / kD0R, b = q % kD0R;
+            const int k0 = threadIdx.x + u * kBlock;
+            if (k0 >= kD0R * kD0R) break;
+            const int a = k0 / kD0R, b = k0 % kD0R;
             const int fi = fi0 + a, fj = fj0 + b;
             const bool in = fi >= 0 && fi < I && fj >= 0 && fj < J;
             const uint8_t k = in ? kq[u] : 0;
-            const float rv = vq[u] * mask01(in);
+            float rv = vq[u];
+            if constexpr (kStep) {
+                rv = rv - alpha * qq[u];
+                if (in && a >= 2 && a < kD0R - 2 && b >= 2 && b < kD0R - 2) {
+                    const int f = fi * J + fj;
+                    rnew[f] = rv;
+                    x[f] = xq[u] + (double)alpha * (double)pq[u];
+                }
+            }
+            rv = rv * mask01(in);
             const float d = l1_diag0(k);
             xs[a][b] = ((k & 0x80) && d > 0.f) ? kMgOmega * rv / d : 0.f;
             rs[a][b] = rv;
@@ -549,6 +597,18 @@ __global__ void __launch_bounds__(kBlock) k_mg_down0(const SceneDev* scenes, con
             acc += (k & 0x80) ? (w1(a - 1) * w1(b - 1)) * rs[2 * li + a][2 * lj + b] : 0.f;
         }
     gbl(L1.r)[c] = 0.25f * acc;
+}
+
+// r as it is (which: 0 = cr, 1 = cr2): the V-cycle that starts a sweep
+__global__ void __launch_bounds__(kBlock) k_mg_down0(const SceneDev* scenes, const int2* map, int which)
+{
+    mg_down0_tile<false>(scenes, map, which);
+}
+
+// the step of PCG iteration it, then its V-cycle's first part
+__global__ void __launch_bounds__(kBlock) k_mg_step0(const SceneDev* scenes, const int2* map, int it)
+{
+    mg_down0_tile<true>(scenes, map, it);
 }
 
 // Level l (1 <= l < t): x = r * dinv, y = res = r - A_l x.
@@ -1218,6 +1278,7 @@ void launch_mg_symmark(dim3 g, hipStream_t st, const SceneDev* sc, int l, int ns
     fg_launch(k_mg_symmark, g, dim3(kBlock), st, sc, l, nsym);
 }
 FG_MG_LAUNCH_MAP(mg_down0, int, which)
+FG_MG_LAUNCH_MAP(mg_step0, int, it)
 FG_MG_LAUNCH_MAP(mg_resid, int, l)
 FG_MG_LAUNCH_MAP(mg_restrict, int, l)
 FG_MG_LAUNCH_MAP(mg_prolong, int, l)

@@ -25,7 +25,8 @@
 // matrix-free IPP (PressureIPPCoeficients.h:23-40) is mis-scaled and not
 // symmetric and does not converge; it is reproduced only in the oracle.
 //
-// Each PCG iteration is two single-pass kernels:
+// Each PCG iteration is two single-pass kernels (with the V-cycle KB is part
+// of its first launch, k_mg_step0, and z comes from its last):
 //   KA(it): rho, ||r||^2 <- partials of KB(it-1); stop test; beta;
 //           p = z + beta p_old (recomputed at the 4 neighbours), q = A' p, p.q
 //   KB(it): p.q <- partials of KA(it); alpha; r = r_old - alpha q (recomputed
@@ -309,8 +310,8 @@ __global__ void __launch_bounds__(kBlock) k_pcg_a(const SceneDev* scenes, const 
     put_partials<1>(s, kSlotPQ, v, sb.block);
 }
 
-// KB: r = r_old - alpha q; x += alpha p (FP64); z = M r; r.z, r.r (with the
-// IPP; with the V-cycle, r and x only)
+// KB: r = r_old - alpha q; x += alpha p (FP64); z = M r; r.z, r.r, with the
+// IPP (with the V-cycle, r and x are k_mg_step0's, z and the sums k_mg_up0's)
 __global__ void __launch_bounds__(kBlock) k_pcg_b(const SceneDev* scenes, const int2* map, int it)
 {
     const SceneBlock sb = scene_block(map, true);
@@ -319,7 +320,8 @@ __global__ void __launch_bounds__(kBlock) k_pcg_b(const SceneDev* scenes, const 
     cptr<SceneScalars> scr = cst(sc);   // values earlier kernels wrote: scalar loads
     const int nb = s.pcg_blocks;
     // one test after the uniform loads, so that they issue together
-    if (!s.active | (scr->outer_done != 0) | (scr->inner_done != 0) | (sb.block >= nb)) return;
+    if (!s.active | (s.precond == kPrecondMG) | (scr->outer_done != 0) | (scr->inner_done != 0) | (sb.block >= nb))
+        return;
     const int J = s.J, C = s.I * s.J;
     gptr<const float> rold = gbl<const float>((it & 1) ? s.cr2 : s.cr);
     gptr<float> rnew = gbl((it & 1) ? s.cr : s.cr2);
@@ -329,50 +331,6 @@ __global__ void __launch_bounds__(kBlock) k_pcg_b(const SceneDev* scenes, const 
     gptr<double> x = gbl(s.x64);
     gptr<const uint8_t> code = gbl<const uint8_t>(s.stencil);
     const Chunk ch = my_chunk(s, sb.block);
-    if (s.precond == kPrecondMG) {
-        // r and x only; the V-cycle that follows forms z, r.z and r.r.  A
-        // pass's loads (kItems cells a thread, clamped to the chunk) are
-        // issued before its stores -- and the first pass's before the p.q
-        // reduction -- since the compiler cannot move a load of r_old above
-        // a store to r_new.
-        float a = 0.f;
-        for (int base = ch.begin; base < ch.end; base += kPass) {
-            float ro[kItems], qc[kItems], pc[kItems];
-            double xc[kItems];
-#pragma unroll
-            for (int k = 0; k < kItems; k++) {
-                const int c = min(base + (int)threadIdx.x + k * kBlock, ch.end - 1);
-                ro[k] = rold[c];
-                qc[k] = q[c];
-                xc[k] = x[c];
-                pc[k] = pnew[c];
-            }
-            if (base == ch.begin) {
-                double t[1];
-                sum_partials<1>(s, kSlotPQ, nb, t);
-                const double pq = t[0];
-                const bool lead = sb.block == 0 && threadIdx.x == 0;
-                if (!(pq > 0.0) || !finite_d(pq)) {
-                    if (lead) sc->inner_done = 1;
-                    return;
-                }
-                a = (float)(scr->gamma[it & 1] / pq);
-                if (lead) {
-                    sc->inner_iters = it + 1;
-                    sc->total_iters += 1;
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < kItems; k++) {
-                const int c = base + (int)threadIdx.x + k * kBlock;
-                if (c < ch.end) {
-                    rnew[c] = ro[k] - a * qc[k];
-                    x[c] = xc[k] + (double)a * (double)pc[k];
-                }
-            }
-        }
-        return;
-    }
     double rz = 0.0, rr = 0.0;
     float alpha = 0.f;
     for (int base = ch.begin; base < ch.end; base += kPass) {

@@ -286,7 +286,9 @@ int fg_batch_autotune_tiling(fg_ctx* ctx, fg_scene* const* scenes, int32_t n, in
  *   PARTICLES    36 P + 8 F + 4 C      (k_advect + k_g2p_count: positions and
  *                                       velocities read and written, keys; U, V,
  *                                       saved U, saved V; solid SDF)
- *   MG_DOWN0     5 C + 5 C1 per V-cycle (stencil code, r; level-1 activity, r1)
+ *   MG_DOWN0     33 C + 5 C1 per iteration (stencil code, r_old, q, p; x read and
+ *                written, r written; level-1 activity, r1), 5 C + 5 C1 for the
+ *                V-cycle that starts a sweep (code, r)
  *   MG_UP0       9 C + 4 C1 per V-cycle (code, r, z; level-1 y)
  *   MG_RESID     per V-cycle, over every level l between level 1 and the
  *                coarse block: 9 C_l + 100 S_l (r, dinv; r_{l+1} written,
@@ -307,7 +309,8 @@ enum fg_kernel_id {
     FG_K_LEVELSET = 4,    /* [C] */
     FG_K_EXTRAPOLATE = 5, /* [C] (faces) */
     FG_K_PCG_A = 6,       /* [C] per iteration (17 B a cell) */
-    FG_K_PCG_B = 7,       /* [C] per iteration (32 B a cell) */
+    FG_K_PCG_B = 7,       /* [C] per iteration (32 B a cell), IPP solves; with the V-cycle r and x
+                           * are formed in its first launch (MG_DOWN0) */
     FG_K_G2P = 8,         /* [P] */
     FG_K_RHS = 9,         /* [C] */
     FG_K_APPLY = 10,      /* [C] */
@@ -316,7 +319,7 @@ enum fg_kernel_id {
                            * every level between level 1 and the coarse block (per-level
                            * kernels, see fg_ctx_set_vcycle_fused: the level-1 residual) */
     FG_K_MG_COARSE = 13,  /* [B] the V-cycle's coarse-levels launch (one block per scene) */
-    FG_K_MG_DOWN0 = 14,   /* [B] level-0 smoothing, residual and restriction */
+    FG_K_MG_DOWN0 = 14,   /* [B] the iteration's step (r, x), level-0 smoothing, residual and restriction */
     FG_K_MG_UP0 = 15,     /* [B] prolongation to level 0 and post-smoothing */
     FG_K_PARTICLES = 16,  /* [B] k_advect and k_g2p_count together (G2P + advection) */
     FG_K_MG_PP = 17,      /* [B] the V-cycle's prolongation + post-smoothing launches, k_mg_pp
