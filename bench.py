@@ -75,7 +75,7 @@ KERNEL_BYTES = {
     "pcg_a": ("K_PCG_A", 17.0, "cells", ["k_pcg_a"]),
     "pcg_b": ("K_PCG_B", 32.0, "cells", ["k_pcg_b"]),
     "mg_down0": ("K_MG_DOWN0", 1.0, "bytes", ["k_mg_step0", "k_mg_down0"]),
-    "mg_up0": ("K_MG_UP0", 1.0, "bytes", ["k_mg_up0", "k_mg_up0_wide"]),
+    "mg_up0": ("K_MG_UP0", 1.0, "bytes", ["k_mg_up0"]),
     "mg_resid": ("K_MG_RESID", 1.0, "bytes", ["k_mg_rr"]),
     "mg_pp": ("K_MG_PP", 1.0, "bytes", ["k_mg_pp"]),
     "mg_coarse": ("K_MG_COARSE", 1.0, "bytes", ["k_mg_coarse"]),

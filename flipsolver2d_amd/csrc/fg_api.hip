@@ -54,11 +54,13 @@ int fail(int code, const std::string& msg)
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Block maps of the solve's per-iteration launches, by kind: 0 = solver
-// chunks, 1 = level-1 tiles of kVcTile (k_mg_down0, and k_mg_pp of level 1);
+// chunks, kUpKind = the blocks of k_mg_up0 (no scene has that many levels),
+// 1 = level-1 tiles of kVcTile (k_mg_down0, and k_mg_pp of level 1);
 // with the fused V-cycle l = level-l tiles of kRRTile (2 <= l <= t: k_mg_rr
 // of level l-1) and kMgMaxLevels + l = level-l tiles of kVcTile (2 <= l < t:
 // k_mg_pp of level l), else 1 + l = level-l cells one per thread (1 <= l < t).
 constexpr int kMapKinds = 2 * kMgMaxLevels;
+constexpr int kUpKind = kMgMaxLevels;
 // the kind of k_mg_pp's launch over level l (fused)
 inline int pp_kind(int l) { return l == 1 ? 1 : kMgMaxLevels + l; }
 constexpr int kMapMaxScenes = 4096;   // scenes one map build handles (LDS prefix)
@@ -697,6 +699,7 @@ __device__ int map_blocks(const SceneDev& s, int kind, bool fused)
 {
     if (kind == 0) return s.pcg_blocks;
     if (s.precond != kPrecondMG) return 0;
+    if (kind == kUpKind) return s.up_blocks;
     const MgLevels& M = *s.mg;
     if (kind == 1) return mg_d0_tiles(M.lv[1].I, M.lv[1].J);
     if (fused) {
@@ -714,6 +717,7 @@ int64_t map_blocks_host(const fg_scene* s, int kind, bool fused)
 {
     if (kind == 0) return s->pcg_blocks;
     if (s->h.precond != kPrecondMG) return 0;
+    if (kind == kUpKind) return s->h.up_blocks;
     const MgLevels& M = s->mgh;
     if (kind == 1) return mg_d0_tiles(M.lv[1].I, M.lv[1].J);
     if (fused) {
@@ -797,7 +801,6 @@ struct Group {
     int64_t cells = 0, faces = 0, parts = 0;
     int max_inner = 0;
     int max_bands = 0;
-    int max_j = 0;                      // the widest scene's J
     bool sources = false;               // some scene has SOURCE cells (afterTransfer, reseeding)
     bool nb = false;                    // NB-FLIP scenes (a group holds one solver class)
     bool visc = false;                  // some scene has viscosity enabled
@@ -813,6 +816,7 @@ struct Group {
     unsigned rr_grid[kMgMaxLevels]{};   // kRRTile tiles of level l (2 <= l <= t): k_mg_rr's blocks a scene
     unsigned pp_grid[kMgMaxLevels]{};   // kVcTile tiles of level l (l < t): k_mg_pp's blocks a scene
     bool fused = true;                  // the context's vcycle_fused when the group was made
+    unsigned up_grid = 0;               // blocks per scene of k_mg_up0
     unsigned mg_grid_d0 = 0;            // blocks per scene of k_mg_down0 (level-1 tiles)
 };
 
@@ -881,6 +885,12 @@ void apply_tiling(const fg_ctx* ctx, fg_scene* s)
     s->pcg_blocks = (int)blocks;
     s->h.pcg_chunk = s->pcg_chunk;
     s->h.pcg_blocks = s->pcg_blocks;
+    // k_mg_up0's tiles: as many to a block as the least chunk holds, more
+    // where the blocks or the partials run out
+    const int64_t tiles = cdiv(s->I, kUpTile) * cdiv(s->J, kUpTile);
+    const int64_t least = cdiv(tiles, std::max(1, ctx->pcg_min_chunk / (kUpTile * kUpTile)));
+    const int64_t ub = std::min<int64_t>({least, ctx->pcg_target_blocks, s->max_blocks});
+    s->h.up_blocks = (int)cdiv(tiles, cdiv(tiles, ub));   // every block has a tile
 }
 
 int ensure_group_buffers(Lane* L, int n)
@@ -937,6 +947,7 @@ int make_group(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const std::vec
                     G.pp_grid[l] = std::max(G.pp_grid[l], (unsigned)mg_tiles(s->mgh.lv[l].I, s->mgh.lv[l].J));
             }
             G.mg_grid_d0 = std::max(G.mg_grid_d0, (unsigned)mg_d0_tiles(s->mgh.lv[1].I, s->mgh.lv[1].J));
+            G.up_grid = std::max(G.up_grid, (unsigned)s->h.up_blocks);
         } else {
             G.ipp = true;
         }
@@ -946,7 +957,6 @@ int make_group(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const std::vec
         else geo_max(G.g, gs);
         first = false;
         G.cells += s->C;
-        G.max_j = std::max(G.max_j, s->J);
         G.faces += s->FU + s->FV;
         G.parts += s->n_bound;
         G.max_inner = std::max(G.max_inner, s->h.max_inner);
@@ -960,7 +970,7 @@ int make_group(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const std::vec
     // capacity = every scene's blocks, the bound for any packed subset
     if (G.n > 1 && G.n <= kMapMaxScenes) {
         // pcg, down0, and levels 1 .. t-1 (fused: through k_mg_pp of level t-1)
-        G.map_kinds = G.fused ? kMgMaxLevels + G.mg_top : G.mg_top + 1;
+        G.map_kinds = G.fused ? kMgMaxLevels + std::max(G.mg_top, 1) : kUpKind + 1;
         int64_t cap[kMapKinds] = {};
         for (fg_scene* s : scenes)
             for (int k = 0; k < G.map_kinds; k++) cap[k] += map_blocks_host(s, k, G.fused);
@@ -1056,13 +1066,14 @@ SolveLaunch group_launch(const Group& G, const SceneDev* d, unsigned ny)
     S.ny = ny;
     S.blocks[0] = G.g.pcg.x;
     S.blocks[1] = G.mg_grid_d0;
+    S.blocks[kUpKind] = G.up_grid;
     if (G.fused)
         for (int l = 2; l < kMgMaxLevels; l++) {
             S.blocks[l] = G.rr_grid[l];
             S.blocks[pp_kind(l)] = G.pp_grid[l];
         }
     else
-        for (int l = 1; l < kMgMaxLevels; l++) S.blocks[1 + l] = G.vc_grid[l];
+        for (int l = 1; l < G.mg_top; l++) S.blocks[1 + l] = G.vc_grid[l];
     return S;
 }
 
@@ -1219,15 +1230,6 @@ struct KProf {
 // scenes of the group run the same sweep and iteration index in lock step;
 // a scene whose solve has stopped skips the launches that remain.
 // ---------------------------------------------------------------------------
-// Whether k_mg_up0 forms the neighbours' smoothing starts in an LDS window
-// over the chunk's rows rather than per cell: for a single scene whose
-// chunks span four rows or more (on one-row chunks and on batches of small
-// scenes the per-cell kernel is faster).  The same window for k_pcg_a's
-// direction (a 4096^2 projection) took 70 us a launch against 51 us per
-// cell: there the neighbours' rows it saves come back from the last-level
-// cache, and the window's prologue and barriers cost more.
-bool ring_window(const Group& G) { return G.n == 1 && G.sc[0]->pcg_chunk >= 4 * (int64_t)G.sc[0]->J; }
-
 // One V-cycle z = M r over the scenes of S whose solve uses it; it < 0: of
 // the residual that starts a sweep (cr), else of iteration it's, whose step
 // its first launch takes.  Level-l launches cover the scenes that have level
@@ -1286,7 +1288,7 @@ void launch_vcycle(const Group& G, hipStream_t st, const SolveLaunch& S, int it)
         }
     }
     KProf kp(G, FG_K_MG_UP0, true);
-    launch_mg_up0(S.grid(0), st, S.d, S.map[0], which, G.max_j, ring_window(G));
+    launch_mg_up0(S.grid(kUpKind), st, S.d, S.map[kUpKind], which);
     kp.done(0);
 }
 

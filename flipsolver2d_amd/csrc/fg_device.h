@@ -32,6 +32,7 @@ __host__ __device__ inline int mg_d0_tiles(int I1, int J1)
 {
     return ((I1 + kD0Tile - 1) / kD0Tile) * ((J1 + kD0Tile - 1) / kD0Tile);
 }
+constexpr int kUpTile = 32;              // k_mg_up0: cells a tile, per side
 constexpr int kVcTile = 16;              // k_mg_pp: level-l cells a block, per side
 constexpr int kRRTile = 8;               // k_mg_rr: level-(l+1) cells a block, per side
 // blocks of a fused V-cycle launch over a level of I x J cells in tiles of t x t
@@ -147,6 +148,7 @@ struct SceneDev {
     int32_t max_blocks;     // stride of the FP64 partials array (>= pcg_blocks)
     int32_t pcg_blocks;     // solver blocks of this scene
     int32_t pcg_chunk;      // cells per solver block (multiple of kBlock)
+    int32_t up_blocks;      // blocks (partials) of k_mg_up0, each a run of kUpTile x kUpTile tiles
     int32_t max_pblocks;    // stride of the particle partials arrays
     int32_t pblocks;        // particle blocks of this scene's current launches (<= max_pblocks)
     int32_t precond;        // kPrecondMG or kPrecondIPP

@@ -65,9 +65,7 @@ FG_DECLARE_LAUNCH(mg_prolong, const int2* map, int l);
 FG_DECLARE_LAUNCH(mg_post, const int2* map, int l);
 FG_DECLARE_LAUNCH(mg_rr, const int2* map, int l);
 FG_DECLARE_LAUNCH(mg_pp, const int2* map, int l);
-// max_j: the largest J of the launch's scenes (sizes the LDS of k_mg_up0);
-// ring: k_mg_up0 (its LDS window) rather than k_mg_up0_wide
-FG_DECLARE_LAUNCH(mg_up0, const int2* map, int which, int max_j, bool ring);
+FG_DECLARE_LAUNCH(mg_up0, const int2* map, int which);
 
 FG_DECLARE_LAUNCH(max_v2);
 FG_DECLARE_LAUNCH(advect, int alive_from_key);

@@ -1065,196 +1065,121 @@ __global__ void __launch_bounds__(kBlock) k_mg_post(const SceneDev* scenes, cons
 
 // Level 0, up: z0 = w r / D1 + P y1 at the cell and its fluid neighbours, then
 // z = z0 + w (r - A' z0) / D1; z = r on non-fluid rows.  Writes z and the
-// partials of r.z and r.r the next PCG iteration reduces (solver chunks).
-// z0 of a fine cell depends on that cell alone, so a block forms it once
-// per cell into an LDS ring over the flat cell index (slot f mod RB, RB =
-// 2J + 2 kUpPass floats of dynamic LDS) instead of once per neighbour.
-// Pass p covers cells p .. p + kUpPass - 1, thread t taking p + t + u kBlock
-// (u = 0 .. kUpItems - 1: the cells and their order of a plain kBlock
-// stride, so the partials keep their order), and reads the ring over
-// [p - J, p + J + kUpPass); the prologue fills the first pass's window,
-// each pass the cells the next one adds (their loads issued first; their
-// slots are those of the cells just behind this pass's window).  The
-// window costs a prologue of 2J + kUpPass cells per block and a barrier per
-// pass: it pays where chunks span several rows of a grid too large for the
-// L2 to keep the neighbouring rows (4096^2); on one-row chunks (1024^2) and
-// on batches of small scenes k_mg_up0_wide is faster, and the host
-// launches that there.
-constexpr int kUpItems = 4;
-constexpr int kUpPass = kUpItems * kBlock;
-constexpr int kUpMaxJ = (16384 - 2 * kUpPass) / 2;   // the ring within 64 KB
+// partials of r.z and r.r the next PCG iteration reduces.
+// A block owns kUpTile x kUpTile tiles of the grid (one, or a run of
+// consecutive ones: SceneDev::up_blocks blocks a scene, a partial each) and
+// stages in LDS the tile with a one-cell halo, code and r, and the level-1
+// patch under it, so z0 is formed once per cell (and once more per halo
+// cell) from LDS instead of five times from 30 global loads, which bound
+// the per-cell form by instruction issue.  The quotients by D1, an integer
+// up to 8, are a product with its reciprocal and one step with the exact
+// remainder (correctly rounded, as the division).  A tile is the fine side of
+// k_mg_step0's, in its order, so what one of them writes the
+// other reads through the same XCD's L2.  Per-cell form (each cell its
+// neighbours' z0) 8.3 us at 128^2, 10.1 us at 1024^2; an LDS window of whole
+// rows over linear chunks 97 us at 4096^2; this form 5.7, 8.2 and 39 us.
+constexpr int kUpR = kUpTile + 2;        // cells a side with the halo
+constexpr int kUpY = kUpTile / 2 + 2;    // level-1 cells a side that the halo's cells prolong from
+static_assert(kUpTile % 2 == 0 && kUpTile * kUpTile % kBlock == 0 && kBlock % kUpTile == 0, "whole rows of a tile a pass");
+
 __global__ void __launch_bounds__(kBlock) k_mg_up0(const SceneDev* scenes, const int2* map, int which)
 {
-    extern __shared__ float zr[];
+    __shared__ float zs[kUpR][kUpR + 1];     // z0
+    __shared__ float rs[kUpR][kUpR + 1];
+    __shared__ uint8_t cs[kUpR][kUpR + 2];
+    __shared__ float ys[kUpY][kUpY + 1];
+    __shared__ float inv[9];                 // 1 / D1
     const SceneBlock sb = scene_block(map, true);
     const SceneDev& s = scenes[sb.scene];
     const auto& L1 = cst(s.mg)->lv[1];
-    if (!mg_iterating(s) | (sb.block >= s.pcg_blocks)) return;
-    const int I = s.I, J = s.J, C = I * J;
+    if (!mg_iterating(s) | (sb.block >= s.up_blocks)) return;
+    const int I = s.I, J = s.J, I1 = L1.I, J1 = L1.J;
     gptr<const float> y1 = gbl<const float>(L1.y);
-    const int I1 = L1.I, J1 = L1.J;
     gptr<const float> r = gbl<const float>(which ? s.cr2 : s.cr);
     gptr<const uint8_t> code = gbl<const uint8_t>(s.stencil);
     gptr<float> z = gbl(s.cu);
-    const Chunk ch = my_chunk(s, sb.block);
-    const int RB = 2 * J + 2 * kUpPass;
-    // z0 of cell f from its code, r and P y1 at it
-    auto z0_of = [&](uint8_t kf, float rf, float pg) {
-        const float dg = l1_diag0(kf);
-        return (dg > 0.f ? kMgOmega * rf / dg : 0.f) + pg;
+    const int tilesJ = (J + kUpTile - 1) / kUpTile, tiles = ((I + kUpTile - 1) / kUpTile) * tilesJ;
+    const int per = (tiles + s.up_blocks - 1) / s.up_blocks;
+    const int t1 = min(tiles, (sb.block + 1) * per);
+    if (threadIdx.x < 9) inv[threadIdx.x] = threadIdx.x ? 1.0f / (float)threadIdx.x : 0.f;
+    // w x / D1 (0 where D1 is)
+    auto over_d = [&](float x, int d) {
+        const float n = kMgOmega * x, rd = inv[d], q = n * rd;
+        return d > 0 ? __builtin_fmaf(__builtin_fmaf(-(float)d, q, n), rd, q) : 0.f;
     };
-    {   // prologue: the first pass's window
-        const int lo = max(ch.begin - J, 0), hi = min(ch.begin + J + kUpPass, C);
-        for (int f0 = lo; f0 < hi; f0 += kUpPass) {
-            uint8_t kq[kUpItems];
-            float rq[kUpItems], pq[kUpItems];
-#pragma unroll
-            for (int u = 0; u < kUpItems; u++) {
-                const int f = min(f0 + (int)threadIdx.x + u * kBlock, hi - 1);   // clamped, not selected
-                const int fi = f / J, fj = f - fi * J;
-                kq[u] = code[f];
-                rq[u] = r[f];
-                pq[u] = prolong_at(y1, I1, J1, fi, fj);
-            }
-#pragma unroll
-            for (int u = 0; u < kUpItems; u++) {
-                const int f = f0 + threadIdx.x + u * kBlock;
-                if (f < hi) zr[f % RB] = z0_of(kq[u], rq[u], pq[u]);
-            }
-        }
-    }
-    __syncthreads();
-    const int di[5] = {0, -1, 1, 0, 0}, dj[5] = {0, 0, 0, -1, 1};
+    auto l1 = [](uint8_t k) { return ((k >> 4) & 7) + __popc(k & 15u); };
     double rz = 0.0, rr = 0.0;
-    int sp = ch.begin % RB;   // the ring slot of cell p
-    for (int p = ch.begin; p < ch.end; p += kUpPass) {
-        // the cells this thread adds for the next pass, and its own cells'
-        // code and r: loads first
-        const bool more = p + kUpPass < ch.end;
-        uint8_t kf[kUpItems], kc[kUpItems];
-        float rf[kUpItems], pf[kUpItems], rcv[kUpItems];
+    for (int tile = sb.block * per; tile < t1; tile++) {
+        const int ti = tile / tilesJ, i0 = kUpTile * ti, j0 = kUpTile * (tile - ti * tilesJ);
+        constexpr int Q = (kUpR * kUpR + kBlock - 1) / kBlock, QY = (kUpY * kUpY + kBlock - 1) / kBlock;
+        uint8_t kq[Q];
+        float vq[Q], yq[QY];
 #pragma unroll
-        for (int u = 0; u < kUpItems; u++) {
-            const int fc = min(p + J + kUpPass + (int)threadIdx.x + u * kBlock, C - 1);
-            const int fi = fc / J, fj = fc - fi * J;
-            kf[u] = code[fc];
-            rf[u] = r[fc];
-            pf[u] = prolong_at(y1, I1, J1, fi, fj);
-            const int c = min(p + (int)threadIdx.x + u * kBlock, ch.end - 1);
-            kc[u] = code[c];
-            rcv[u] = r[c];
+        for (int u = 0; u < Q; u++) {
+            const int k = min((int)threadIdx.x + u * kBlock, kUpR * kUpR - 1);
+            const int f = min(max(i0 - 1 + k / kUpR, 0), I - 1) * J + min(max(j0 - 1 + k % kUpR, 0), J - 1);
+            kq[u] = code[f];
+            vq[u] = r[f];
         }
 #pragma unroll
-        for (int u = 0; u < kUpItems; u++) {
-            const int c = p + threadIdx.x + u * kBlock;
-            if (c >= ch.end) break;
-            const uint8_t k = kc[u];
-            const float rc = rcv[u];
-            float zc = rc;
-            if (k & 0x80) {
-                const int ci = c / J, cj = c - ci * J;
-                // the fluid neighbours that enter A' (not the row-wrapping coupling)
-                bool use[5];
-                use[0] = true;
+        for (int u = 0; u < QY; u++) {
+            const int k = min((int)threadIdx.x + u * kBlock, kUpY * kUpY - 1);
+            const int ci = i0 / 2 - 1 + k / kUpY, cj = j0 / 2 - 1 + k % kUpY;
+            const bool ok = ci >= 0 && ci < I1 && cj >= 0 && cj < J1;
+            yq[u] = y1[min(max(ci, 0), I1 - 1) * J1 + min(max(cj, 0), J1 - 1)] * mask01(ok);
+        }
+        __syncthreads();   // the tile before is done with the LDS
 #pragma unroll
-                for (int e = 1; e < 5; e++) use[e] = (k & (1 << (e - 1))) != 0;
-                use[3] = use[3] && cj > 0;
-                use[4] = use[4] && cj < J - 1;
-                int sc0 = sp + (int)threadIdx.x + u * kBlock;
-                sc0 -= sc0 >= RB ? RB : 0;
-                float z0[5];
-#pragma unroll
-                for (int e = 0; e < 5; e++) {
-                    const int gi = min(max(ci + di[e], 0), I - 1), gj = min(max(cj + dj[e], 0), J - 1);
-                    int sg = sc0 + (gi - ci) * J + (gj - cj);
-                    sg += sg < 0 ? RB : 0;
-                    sg -= sg >= RB ? RB : 0;
-                    z0[e] = use[e] ? zr[sg] : 0.f;
-                }
-                const float dc = l1_diag0(k);
-                float ax = (float)((k >> 4) & 7) * z0[0];
-#pragma unroll
-                for (int e = 1; e < 5; e++) ax -= z0[e];
-                zc = ((k & 0x80) && dc > 0.f) ? z0[0] + kMgOmega * (rc - ax) / dc : rc;
-                rz += (double)rc * (double)zc;
-            } else {   // identity row: z = r
-                rz += (double)rc * (double)rc;
-            }
-            z[c] = zc;
-            rr += (double)rc * (double)rc;
+        for (int u = 0; u < Q; u++) {
+            const int k = threadIdx.x + u * kBlock;
+            if (k >= kUpR * kUpR) break;
+            cs[k / kUpR][k % kUpR] = kq[u];
+            rs[k / kUpR][k % kUpR] = vq[u];
         }
 #pragma unroll
-        for (int u = 0; u < kUpItems; u++) {
-            const int f = p + J + kUpPass + threadIdx.x + u * kBlock;
-            if (more && f < C) zr[f % RB] = z0_of(kf[u], rf[u], pf[u]);
+        for (int u = 0; u < QY; u++) {
+            const int k = threadIdx.x + u * kBlock;
+            if (k < kUpY * kUpY) ys[k / kUpY][k % kUpY] = yq[u];
         }
         __syncthreads();
-        sp += kUpPass;
-        sp -= sp >= RB ? RB : 0;
-    }
-    double v[2] = {rz, rr};
-    put_partials<2>(s, kSlotCG, v, sb.block);
-}
-
-// k_mg_up0 for grids wider than its LDS window allows: each cell forms the
-// smoothing start z0 of its fluid neighbours itself (the same values).
-__global__ void __launch_bounds__(kBlock) k_mg_up0_wide(const SceneDev* scenes, const int2* map, int which)
-{
-    const SceneBlock sb = scene_block(map, true);
-    const SceneDev& s = scenes[sb.scene];
-    const auto& L1 = cst(s.mg)->lv[1];
-    if (!mg_iterating(s) | (sb.block >= s.pcg_blocks)) return;
-    const int J = s.J;
-    gptr<const float> y1 = gbl<const float>(L1.y);
-    const int I1 = L1.I, J1 = L1.J;
-    gptr<const float> r = gbl<const float>(which ? s.cr2 : s.cr);
-    gptr<const uint8_t> code = gbl<const uint8_t>(s.stencil);
-    gptr<float> z = gbl(s.cu);
-    const Chunk ch = my_chunk(s, sb.block);
-    double rz = 0.0, rr = 0.0;
-    for (int c = ch.begin + threadIdx.x; c < ch.end; c += kBlock) {
-        const uint8_t k = code[c];
-        const float rc = r[c];
-        if (!(k & 0x80)) {   // identity row: z = r, no neighbourhood
-            z[c] = rc;
-            rz += (double)rc * (double)rc;
+        // z0 of the tile and its halo (outside the grid: not used)
+#pragma unroll
+        for (int u = 0; u < Q; u++) {
+            const int k = threadIdx.x + u * kBlock;
+            if (k >= kUpR * kUpR) break;
+            const int a = k / kUpR, b = k % kUpR;   // cell (i0 - 1 + a, j0 - 1 + b), i0 and j0 even
+            // prolong_at on the patch, whose first cell is (i0 / 2 - 1, j0 / 2 - 1): an
+            // even cell (odd a) takes its own parent and the one before, an odd one the next
+            const int p0 = (a + 1) >> 1, q0 = (b + 1) >> 1;
+            const int p1 = (a & 1) ? p0 - 1 : p0 + 1, q1 = (b & 1) ? q0 - 1 : q0 + 1;
+            float acc = 0.f;
+            acc += (0.75f * 0.75f) * ys[p0][q0];
+            acc += (0.75f * 0.25f) * ys[p0][q1];
+            acc += (0.25f * 0.75f) * ys[p1][q0];
+            acc += (0.25f * 0.25f) * ys[p1][q1];
+            zs[a][b] = over_d(vq[u], l1(kq[u])) + acc;
+        }
+        __syncthreads();
+        const int b = 1 + (int)threadIdx.x % kUpTile, j = j0 + b - 1;
+#pragma unroll
+        for (int u = 0; u < kUpTile * kUpTile / kBlock; u++) {
+            const int a = 1 + (int)threadIdx.x / kUpTile + u * (kBlock / kUpTile), i = i0 + a - 1;
+            if (i >= I || j >= J) continue;
+            const uint8_t k = cs[a][b];
+            const float rc = rs[a][b];
+            // the fluid neighbours that enter A' (not the row-wrapping coupling)
+            const float z0 = zs[a][b];
+            float ax = (float)((k >> 4) & 7) * z0;
+            ax -= (k & 1) ? zs[a - 1][b] : 0.f;
+            ax -= (k & 2) ? zs[a + 1][b] : 0.f;
+            ax -= ((k & 4) && j > 0) ? zs[a][b - 1] : 0.f;
+            ax -= ((k & 8) && j < J - 1) ? zs[a][b + 1] : 0.f;
+            const int d = l1(k);
+            const float zc = ((k & 0x80) && d > 0) ? z0 + over_d(rc - ax, d) : rc;
+            z[i * J + j] = zc;
+            rz += (double)rc * (double)zc;
             rr += (double)rc * (double)rc;
-            continue;
         }
-        const int ci = c / J, cj = c - ci * J;
-        const int di[5] = {0, -1, 1, 0, 0}, dj[5] = {0, 0, 0, -1, 1};
-        // the fluid neighbours that enter A' (not the row-wrapping coupling)
-        bool use[5];
-        use[0] = true;
-#pragma unroll
-        for (int e = 1; e < 5; e++) use[e] = (k & (1 << (e - 1))) != 0;
-        use[3] = use[3] && cj > 0;
-        use[4] = use[4] && cj < J - 1;
-        uint8_t kg[5];
-        float rg[5], pg[5];
-        const int I = s.I;
-#pragma unroll
-        for (int e = 0; e < 5; e++) {
-            // clamped coordinates (not a select of c), so every load issues
-            const int gi = min(max(ci + di[e], 0), I - 1), gj = min(max(cj + dj[e], 0), J - 1);
-            kg[e] = code[gi * J + gj];
-            rg[e] = r[gi * J + gj];
-            pg[e] = prolong_at(y1, I1, J1, gi, gj);
-        }
-        float z0[5];
-#pragma unroll
-        for (int e = 0; e < 5; e++) {
-            const float dg = l1_diag0(kg[e]);
-            z0[e] = use[e] ? (dg > 0.f ? kMgOmega * rg[e] / dg : 0.f) + pg[e] : 0.f;
-        }
-        const float dc = l1_diag0(k);
-        float ax = (float)((k >> 4) & 7) * z0[0];
-#pragma unroll
-        for (int e = 1; e < 5; e++) ax -= z0[e];
-        const float zc = ((k & 0x80) && dc > 0.f) ? z0[0] + kMgOmega * (rc - ax) / dc : rc;
-        z[c] = zc;
-        rz += (double)rc * (double)zc;
-        rr += (double)rc * (double)rc;
     }
     double v[2] = {rz, rr};
     put_partials<2>(s, kSlotCG, v, sb.block);
@@ -1279,19 +1204,13 @@ void launch_mg_symmark(dim3 g, hipStream_t st, const SceneDev* sc, int l, int ns
 }
 FG_MG_LAUNCH_MAP(mg_down0, int, which)
 FG_MG_LAUNCH_MAP(mg_step0, int, it)
+FG_MG_LAUNCH_MAP(mg_up0, int, which)
 FG_MG_LAUNCH_MAP(mg_resid, int, l)
 FG_MG_LAUNCH_MAP(mg_restrict, int, l)
 FG_MG_LAUNCH_MAP(mg_prolong, int, l)
 FG_MG_LAUNCH_MAP(mg_post, int, l)
 FG_MG_LAUNCH_MAP(mg_rr, int, l)
 FG_MG_LAUNCH_MAP(mg_pp, int, l)
-void launch_mg_up0(dim3 g, hipStream_t st, const SceneDev* sc, const int2* map, int which, int max_j, bool ring)
-{
-    if (ring && max_j <= kUpMaxJ)
-        fg_launch_shm(k_mg_up0, g, dim3(kBlock), sizeof(float) * (2 * max_j + 2 * kUpPass), st, sc, map, which);
-    else
-        fg_launch(k_mg_up0_wide, g, dim3(kBlock), st, sc, map, which);
-}
 void launch_mg_coarse(dim3 g, hipStream_t st, const SceneDev* sc, int max_halo)
 {
     fg_launch_shm(k_mg_coarse, g, dim3(kMgCoarseThreads), 2 * sizeof(float) * max_halo, st, sc);

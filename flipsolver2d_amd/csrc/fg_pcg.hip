@@ -256,7 +256,8 @@ __global__ void __launch_bounds__(kBlock) k_pcg_a(const SceneDev* scenes, const 
         }
         if (base == ch.begin) {
             double t[2];
-            sum_partials<2>(s, kSlotCG, nb, t);   // rho = r.z, ||r||^2 of the current residual
+            // rho = r.z, ||r||^2 of the current residual
+            sum_partials<2>(s, kSlotCG, s.precond == kPrecondMG ? s.up_blocks : nb, t);
             const double rho = t[0], rr = t[1];
             const bool lead = sb.block == 0 && threadIdx.x == 0;
             const double rr0 = first ? rr : scr->rr0;
