@@ -72,7 +72,7 @@ KERNEL_BYTES = {
     "p2g": ("K_P2G", 1.0, "bytes", ["k_p2g"]),
     "particles": ("K_PARTICLES", 1.0, "bytes", ["k_advect", "k_g2p_count"]),
     "sdf": ("K_SDF", 1.0, "bytes", ["k_sdf_materials"]),
-    "pcg_a": ("K_PCG_A", 17.0, "cells", ["k_pcg_a"]),
+    "pcg_a": ("K_PCG_A", 17.0, "cells", ["k_pcg_dir", "k_pcg_a"]),
     "pcg_b": ("K_PCG_B", 32.0, "cells", ["k_pcg_b"]),
     "mg_down0": ("K_MG_DOWN0", 1.0, "bytes", ["k_mg_step0", "k_mg_down0"]),
     "mg_up0": ("K_MG_UP0", 1.0, "bytes", ["k_mg_up0"]),

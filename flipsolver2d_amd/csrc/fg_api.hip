@@ -54,7 +54,7 @@ int fail(int code, const std::string& msg)
 inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Block maps of the solve's per-iteration launches, by kind: 0 = solver
-// chunks, kUpKind = the blocks of k_mg_up0 (no scene has that many levels),
+// chunks, kUpKind = the blocks of k_mg_up0 and k_pcg_dir (no scene has that many levels),
 // 1 = level-1 tiles of kVcTile (k_mg_down0, and k_mg_pp of level 1);
 // with the fused V-cycle l = level-l tiles of kRRTile (2 <= l <= t: k_mg_rr
 // of level l-1) and kMgMaxLevels + l = level-l tiles of kVcTile (2 <= l < t:
@@ -1296,12 +1296,17 @@ void launch_vcycle(const Group& G, hipStream_t st, const SolveLaunch& S, int it)
 // kernel; the others: the V-cycle, whose first launch makes r and x).
 void launch_iteration(const Group& G, hipStream_t st, const SolveLaunch& S, int it)
 {
-    {
+    if (G.mg_levels) {
         KProf kp(G, FG_K_PCG_A, true);
-        launch_pcg_a(S.grid(0), st, S.d, S.map[0], it);
+        launch_pcg_dir(S.grid(kUpKind), st, S.d, S.map[kUpKind], it);
         kp.done(0);   // units: at the end of the solve
     }
     if (G.ipp) {
+        {
+            KProf kp(G, FG_K_PCG_A, true);
+            launch_pcg_a(S.grid(0), st, S.d, S.map[0], it);
+            kp.done(0);
+        }
         KProf kp(G, FG_K_PCG_B, true);
         launch_pcg_b(S.grid(0), st, S.d, S.map[0], it);
         kp.done(0);

@@ -138,6 +138,7 @@ FG_DECLARE_LAUNCH(nb_materials);
 // fg_pcg.hip
 FG_DECLARE_LAUNCH(refine_residual, int spec);
 FG_DECLARE_LAUNCH(cg_init, int sweep, int spec);
+FG_DECLARE_LAUNCH(pcg_dir, const int2* map, int it);
 FG_DECLARE_LAUNCH(pcg_a, const int2* map, int it);
 FG_DECLARE_LAUNCH(pcg_b, const int2* map, int it);
 FG_DECLARE_LAUNCH(solve_begin);

@@ -531,7 +531,7 @@ __device__ __forceinline__ void mg_down0_tile(const SceneDev* scenes, const int2
         float alpha = 0.f;
         if constexpr (kStep) {
             double t[1];
-            sum_partials<1>(s, kSlotPQ, s.pcg_blocks, t);
+            sum_partials<1>(s, kSlotPQ, s.up_blocks, t);   // k_pcg_dir's
             const bool lead = sb.block == 0 && threadIdx.x == 0;
             if (!(t[0] > 0.0) || !finite_d(t[0])) {   // breakdown: end this sweep (every block sees it)
                 if (lead) s.sc->inner_done = 1;
@@ -1074,7 +1074,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_post(const SceneDev* scenes, cons
 // the per-cell form by instruction issue.  The quotients by D1, an integer
 // up to 8, are a product with its reciprocal and one step with the exact
 // remainder (correctly rounded, as the division).  A tile is the fine side of
-// k_mg_step0's, in its order, so what one of them writes the
+// k_mg_step0's and k_pcg_dir's, in their order, so what one writes the
 // other reads through the same XCD's L2.  Per-cell form (each cell its
 // neighbours' z0) 8.3 us at 128^2, 10.1 us at 1024^2; an LDS window of whole
 // rows over linear chunks 97 us at 4096^2; this form 5.7, 8.2 and 39 us.

@@ -205,16 +205,142 @@ __global__ void __launch_bounds__(kBlock) k_cg_init(const SceneDev* scenes, int 
     put_partials<2>(s, kSlotCG, v, blk);
 }
 
-// KA: p = z + beta p_old; q = A' p; p.q        (z lives in cu)
+// The scalars of KA, the same in every block: rho = r.z and ||r||^2 from the
+// ncg partials of the kernel before; whether the sweep stops here; beta.
+__device__ __forceinline__ bool pcg_a_scalars(const SceneDev& s, int ncg, int it, bool lead, float& beta)
+{
+    SceneScalars* sc = s.sc;
+    cptr<SceneScalars> scr = cst(sc);
+    const bool first = it == 0;
+    double t[2];
+    sum_partials<2>(s, kSlotCG, ncg, t);
+    const double rho = t[0], rr = t[1];
+    const double rr0 = first ? rr : scr->rr0;
+    if (first && lead) sc->rr0 = rr;
+    bool stop = false;
+    if (!finite_d(rho) || !finite_d(rr)) {
+        stop = true;
+        if (lead) {
+            sc->numeric_bad = 1;
+            sc->outer_done = 1;
+        }
+    } else if (rr == 0.0 || (!first && rr <= scr->inner_eps2 * rr0) || it >= s.max_inner) {
+        stop = true;
+    }
+    if (stop) {
+        if (lead) {
+            sc->inner_done = 1;
+            sc->rr = rr;
+        }
+        return false;
+    }
+    if (lead) sc->gamma[it & 1] = rho;
+    beta = first ? 0.f : (float)(rho / scr->gamma[(it - 1) & 1]);
+    return true;
+}
+
+// q = A' p of one cell from its code and the p of it and its neighbours (up,
+// down, left, right), summed in FP64 (integer weights times FP32 values:
+// exact but for the rare exponent spread) and rounded once by the caller: for
+// a smooth p, n p_c - sum p_k cancels to far below |p|, and an FP32 sum's
+// error (about eps32 * 8 |p|) would enter the residual recurrence and
+// separate it from the true residual.
+__device__ __forceinline__ double pcg_row(uint8_t cc, const float (&P)[5])
+{
+    double qd = (double)P[0];
+    if (cc & 0x80) {
+        qd = (double)((cc >> 4) & 7) * (double)P[0];
+        if (cc & 1) qd -= (double)P[1];
+        if (cc & 2) qd -= (double)P[2];
+        if (cc & 4) qd -= (double)P[3];
+        if (cc & 8) qd -= (double)P[4];
+    }
+    return qd;
+}
+
+// KA with the V-cycle: p = z + beta p_old; q = A' p; p.q (z lives in cu),
+// over the kUpTile x kUpTile tiles of k_mg_up0, SceneDev::up_blocks blocks a
+// scene: p is formed once per cell of the tile and its one-cell halo in LDS
+// (two loads instead of ten a cell) and z is read through the L2 of the XCD
+// that wrote it.  The halo is addressed linearly, so a row's end couples to
+// the next row's first cell where the reference's matrix does.
+// Per cell over linear chunks 7.3 us at 128^2, 11.1 at 1024^2, 56 at 4096^2;
+// this form 6.7, 10.6 and 46 us.
+__global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, const int2* map, int it)
+{
+    constexpr int R = kUpTile + 2;
+    __shared__ float ps[R][R + 1];
+    const SceneBlock sb = scene_block(map, true);
+    const SceneDev& s = scenes[sb.scene];
+    cptr<SceneScalars> scr = cst(s.sc);
+    // one test after the uniform loads, so that they issue together
+    if (!s.active | (s.precond != kPrecondMG) | (scr->outer_done != 0) | (scr->inner_done != 0) | (sb.block >= s.up_blocks))
+        return;
+    const int I = s.I, J = s.J, C = I * J;
+    const bool first = it == 0;
+    gptr<const float> z = gbl<const float>(s.cu);
+    gptr<const float> pold = gbl<const float>((it & 1) ? s.cp : s.cs1);
+    gptr<float> pnew = gbl((it & 1) ? s.cs1 : s.cp);
+    gptr<float> q = gbl<float>(s.cw);
+    gptr<const uint8_t> code = gbl<const uint8_t>(s.stencil);
+    const int tilesJ = (J + kUpTile - 1) / kUpTile, tiles = ((I + kUpTile - 1) / kUpTile) * tilesJ;
+    const int per = (tiles + s.up_blocks - 1) / s.up_blocks;
+    const int t0 = sb.block * per, t1 = min(tiles, t0 + per);
+    double pq = 0.0;
+    float beta = 0.f;
+    for (int tile = t0; tile < t1; tile++) {
+        const int ti = tile / tilesJ, i0 = kUpTile * ti, j0 = kUpTile * (tile - ti * tilesJ);
+        constexpr int Q = (R * R + kBlock - 1) / kBlock, N = kUpTile * kUpTile / kBlock;
+        const int b = (int)threadIdx.x % kUpTile, a0 = (int)threadIdx.x / kUpTile;   // own cells (a0 + u kBlock / kUpTile, b)
+        float zq[Q], oq[Q];
+        uint8_t cc[N];
+#pragma unroll
+        for (int u = 0; u < Q; u++) {
+            const int k = min((int)threadIdx.x + u * kBlock, R * R - 1);
+            const int f = min(max((i0 - 1 + k / R) * J + (j0 - 1 + k % R), 0), C - 1);
+            zq[u] = z[f];
+            oq[u] = first ? 0.f : pold[f];
+        }
+#pragma unroll
+        for (int u = 0; u < N; u++)
+            cc[u] = code[min((i0 + a0 + u * (kBlock / kUpTile)) * J + min(j0 + b, J - 1), C - 1)];
+        if (tile == t0) {
+            if (!pcg_a_scalars(s, s.up_blocks, it, sb.block == 0 && threadIdx.x == 0, beta)) return;
+        } else {
+            __syncthreads();   // the tile before is done with the LDS
+        }
+#pragma unroll
+        for (int u = 0; u < Q; u++) {
+            const int k = threadIdx.x + u * kBlock;
+            if (k < R * R) ps[k / R][k % R] = first ? zq[u] : zq[u] + beta * oq[u];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < N; u++) {
+            const int a = a0 + u * (kBlock / kUpTile), i = i0 + a, j = j0 + b;
+            if (i >= I || j >= J) continue;
+            const float P[5] = {ps[a + 1][b + 1], ps[a][b + 1], ps[a + 2][b + 1], ps[a + 1][b], ps[a + 1][b + 2]};
+            const double qd = pcg_row(cc[u], P);
+            pnew[i * J + j] = P[0];
+            q[i * J + j] = (float)qd;
+            pq += (double)P[0] * qd;
+        }
+    }
+    double v[1] = {pq};
+    put_partials<1>(s, kSlotPQ, v, sb.block);
+}
+
+// KA with the IPP: p = z + beta p_old; q = A' p; p.q (z lives in cu), over
+// the solver's chunks
 __global__ void __launch_bounds__(kBlock) k_pcg_a(const SceneDev* scenes, const int2* map, int it)
 {
     const SceneBlock sb = scene_block(map, true);
     const SceneDev& s = scenes[sb.scene];
-    SceneScalars* sc = s.sc;
-    cptr<SceneScalars> scr = cst(sc);   // values earlier kernels wrote: scalar loads
+    cptr<SceneScalars> scr = cst(s.sc);   // values earlier kernels wrote: scalar loads
     const int nb = s.pcg_blocks;
     // one test after the uniform loads, so that they issue together
-    if (!s.active | (scr->outer_done != 0) | (scr->inner_done != 0) | (sb.block >= nb)) return;
+    if (!s.active | (s.precond == kPrecondMG) | (scr->outer_done != 0) | (scr->inner_done != 0) | (sb.block >= nb))
+        return;
     const int J = s.J, C = s.I * s.J;
     const bool first = it == 0;
     gptr<const float> z = gbl<const float>(s.cu);
@@ -254,34 +380,7 @@ __global__ void __launch_bounds__(kBlock) k_pcg_a(const SceneDev* scenes, const 
                 pc[k][e] = pl[e] * m;
             }
         }
-        if (base == ch.begin) {
-            double t[2];
-            // rho = r.z, ||r||^2 of the current residual
-            sum_partials<2>(s, kSlotCG, s.precond == kPrecondMG ? s.up_blocks : nb, t);
-            const double rho = t[0], rr = t[1];
-            const bool lead = sb.block == 0 && threadIdx.x == 0;
-            const double rr0 = first ? rr : scr->rr0;
-            if (first && lead) sc->rr0 = rr;
-            bool stop = false;
-            if (!finite_d(rho) || !finite_d(rr)) {
-                stop = true;
-                if (lead) {
-                    sc->numeric_bad = 1;
-                    sc->outer_done = 1;
-                }
-            } else if (rr == 0.0 || (!first && rr <= scr->inner_eps2 * rr0) || it >= s.max_inner) {
-                stop = true;
-            }
-            if (stop) {
-                if (lead) {
-                    sc->inner_done = 1;
-                    sc->rr = rr;
-                }
-                return;
-            }
-            if (lead) sc->gamma[it & 1] = rho;
-            beta = first ? 0.f : (float)(rho / scr->gamma[(it - 1) & 1]);
-        }
+        if (base == ch.begin && !pcg_a_scalars(s, nb, it, sb.block == 0 && threadIdx.x == 0, beta)) return;
 #pragma unroll
         for (int k = 0; k < kItems; k++) {
             const int c = base + threadIdx.x + k * kBlock;
@@ -289,19 +388,7 @@ __global__ void __launch_bounds__(kBlock) k_pcg_a(const SceneDev* scenes, const 
             float P[5];
 #pragma unroll
             for (int e = 0; e < 5; e++) P[e] = first ? zc[k][e] : zc[k][e] + beta * pc[k][e];
-            // q = A' p summed in FP64 (integer weights times FP32 values:
-            // exact but for the rare exponent spread), rounded once: for a
-            // smooth p, n p_c - sum p_k cancels to far below |p|, and an
-            // FP32 sum's error (about eps32 * 8 |p|) would enter the
-            // residual recurrence and separate it from the true residual
-            double qd = (double)P[0];
-            if (cc[k] & 0x80) {
-                qd = (double)((cc[k] >> 4) & 7) * (double)P[0];
-                if (cc[k] & 1) qd -= (double)P[1];
-                if (cc[k] & 2) qd -= (double)P[2];
-                if (cc[k] & 4) qd -= (double)P[3];
-                if (cc[k] & 8) qd -= (double)P[4];
-            }
+            const double qd = pcg_row(cc[k], P);
             pnew[c] = P[0];
             q[c] = (float)qd;
             pq += (double)P[0] * qd;
@@ -467,6 +554,10 @@ void launch_cg_init(dim3 g, hipStream_t st, const SceneDev* sc, int sweep, int s
 void launch_pcg_a(dim3 g, hipStream_t st, const SceneDev* sc, const int2* map, int it)
 {
     fg_launch(k_pcg_a, g, dim3(kBlock), st, sc, map, it);
+}
+void launch_pcg_dir(dim3 g, hipStream_t st, const SceneDev* sc, const int2* map, int it)
+{
+    fg_launch(k_pcg_dir, g, dim3(kBlock), st, sc, map, it);
 }
 void launch_pcg_b(dim3 g, hipStream_t st, const SceneDev* sc, const int2* map, int it)
 {
