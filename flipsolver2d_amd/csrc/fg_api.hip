@@ -97,6 +97,23 @@ struct Lane {
     int64_t work[FG_K_NUM] = {};
 };
 
+// The memory of one scene: its arena, descriptor and pinned staging.  A
+// destroyed scene's goes to its context's pool and serves the next one that
+// fits, since allocating and freeing it costs 0.3 + 0.5 ms (and a device
+// synchronisation) whatever its size -- ten times a 64^2 substep.  The pool
+// holds at most kPoolBytes and kPoolBlocks, leaves room for live scenes under
+// the context's budget, gives everything back when an allocation fails and
+// when the context goes, and is the context's alone (one host thread).
+struct SceneMem {
+    void* arena = nullptr;
+    uint64_t bytes = 0;
+    SceneDev* d = nullptr;
+    SceneDev* hpin = nullptr;
+    SceneScalars* hsc = nullptr;
+};
+constexpr uint64_t kPoolBytes = 4ull << 30;
+constexpr size_t kPoolBlocks = 64;
+
 struct fg_ctx {
     int device = 0;
     uint64_t budget = 0;
@@ -111,6 +128,16 @@ struct fg_ctx {
     int precond = kPrecondMG;                // pressure PCG preconditioner
     bool vcycle_fused = true;                // V-cycle levels as k_mg_rr / k_mg_pp (else per-level kernels)
     std::vector<Lane*> lanes;
+    // pinned host memory that states are packed into (two windows) and
+    // set-ups uploaded from, grown as needed
+    char* io[2] = {nullptr, nullptr};
+    uint64_t io_cap[2] = {0, 0};
+    hipEvent_t io_ev[2] = {nullptr, nullptr};
+    char* up = nullptr;
+    uint64_t up_cap = 0;
+    int64_t* totals = nullptr;      // pinned: counts the device reports
+    std::vector<SceneMem> pool;   // memory of destroyed scenes, oldest first
+    uint64_t pooled = 0;
 };
 
 struct fg_scene {
@@ -125,6 +152,7 @@ struct fg_scene {
     int max_pblocks = 0;    // particle blocks at capacity
     void* arena = nullptr;
     uint64_t bytes = 0;
+    uint64_t block_bytes = 0;     // of the arena's allocation (a pooled one may be larger)
     SceneDev h{};                 // host copy of the descriptor
     MgLevels mgh{};               // host copy of the multigrid hierarchy (device pointers)
     bool mg_ok = false;           // the hierarchy fits kMgMaxLevels
@@ -506,6 +534,75 @@ int setup_scene_memory(fg_scene* s)
     return FG_OK;
 }
 
+void free_block(const SceneMem& m)
+{
+    if (m.arena) hipFree(m.arena);
+    if (m.d) hipFree(m.d);
+    if (m.hpin) hipHostFree(m.hpin);
+    if (m.hsc) hipHostFree(m.hsc);
+}
+
+// Give back pooled memory, oldest first, until at most `bytes` are pooled.
+void trim_pool(fg_ctx* ctx, uint64_t bytes, size_t blocks = kPoolBlocks)
+{
+    size_t k = 0;
+    while (k < ctx->pool.size() && (ctx->pooled > bytes || ctx->pool.size() - k > blocks)) {
+        ctx->pooled -= ctx->pool[k].bytes;
+        free_block(ctx->pool[k++]);
+    }
+    ctx->pool.erase(ctx->pool.begin(), ctx->pool.begin() + (ptrdiff_t)k);
+}
+
+// Memory for a scene of `need` bytes: the pooled block that fits best, if it
+// is at most a quarter (or 16 MiB) too large, else a new one.
+hipError_t take_block(fg_ctx* ctx, uint64_t need, SceneMem* out)
+{
+    size_t best = ctx->pool.size();
+    for (size_t k = 0; k < ctx->pool.size(); k++) {
+        const uint64_t b = ctx->pool[k].bytes;
+        if (b >= need && b <= need + std::max<uint64_t>(need / 4, 16ull << 20) &&
+            (best == ctx->pool.size() || b < ctx->pool[best].bytes))
+            best = k;
+    }
+    if (best < ctx->pool.size()) {
+        *out = ctx->pool[best];
+        ctx->pooled -= out->bytes;
+        ctx->pool.erase(ctx->pool.begin() + (ptrdiff_t)best);
+        return hipSuccess;
+    }
+    // under a budget the pool takes only what live scenes leave
+    if (ctx->budget) trim_pool(ctx, ctx->budget - std::min(ctx->budget, ctx->used + need));
+    for (int attempt = 0;; attempt++) {
+        SceneMem m;
+        m.bytes = need;
+        hipError_t e = hipMalloc(&m.arena, need);
+        if (e == hipSuccess) e = hipMalloc(&m.d, sizeof(SceneDev));
+        if (e == hipSuccess) e = hipHostMalloc((void**)&m.hpin, sizeof(SceneDev), hipHostMallocDefault);
+        if (e == hipSuccess) e = hipHostMalloc((void**)&m.hsc, sizeof(SceneScalars), hipHostMallocDefault);
+        if (e == hipSuccess) {
+            *out = m;
+            return e;
+        }
+        free_block(m);
+        if (attempt || ctx->pool.empty()) return e;
+        (void)hipGetLastError();   // the failed allocation's, answered here
+        trim_pool(ctx, 0, 0);
+    }
+}
+
+void give_block(fg_ctx* ctx, const SceneMem& m)
+{
+    if (m.bytes > kPoolBytes) {
+        free_block(m);
+        return;
+    }
+    ctx->pool.push_back(m);
+    ctx->pooled += m.bytes;
+    uint64_t limit = kPoolBytes;
+    if (ctx->budget) limit = std::min(limit, ctx->budget - std::min(ctx->budget, ctx->used));
+    trim_pool(ctx, limit);
+}
+
 int create_scene(fg_ctx* ctx, const fg_scene_params* p, bool solver_only, fg_scene** out)
 {
     FGCHK(validate_params(p));
@@ -520,21 +617,17 @@ int create_scene(fg_ctx* ctx, const fg_scene_params* p, bool solver_only, fg_sce
         delete s;
         return fail(FG_E_BUDGET, "scene needs " + std::to_string(need) + " bytes beyond the HBM budget");
     }
-    hipError_t e = hipMalloc(&s->arena, s->bytes);
+    SceneMem m;
+    const hipError_t e = take_block(ctx, s->bytes, &m);
     if (e != hipSuccess) {
         delete s;
         return fail(FG_E_DEVICE, std::string("hipMalloc arena: ") + hipGetErrorString(e));
     }
-    e = hipMalloc(&s->d, sizeof(SceneDev));
-    if (e == hipSuccess) e = hipHostMalloc((void**)&s->hpin, sizeof(SceneDev), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&s->hsc, sizeof(SceneScalars), hipHostMallocDefault);
-    if (e != hipSuccess) {
-        hipFree(s->arena);
-        if (s->d) hipFree(s->d);
-        if (s->hpin) hipHostFree(s->hpin);
-        delete s;
-        return fail(FG_E_DEVICE, std::string("descriptor alloc: ") + hipGetErrorString(e));
-    }
+    s->arena = m.arena;
+    s->block_bytes = m.bytes;
+    s->d = m.d;
+    s->hpin = m.hpin;
+    s->hsc = m.hsc;
     ctx->used += s->bytes;
     const int rc = setup_scene_memory(s);
     if (rc != FG_OK) {
@@ -2086,6 +2179,113 @@ int step_frames_split(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const s
 }
 
 
+// Split `bytes` of copying over a few host threads (a fresh 134 MB result
+// takes 10 ms to fault in and fill on one, 3 on eight); where no thread can
+// be had, this one does their part.
+template <typename F>
+void copy_parallel(int64_t lo, int64_t hi, F copy)
+{
+    constexpr int64_t kLeast = 1 << 20;
+    const int64_t n = std::min<int64_t>({8, (int64_t)std::max(1u, std::thread::hardware_concurrency()), (hi - lo) / kLeast});
+    if (n <= 1) {
+        copy(lo, hi);
+        return;
+    }
+    const int64_t step = ((hi - lo + n - 1) / n + 4095) & ~int64_t(4095);
+    std::thread crew[8];
+    for (int64_t k = 1; k < n; k++) {
+        const int64_t a = std::min(hi, lo + k * step), b = std::min(hi, a + step);
+        try {
+            crew[k] = std::thread(copy, a, b);
+        } catch (...) {
+            copy(a, b);
+        }
+    }
+    copy(lo, std::min(hi, lo + step));
+    for (std::thread& t : crew)
+        if (t.joinable()) t.join();
+}
+
+// Read device arrays back: packed into pinned windows by k_pack, the next
+// window on its way while the host copies this one out.
+constexpr int64_t kIoWindow = 16 << 20;
+struct ReadBack {
+    PackArgs a{};
+    struct Out {
+        char* dst;
+        int64_t off, bytes;   // bytes < 0: as many particles as live, 4 bytes each
+    };
+    std::vector<Out> outs;
+    int64_t end = 0;
+    ReadBack()
+    {
+        for (int64_t& p : a.part) p = -1;
+    }
+    void particles(int what, void* dst, int64_t bound)
+    {
+        if (!dst) return;
+        a.part[what] = end;
+        outs.push_back(Out{static_cast<char*>(dst), end, -1});
+        end = (end + 4 * bound + 255) & ~int64_t(255);
+    }
+    void array(void* dst, const void* src, int64_t bytes)
+    {
+        if (!dst || bytes <= 0) return;
+        a.seg[a.nseg++] = PackSeg{src, end, bytes};
+        outs.push_back(Out{static_cast<char*>(dst), end, bytes});
+        end = (end + bytes + 255) & ~int64_t(255);
+    }
+    int run(fg_ctx* ctx, const SceneDev* d, int64_t* live)
+    {
+        hipStream_t q = ctx->stream;
+        const int64_t windows = std::max<int64_t>(1, cdiv(end, kIoWindow));
+        for (int k = 0; k < (windows > 1 ? 2 : 1); k++) {
+            uint64_t need = 64 << 10;
+            while ((int64_t)need < std::min(end, kIoWindow)) need *= 2;
+            if (!ctx->io_ev[k]) HIPCHK(hipEventCreateWithFlags(&ctx->io_ev[k], hipEventDisableTiming));
+            if (need <= ctx->io_cap[k]) continue;
+            if (ctx->io[k]) hipHostFree(ctx->io[k]);   // idle: every read-back waits for its windows
+            ctx->io[k] = nullptr;
+            ctx->io_cap[k] = 0;
+            HIPCHK(hipHostMalloc((void**)&ctx->io[k], need, hipHostMallocDefault));
+            ctx->io_cap[k] = need;
+        }
+        const int64_t arrays = a.nseg ? a.seg[0].off : end;
+        const int pblocks = a.pblocks;
+        auto launch = [&](int64_t w) -> int {
+            a.lo = w * kIoWindow;
+            a.hi = std::min(end, a.lo + kIoWindow);
+            a.first = std::max(a.lo, arrays);
+            a.pblocks = a.lo < arrays ? pblocks : 0;
+            a.out = ctx->io[w & 1];
+            launch_pack(q, d, a);
+            HIPCHK(hipGetLastError());
+            HIPCHK(hipEventRecord(ctx->io_ev[w & 1], q));
+            return FG_OK;
+        };
+        FGCHK(launch(0));
+        for (int64_t w = 0; w < windows; w++) {
+            if (w + 1 < windows) {
+                const int rc = launch(w + 1);
+                if (rc != FG_OK) {
+                    hipStreamSynchronize(q);
+                    return rc;
+                }
+            }
+            HIPCHK(hipEventSynchronize(ctx->io_ev[w & 1]));
+            const int64_t n = live ? *live : 0, lo = w * kIoWindow, hi = std::min(end, lo + kIoWindow);
+            const char* const from = ctx->io[w & 1];
+            copy_parallel(lo, hi, [&](int64_t b0, int64_t b1) {
+                for (const Out& o : outs) {
+                    const int64_t x0 = std::max(b0, o.off), x1 = std::min(b1, o.off + (o.bytes < 0 ? 4 * n : o.bytes));
+                    if (x0 < x1) std::memcpy(o.dst + (x0 - o.off), from + (x0 - lo), (size_t)(x1 - x0));
+                }
+            });
+        }
+        return FG_OK;
+    }
+};
+
 // The solver-only scene of an isolated solve (LinearSolver::solve replacement).
 fg_scene_params solve_params(int32_t size_i, int32_t size_j, double rel_tol, int32_t max_iters)
 {
@@ -2102,9 +2302,12 @@ fg_scene_params solve_params(int32_t size_i, int32_t size_j, double rel_tol, int
 
 // Upload the system into a solver-only scene, solve, download x.  The
 // matrix comes as materials (assembled on the device, k_stencil) or as its
-// bytes (one per cell, the stencil format of fg_scene_state).
+// bytes (one per cell, the stencil format of fg_scene_state).  staged: a
+// result of kStagedLeast or more comes back through the context's pinned
+// windows, which a caller that may not allocate does without.
+constexpr int64_t kStagedLeast = 4 << 20;
 int solve_on_scene(fg_scene* s, const int8_t* material, const uint8_t* stencil, double scale, const double* b,
-                   double* x, fg_solve_stats* stats)
+                   double* x, fg_solve_stats* stats, bool staged)
 {
     fg_ctx* ctx = s->ctx;
     hipStream_t q = ctx->stream;
@@ -2131,8 +2334,14 @@ int solve_on_scene(fg_scene* s, const int8_t* material, const uint8_t* stencil, 
         }
     }
     const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    if (rc == FG_OK || rc == FG_E_NUMERIC) {
-        hipError_t e = hipMemcpyAsync(x, s->h.x64, sizeof(double) * C, hipMemcpyDeviceToHost, q);
+    const int64_t x_bytes = (int64_t)sizeof(double) * C;
+    if ((rc == FG_OK || rc == FG_E_NUMERIC) && staged && x_bytes >= kStagedLeast) {
+        ReadBack rb;
+        rb.array(x, s->h.x64, x_bytes);
+        const int r = rb.run(ctx, s->d, nullptr);
+        if (rc == FG_OK) rc = r;
+    } else if (rc == FG_OK || rc == FG_E_NUMERIC) {
+        hipError_t e = hipMemcpyAsync(x, s->h.x64, x_bytes, hipMemcpyDeviceToHost, q);
         if (e == hipSuccess) e = hipStreamSynchronize(q);
         if (e != hipSuccess && rc == FG_OK) rc = fail(FG_E_DEVICE, hipGetErrorString(e));
     }
@@ -2166,9 +2375,26 @@ int batch_args(fg_ctx* ctx, fg_scene* const* scenes, int32_t n, fg_stats* stats,
     return FG_OK;
 }
 
-// Polygons of a set-up packed for k_init_cells: vertex offsets, then the
-// vertices as float2, in the set order sinks, sources, solids, fluids.
-int upload_geometry(fg_scene* s, const fg_polygons* sets[4], const float* const visc[4], InitGeo* geo)
+// Pinned host memory of at least `bytes` for an upload on lane 0's stream.
+// Its last upload has ended: every call that makes one synchronises.
+int upload_buffer(fg_ctx* ctx, uint64_t bytes)
+{
+    if (bytes <= ctx->up_cap) return FG_OK;
+    if (ctx->up) hipHostFree(ctx->up);
+    ctx->up = nullptr;
+    ctx->up_cap = 0;
+    const uint64_t cap = std::max<uint64_t>(bytes, 64 << 10);
+    HIPCHK(hipHostMalloc((void**)&ctx->up, cap, hipHostMallocDefault));
+    ctx->up_cap = cap;
+    return FG_OK;
+}
+
+// A set-up's tables on their way to the device, one copy: the friction table
+// (256 floats) and the emitter table (kMaxEmitters float4), for
+// k_init_commit; polygons for k_init_cells: vertex offsets, viscosities, then
+// the vertices as float2, in the set order sinks, sources, solids, fluids.
+int upload_geometry(fg_scene* s, const fg_polygons* sets[4], const float* const visc[4], const std::vector<float>& friction,
+                    const std::vector<float4>& emitters, InitGeo* geo, const float** tables)
 {
     std::vector<int32_t> voff(1, 0);
     std::vector<float2> verts;
@@ -2188,49 +2414,57 @@ int upload_geometry(fg_scene* s, const fg_polygons* sets[4], const float* const 
         }
         first += P.n;
     }
-    const size_t off_bytes = (sizeof(int32_t) * voff.size() + 255) & ~size_t(255);
-    const size_t visc_bytes = (sizeof(float) * std::max<size_t>(pvisc.size(), 1) + 255) & ~size_t(255);
-    const size_t bytes = off_bytes + visc_bytes + sizeof(float2) * std::max<size_t>(verts.size(), 1);
+    auto pad = [](size_t b) { return (b + 255) & ~size_t(255); };
+    const size_t tab_bytes = pad(sizeof(float) * 256 + sizeof(float4) * kMaxEmitters);
+    const size_t off_bytes = pad(sizeof(int32_t) * voff.size());
+    const size_t visc_bytes = pad(sizeof(float) * std::max<size_t>(pvisc.size(), 1));
+    const size_t bytes = tab_bytes + off_bytes + visc_bytes + sizeof(float2) * std::max<size_t>(verts.size(), 1);
     Lane* L = s->ctx->lanes[0];
+    FGCHK(upload_buffer(s->ctx, bytes));
     if (bytes > L->bgeo_cap) {
         HIPCHK(hipStreamSynchronize(L->stream));
         if (L->bgeo) hipFree(L->bgeo);
         L->bgeo = nullptr;
         L->bgeo_cap = 0;
-        HIPCHK(hipMalloc(&L->bgeo, bytes));
-        L->bgeo_cap = bytes;
+        HIPCHK(hipMalloc(&L->bgeo, std::max<size_t>(bytes, 64 << 10)));
+        L->bgeo_cap = std::max<size_t>(bytes, 64 << 10);
     }
-    char* base = static_cast<char*>(L->bgeo);
-    HIPCHK(hipMemcpyAsync(base, voff.data(), sizeof(int32_t) * voff.size(), hipMemcpyHostToDevice, L->stream));
-    if (!pvisc.empty())
-        HIPCHK(hipMemcpyAsync(base + off_bytes, pvisc.data(), sizeof(float) * pvisc.size(), hipMemcpyHostToDevice,
-                              L->stream));
-    if (!verts.empty())
-        HIPCHK(hipMemcpyAsync(base + off_bytes + visc_bytes, verts.data(), sizeof(float2) * verts.size(),
-                              hipMemcpyHostToDevice, L->stream));
-    geo->voff = reinterpret_cast<const int32_t*>(base);
-    geo->visc = reinterpret_cast<const float*>(base + off_bytes);
-    geo->verts = reinterpret_cast<const float2*>(base + off_bytes + visc_bytes);
+    char* const up = s->ctx->up;
+    std::memcpy(up, friction.data(), sizeof(float) * 256);
+    std::memcpy(up + sizeof(float) * 256, emitters.data(), sizeof(float4) * kMaxEmitters);
+    std::memcpy(up + tab_bytes, voff.data(), sizeof(int32_t) * voff.size());
+    std::memcpy(up + tab_bytes + off_bytes, pvisc.data(), sizeof(float) * pvisc.size());
+    std::memcpy(up + tab_bytes + off_bytes + visc_bytes, verts.data(), sizeof(float2) * verts.size());
+    char* const base = static_cast<char*>(L->bgeo);
+    HIPCHK(hipMemcpyAsync(base, up, bytes, hipMemcpyHostToDevice, L->stream));
+    *tables = reinterpret_cast<const float*>(base);
+    geo->voff = reinterpret_cast<const int32_t*>(base + tab_bytes);
+    geo->visc = reinterpret_cast<const float*>(base + tab_bytes + off_bytes);
+    geo->verts = reinterpret_cast<const float2*>(base + tab_bytes + off_bytes + visc_bytes);
     geo->dx = (float)s->p.dx;
-    // the host vectors are read by the copies above: wait for them
-    HIPCHK(hipStreamSynchronize(L->stream));
     return FG_OK;
 }
 
-// The emitter table (fg_scene_set_emitters; with the sources' viscosity
-// from fg_scene_init_objects).
-int set_emitters(fg_scene* s, int32_t n, const float* velocity, const uint8_t* transfer, const float* viscosity,
-                 uint32_t seed)
+// per emitter the face values afterTransfer writes: velocity / dx in double,
+// rounded to float (flipsolver2d.cpp:402-403)
+std::vector<float4> emitter_table(const fg_scene* s, int32_t n, const float* velocity, const uint8_t* transfer,
+                                  const float* viscosity)
+{
+    std::vector<float4> tab(kMaxEmitters, make_float4(0.f, 0.f, 0.f, 0.f));
+    for (int32_t k = 0; k < n; k++)
+        tab[k] = make_float4(velocity ? (float)((double)velocity[2 * k] / s->p.dx) : 0.f,
+                             velocity ? (float)((double)velocity[2 * k + 1] / s->p.dx) : 0.f,
+                             transfer && transfer[k] ? 1.f : 0.f, viscosity ? viscosity[k] : 0.f);
+    return tab;
+}
+
+// The emitter table (fg_scene_set_emitters).
+int set_emitters(fg_scene* s, int32_t n, const float* velocity, const uint8_t* transfer, uint32_t seed)
 {
     if (!s || (n > 0 && !velocity)) return fail(FG_E_INVALID, "NULL argument");
     if (n < 0 || n > kMaxEmitters) return fail(FG_E_INVALID, "at most 256 emitters");
     if (s->solver_only) return fail(FG_E_STATE, "solver-only scene");
-    // per emitter the face values afterTransfer writes: velocity / dx in
-    // double, rounded to float (flipsolver2d.cpp:402-403)
-    std::vector<float4> tab(kMaxEmitters, make_float4(0.f, 0.f, 0.f, 0.f));
-    for (int32_t k = 0; k < n; k++)
-        tab[k] = make_float4((float)((double)velocity[2 * k] / s->p.dx), (float)((double)velocity[2 * k + 1] / s->p.dx),
-                             transfer && transfer[k] ? 1.f : 0.f, viscosity ? viscosity[k] : 0.f);
+    const std::vector<float4> tab = emitter_table(s, n, velocity, transfer, nullptr);
     HIPCHK(hipMemcpyAsync(s->h.emitters, tab.data(), sizeof(float4) * kMaxEmitters, hipMemcpyHostToDevice,
                           s->ctx->stream));
     s->h.n_emitters = n;
@@ -2272,6 +2506,11 @@ int fg_ctx_create(int32_t device, uint64_t hbm_budget_bytes, fg_ctx** out)
     }
     c->lanes.push_back(L);
     c->stream = L->stream;
+    const hipError_t e = hipHostMalloc((void**)&c->totals, 2 * sizeof(int64_t), hipHostMallocDefault);
+    if (e != hipSuccess) {
+        fg_ctx_destroy(c);
+        return fail(FG_E_DEVICE, std::string("hipHostMalloc: ") + hipGetErrorString(e));
+    }
     *out = c;
     return FG_OK;
 }
@@ -2280,6 +2519,13 @@ int fg_ctx_destroy(fg_ctx* ctx)
 {
     if (!ctx) return FG_OK;
     for (Lane* L : ctx->lanes) lane_destroy(L);
+    trim_pool(ctx, 0, 0);
+    for (int k = 0; k < 2; k++) {
+        if (ctx->io[k]) hipHostFree(ctx->io[k]);
+        if (ctx->io_ev[k]) hipEventDestroy(ctx->io_ev[k]);
+    }
+    if (ctx->up) hipHostFree(ctx->up);
+    if (ctx->totals) hipHostFree(ctx->totals);
     if (ctx->prof_ref) hipEventDestroy(ctx->prof_ref);
     delete ctx;
     return FG_OK;
@@ -2442,12 +2688,16 @@ int fg_scene_create(fg_ctx* ctx, const fg_scene_params* p, fg_scene** out)
 int fg_scene_destroy(fg_scene* s)
 {
     if (!s) return FG_OK;
-    hipStreamSynchronize(s->ctx->stream);
-    hipFree(s->arena);
-    hipFree(s->d);
-    hipHostFree(s->hpin);
-    hipHostFree(s->hsc);
-    s->ctx->used -= s->bytes;
+    fg_ctx* ctx = s->ctx;
+    hipStreamSynchronize(ctx->stream);   // the other lanes' work ended with the calls that queued it
+    ctx->used -= s->bytes;
+    SceneMem m;
+    m.arena = s->arena;
+    m.bytes = s->block_bytes;
+    m.d = s->d;
+    m.hpin = s->hpin;
+    m.hsc = s->hsc;
+    give_block(ctx, m);
     delete s;
     return FG_OK;
 }
@@ -2548,40 +2798,34 @@ int fg_scene_get_state(fg_scene* s, fg_scene_state* st)
 {
     if (!s || !st) return fail(FG_E_INVALID, "NULL argument");
     if (s->solver_only) return fail(FG_E_STATE, "solver-only scene");
-    hipStream_t q = s->ctx->stream;
     const SceneDev& h = s->h;
-    FGCHK(read_scalars(s));
-    const int64_t n = s->hsc->n_particles;
-    std::vector<float2> pos(n), vel(n);
-    std::vector<uint32_t> pid(n), key(n);
-    std::vector<float> pv(h.visc_on ? n : 0);
-    if (n > 0) {
-        if (h.visc_on) HIPCHK(hipMemcpyAsync(pv.data(), h.pvisc, sizeof(float) * n, hipMemcpyDeviceToHost, q));
-        HIPCHK(hipMemcpyAsync(pos.data(), h.pos, sizeof(float2) * n, hipMemcpyDeviceToHost, q));
-        HIPCHK(hipMemcpyAsync(vel.data(), h.vel, sizeof(float2) * n, hipMemcpyDeviceToHost, q));
-        HIPCHK(hipMemcpyAsync(pid.data(), h.pid, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, q));
-        HIPCHK(hipMemcpyAsync(key.data(), h.key, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, q));
-    }
-    auto dl = [&](void* dst, const void* src, size_t bytes) -> int {
-        if (dst) HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, q));
-        return FG_OK;
-    };
-    FGCHK(dl(st->u, h.uf, sizeof(float) * s->FU));
-    FGCHK(dl(st->v, h.vf, sizeof(float) * s->FV));
-    FGCHK(dl(st->u_valid, h.uvalF, s->FU));
-    FGCHK(dl(st->v_valid, h.vvalF, s->FV));
-    FGCHK(dl(st->material, h.mat, s->C));
-    FGCHK(dl(st->solid_sdf, h.ssdf, sizeof(float) * s->C));
-    FGCHK(dl(st->fluid_sdf, h.fsdf, sizeof(float) * s->C));
-    FGCHK(dl(st->solid_id, h.sid, sizeof(int32_t) * s->C));
-    FGCHK(dl(st->particle_counts, h.pcount, sizeof(int32_t) * s->C));
-    FGCHK(dl(st->saved_u, h.su, sizeof(float) * s->FU));
-    FGCHK(dl(st->saved_v, h.sv, sizeof(float) * s->FV));
-    FGCHK(dl(st->pressure, h.x64, sizeof(double) * s->C));
-    FGCHK(dl(st->rhs, h.b, sizeof(double) * s->C));
-    FGCHK(dl(st->stencil, h.stencil, s->C));
-    FGCHK(dl(st->emitter_id, h.eid, sizeof(int32_t) * s->C));
-    if (h.visc_on) FGCHK(dl(st->viscosity, h.cvisc, sizeof(float) * s->C));
+    // n_bound bounds the particles (also between the stages of a substep)
+    const int64_t bound = s->n_bound;
+    ReadBack rb;
+    rb.a.pblocks = (int)cdiv(bound, kBlock);
+    rb.particles(0, st->px, bound);
+    rb.particles(1, st->py, bound);
+    rb.particles(2, st->vx, bound);
+    rb.particles(3, st->vy, bound);
+    rb.particles(4, st->pid, bound);
+    if (h.visc_on) rb.particles(5, st->particle_viscosity, bound);
+    const int64_t U4 = sizeof(float) * s->FU, V4 = sizeof(float) * s->FV, C4 = sizeof(float) * s->C;
+    rb.array(st->u, h.uf, U4);
+    rb.array(st->v, h.vf, V4);
+    rb.array(st->u_valid, h.uvalF, s->FU);
+    rb.array(st->v_valid, h.vvalF, s->FV);
+    rb.array(st->material, h.mat, s->C);
+    rb.array(st->solid_sdf, h.ssdf, C4);
+    rb.array(st->fluid_sdf, h.fsdf, C4);
+    rb.array(st->solid_id, h.sid, C4);
+    rb.array(st->particle_counts, h.pcount, C4);
+    rb.array(st->saved_u, h.su, U4);
+    rb.array(st->saved_v, h.sv, V4);
+    rb.array(st->pressure, h.x64, 2 * C4);
+    rb.array(st->rhs, h.b, 2 * C4);
+    rb.array(st->stencil, h.stencil, s->C);
+    rb.array(st->emitter_id, h.eid, C4);
+    if (h.visc_on) rb.array(st->viscosity, h.cvisc, C4);
     else if (st->viscosity) std::fill(st->viscosity, st->viscosity + s->C, 0.f);
     {   // the grid fluidVelocityGrid holds after the last stage hook
         const float *wu = h.u, *wv = h.v;   // P2G .. SDF, FORCES, PROJECT (+ SOLIDS)
@@ -2592,23 +2836,17 @@ int fg_scene_get_state(fg_scene* s, fg_scene_state* st)
             wu = h.uf;
             wv = h.vf;
         }
-        FGCHK(dl(st->work_u, wu, sizeof(float) * s->FU));
-        FGCHK(dl(st->work_v, wv, sizeof(float) * s->FV));
+        rb.array(st->work_u, wu, U4);
+        rb.array(st->work_v, wv, V4);
     }
     st->rng_epoch = s->epoch;
     st->next_pid = s->next_pid;
-    HIPCHK(hipStreamSynchronize(q));
-    int64_t w = 0;
-    for (int64_t k = 0; k < n; k++) {
-        if (key[k] == kDead) continue;
-        if (st->px) st->px[w] = pos[k].x;
-        if (st->py) st->py[w] = pos[k].y;
-        if (st->vx) st->vx[w] = vel[k].x;
-        if (st->vy) st->vy[w] = vel[k].y;
-        if (st->pid) st->pid[w] = pid[k];
-        if (st->particle_viscosity) st->particle_viscosity[w] = h.visc_on ? pv[k] : 0.f;
-        w++;
-    }
+    int64_t* const live = s->ctx->totals;
+    *live = 0;
+    if (rb.a.pblocks) launch_live_counts(s->ctx->stream, s->d, rb.a.pblocks, live);
+    FGCHK(rb.run(s->ctx, s->d, live));
+    const int64_t w = *live;
+    if (!h.visc_on && st->particle_viscosity) std::fill(st->particle_viscosity, st->particle_viscosity + w, 0.f);
     st->n_particles = w;
     return FG_OK;
 }
@@ -2633,7 +2871,7 @@ int fg_scene_particle_count(fg_scene* s, int64_t* out)
 
 int fg_scene_set_emitters(fg_scene* s, int32_t n, const float* velocity, const uint8_t* transfer, uint32_t seed)
 {
-    return set_emitters(s, n, velocity, transfer, nullptr, seed);
+    return set_emitters(s, n, velocity, transfer, seed);
 }
 
 int fg_scene_init_objects(fg_scene* s, const fg_scene_objects* o)
@@ -2645,30 +2883,40 @@ int fg_scene_init_objects(fg_scene* s, const fg_scene_objects* o)
     s->last_stage = -1;
     const fg_polygons* sets[4] = {&o->sinks, &o->sources, &o->solids, &o->fluids};
     const float* const visc[4] = {nullptr, o->source_viscosity, nullptr, o->fluid_viscosity};
+    // validated by upload_geometry before anything of the scene changes
+    std::vector<float> friction(256, 0.f);
+    const int32_t nf = o->friction ? std::max(o->solids.n, 0) : 0;
+    if (nf > 0) std::copy(o->friction, o->friction + nf, friction.begin());
+    const std::vector<float4> emitters =
+        emitter_table(s, std::max(o->sources.n, 0), o->source_velocity, o->source_transfer, o->source_viscosity);
     InitGeo geo{};
-    FGCHK(upload_geometry(s, sets, visc, &geo));
+    const float* tables = nullptr;
+    FGCHK(upload_geometry(s, sets, visc, friction, emitters, &geo, &tables));
     hipStream_t q = s->ctx->stream;
     SceneDev& h = s->h;
+    h.n_friction = nf;
+    h.friction_any = 0;
+    for (int k = 0; k < nf; k++)
+        if (friction[k] != 0.f) h.friction_any = 1;
+    h.n_emitters = o->sources.n;
+    h.rseed = o->seed;
+    h.has_sources = o->sources.n > 0;   // SOURCE cells can only come from sources
+    FGCHK(upload_desc(s));
     // grids of a scene at rest; the cell pass writes materials, ids, SDFs
-    HIPCHK(hipMemsetAsync(h.uf, 0, sizeof(float) * s->FU, q));
-    HIPCHK(hipMemsetAsync(h.vf, 0, sizeof(float) * s->FV, q));
-    HIPCHK(hipMemsetAsync(h.uvalF, 0, s->FU, q));
-    HIPCHK(hipMemsetAsync(h.vvalF, 0, s->FV, q));
     const dim3 cells((unsigned)cdiv(s->C, kBlock));
     const dim3 scan((unsigned)cdiv(s->C, kScanTileCells));
+    launch_init_faces(dim3((unsigned)cdiv(std::max(s->FU, s->FV), kBlock)), q, s->d);
     launch_init_cells(cells, q, s->d, geo);
     launch_scan_local(scan, q, s->d);
     launch_scan_top(dim3(1), q, s->d);
     launch_scan_add(scan, q, s->d);
-    int32_t total = 0;
-    HIPCHK(hipMemcpyAsync(&total, h.cellStart + s->C, sizeof(int32_t), hipMemcpyDeviceToHost, q));
-    HIPCHK(hipStreamSynchronize(q));
-    const bool fits = total <= s->cap;
-    if (fits) launch_seed(cells, q, s->d, o->seed);
-    else launch_clear_counts(cells, q, s->d);
-    const int32_t n = fits ? total : 0;
-    hipLaunchKernelGGL(k_set_count, dim3(1), dim3(64), 0, q, s->d, (int)n);
+    launch_seed(cells, q, s->d, o->seed);
+    launch_init_commit(q, s->d, tables, s->ctx->totals);
     HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(q));
+    const int64_t total = s->ctx->totals[0];
+    const bool fits = total <= s->cap;
+    const int64_t n = fits ? total : 0;
     s->n_bound = n;
     s->n_live = n;
     s->vmax_ready = false;
@@ -2676,12 +2924,6 @@ int fg_scene_init_objects(fg_scene* s, const fg_scene_objects* o)
     s->status = FG_OK;
     s->epoch = 0;
     s->next_pid = (uint32_t)n;
-    s->h.has_sources = o->sources.n > 0;   // SOURCE cells can only come from sources
-    if (o->friction && o->solids.n > 0) FGCHK(fg_scene_set_friction(s, o->solids.n, o->friction));
-    else FGCHK(fg_scene_set_friction(s, 0, nullptr));
-    std::vector<float> vel(2 * std::max(o->sources.n, 0), 0.f);
-    if (o->source_velocity) std::copy(o->source_velocity, o->source_velocity + vel.size(), vel.begin());
-    FGCHK(set_emitters(s, o->sources.n, vel.data(), o->source_transfer, o->source_viscosity, o->seed));
     if (!fits) return fail(FG_E_CAPACITY, "seeded particles exceed max_particles");
     return FG_OK;
 }
@@ -2932,7 +3174,7 @@ int fg_poisson_solve(fg_ctx* ctx, int32_t size_i, int32_t size_j, const int8_t* 
     const fg_scene_params p = solve_params(size_i, size_j, rel_tol, max_iters);
     fg_scene* s = nullptr;
     FGCHK(create_scene(ctx, &p, true, &s));
-    const int rc = solve_on_scene(s, material, nullptr, scale, b, x, stats);
+    const int rc = solve_on_scene(s, material, nullptr, scale, b, x, stats, true);
     fg_scene_destroy(s);
     return rc;
 }
@@ -2945,7 +3187,7 @@ int fg_poisson_solve_matrix(fg_ctx* ctx, int32_t size_i, int32_t size_j, const u
     const fg_scene_params p = solve_params(size_i, size_j, rel_tol, max_iters);
     fg_scene* s = nullptr;
     FGCHK(create_scene(ctx, &p, true, &s));
-    const int rc = solve_on_scene(s, nullptr, matrix, scale, b, x, stats);
+    const int rc = solve_on_scene(s, nullptr, matrix, scale, b, x, stats, true);
     fg_scene_destroy(s);
     return rc;
 }
@@ -2979,7 +3221,7 @@ int fg_poisson_solve_noalloc(fg_ctx* ctx, int32_t size_i, int32_t size_j, const 
     sc.hpin = &slot.desc_stage;
     sc.hsc = &slot.scalars;
     FGCHK(setup_scene_memory(&sc));
-    return solve_on_scene(&sc, material, nullptr, scale, b, x, stats);
+    return solve_on_scene(&sc, material, nullptr, scale, b, x, stats, false);
 }
 
 }  // extern "C"

@@ -159,11 +159,11 @@ __global__ void __launch_bounds__(kBlock) k_seed(const SceneDev* scenes, uint32_
     const int cnt = s.cellCount[c];
     if (cnt == 0) return;
     s.cellCount[c] = 0;
+    if (s.cellStart[C] > s.cap) return;   // the seeding overflows: none is done, and the host refuses it
     const int i = c / J, j = c - (c / J) * J;
     const int base = s.cellStart[c];
     for (int k = 0; k < cnt; k++) {
         const int64_t idx = (int64_t)base + k;
-        if (idx >= s.cap) return;   // the host refuses a scene whose seeding overflows
         const int q = k & 3;
         const float qi = (float)(q >> 1), qj = (float)(q & 1);
         const float x = (float)i + 0.5f * (qi + jitter(seed, (uint32_t)c, (uint32_t)k, 0));
@@ -177,13 +177,33 @@ __global__ void __launch_bounds__(kBlock) k_seed(const SceneDev* scenes, uint32_
     }
 }
 
-// Clear the cell counts of a set-up that stops after the scan (a scene
-// whose seeding would overflow its capacity).
-__global__ void __launch_bounds__(kBlock) k_clear_counts(const SceneDev* scenes)
+// The faces of a scene at rest.
+__global__ void __launch_bounds__(kBlock) k_init_faces(const SceneDev* scenes)
 {
     const SceneDev& s = scenes[blockIdx.y];
-    const int c = blockIdx.x * kBlock + threadIdx.x;
-    if (c < s.I * s.J) s.cellCount[c] = 0;
+    const int k = blockIdx.x * kBlock + threadIdx.x;
+    if (k < (s.I + 1) * s.J) {
+        s.uf[k] = 0.f;
+        s.uvalF[k] = 0;
+    }
+    if (k < s.I * (s.J + 1)) {
+        s.vf[k] = 0.f;
+        s.vvalF[k] = 0;
+    }
+}
+
+__global__ void __launch_bounds__(kBlock) k_init_commit(const SceneDev* scenes, const float* tables, int64_t* total)
+{
+    static_assert(kBlock == 256 && kMaxEmitters == 256, "a table entry a thread");
+    const SceneDev& s = scenes[0];
+    const int t = threadIdx.x;
+    s.friction[t] = tables[t];
+    s.emitters[t] = reinterpret_cast<const float4*>(tables + 256)[t];
+    if (t == 0) {
+        const int64_t n = s.cellStart[s.I * s.J];
+        s.sc->n_particles = n <= s.cap ? (int32_t)n : 0;
+        *total = n;
+    }
 }
 
 // FlipSolver::afterTransfer, flipsolver2d.cpp:390-410: the working grid's
@@ -321,9 +341,13 @@ void launch_seed(dim3 g, hipStream_t st, const SceneDev* sc, uint32_t seed)
 {
     hipLaunchKernelGGL(k_seed, g, dim3(kBlock), 0, st, sc, seed);
 }
-void launch_clear_counts(dim3 g, hipStream_t st, const SceneDev* sc)
+void launch_init_faces(dim3 g, hipStream_t st, const SceneDev* sc)
 {
-    hipLaunchKernelGGL(k_clear_counts, g, dim3(kBlock), 0, st, sc);
+    hipLaunchKernelGGL(k_init_faces, g, dim3(kBlock), 0, st, sc);
+}
+void launch_init_commit(hipStream_t st, const SceneDev* sc, const float* tables, int64_t* total)
+{
+    hipLaunchKernelGGL(k_init_commit, dim3(1), dim3(kBlock), 0, st, sc, tables, total);
 }
 void launch_after_transfer(dim3 g, hipStream_t st, const SceneDev* sc)
 {

@@ -110,9 +110,29 @@ struct InitGeo {
     const float* visc;      // per polygon: Emitter::viscosity of sources and fluids (0 otherwise)
     float dx;
 };
+// fg_io.hip: a state packed into one stream of 256-byte aligned sections --
+// the particles' components (part: px, py, vx, vy, pid, viscosity; -1: not
+// wanted), then plain arrays (seg) -- of which a launch writes [lo, hi) to out
+constexpr int kPackSegs = 24, kPackBytes = 16 * kBlock * 4;
+struct PackSeg {
+    const void* src;
+    int64_t off, bytes;
+};
+struct PackArgs {
+    PackSeg seg[kPackSegs];
+    int64_t part[6];
+    int64_t lo, hi, first;   // first: where the plain arrays' blocks begin in this launch
+    char* out;
+    int32_t nseg, pblocks;
+};
+void launch_live_counts(hipStream_t st, const SceneDev* scene, int blocks, int64_t* total);
+void launch_pack(hipStream_t st, const SceneDev* scene, const PackArgs& a);
+
 void launch_init_cells(dim3 grid, hipStream_t st, const SceneDev* scenes, const InitGeo& geo);
 void launch_seed(dim3 grid, hipStream_t st, const SceneDev* scenes, uint32_t seed);
-FG_DECLARE_LAUNCH(clear_counts);
+FG_DECLARE_LAUNCH(init_faces);
+// commits the seeded count and fills the friction and emitter tables from `tables` (256 floats, then kMaxEmitters float4)
+void launch_init_commit(hipStream_t st, const SceneDev* scene, const float* tables, int64_t* total);
 FG_DECLARE_LAUNCH(after_transfer);
 FG_DECLARE_LAUNCH(reseed_count);
 FG_DECLARE_LAUNCH(reseed_write);
