@@ -34,7 +34,7 @@ __host__ __device__ inline int mg_d0_tiles(int I1, int J1)
 }
 constexpr int kUpTile = 32;              // k_mg_up0: cells a tile, per side
 constexpr int kVcTile = 16;              // k_mg_pp: level-l cells a block, per side
-constexpr int kRRTile = 8;               // k_mg_rr: level-(l+1) cells a block, per side
+constexpr int kRRTile = 7;               // k_mg_rr: level-(l+1) cells a block, per side
 // blocks of a fused V-cycle launch over a level of I x J cells in tiles of t x t
 __host__ __device__ inline int mg_tiles(int I, int J, int t = kVcTile)
 {
