@@ -427,13 +427,42 @@ __device__ __forceinline__ SceneBlock scene_block(const int2* map, bool tiled)
     return SceneBlock{(int)blockIdx.y, tiled ? xcd_tile(blockIdx.x, gridDim.x) : (int)blockIdx.x};
 }
 
+// Sum of v over the wave in lane 0: lanes i and i + 32, then 16, 8, 4, 2, 1
+// apart.  The last four stay inside a row of 16 lanes, where a DPP move brings
+// the partner in a few cycles; a lane permute through LDS takes over 100.
+template <int CTRL>
+__device__ __forceinline__ double row_shl(double v)
+{
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+template <int NV>
+__device__ __forceinline__ void wave_sum(double (&v)[NV])
+{
+#pragma unroll
+    for (int o = 32; o >= 16; o >>= 1)
+#pragma unroll
+        for (int q = 0; q < NV; q++) v[q] += __shfl_down(v[q], o, 64);
+#pragma unroll
+    for (int q = 0; q < NV; q++) v[q] += row_shl<0x108>(v[q]);   // row_shl:8
+#pragma unroll
+    for (int q = 0; q < NV; q++) v[q] += row_shl<0x104>(v[q]);
+#pragma unroll
+    for (int q = 0; q < NV; q++) v[q] += row_shl<0x102>(v[q]);
+#pragma unroll
+    for (int q = 0; q < NV; q++) v[q] += row_shl<0x101>(v[q]);
+}
+
 // wave64 + block reduction of doubles; result valid in thread 0.
 __device__ __forceinline__ double block_sum(double v, double* lds)
 {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+    double w1[1] = {v};
+    wave_sum<1>(w1);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     __syncthreads();
-    if (lane == 0) lds[w] = v;
+    if (lane == 0) lds[w] = w1[0];
     __syncthreads();
     double t = 0.0;
     if (threadIdx.x == 0)
@@ -483,35 +512,56 @@ __device__ __forceinline__ Chunk my_chunk(const SceneDev& s, int blk)
 }
 
 // Sum of the nb per-block partials of `slot`, in a fixed order (thread t
-// takes partials t, t+256, ...; then a fixed shuffle/LDS tree), broadcast to
-// every thread.  Every block computing it gets the identical value.
+// takes partials t, t+256, ...; then a fixed wave and LDS tree), in every
+// thread.  Every block computing it gets the identical value.  Every thread
+// adds the waves' sums itself, so one barrier serves all NV values; a kernel
+// calls it once (its LDS is not reused).
 template <int NV>
 __device__ __forceinline__ void sum_partials(const SceneDev& s, int slot, int nb, double (&out)[NV])
 {
-    __shared__ double red[kBlock / 64];
-    __shared__ double bc[NV];
+    __shared__ double red[NV][kBlock / 64];
+    double acc[NV];
 #pragma unroll
     for (int q = 0; q < NV; q++) {
         gptr<const double> part = gbl<const double>(s.partials + (size_t)(slot + q) * s.max_blocks);
-        double acc = 0.0;
-        for (int b = threadIdx.x; b < nb; b += kBlock) acc += part[b];
-        const double t = block_sum(acc, red);
-        if (threadIdx.x == 0) bc[q] = t;
+        acc[q] = 0.0;
+        for (int b = threadIdx.x; b < nb; b += kBlock) acc[q] += part[b];
     }
+    wave_sum<NV>(acc);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0)
+#pragma unroll
+        for (int q = 0; q < NV; q++) red[q][w] = acc[q];
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < NV; q++) out[q] = bc[q];
+    for (int q = 0; q < NV; q++) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; k++) t += red[q][k];
+        out[q] = t;
+    }
 }
 
-// Block-reduce NV doubles and store them as the partials of solver block blk.
+// Block-reduce NV doubles and store them as the partials of solver block blk
+// (once a kernel, as above).
 template <int NV>
 __device__ __forceinline__ void put_partials(const SceneDev& s, int slot, double (&v)[NV], int blk)
 {
-    __shared__ double red[kBlock / 64];
+    __shared__ double red[NV][kBlock / 64];
+    double acc[NV];
 #pragma unroll
-    for (int q = 0; q < NV; q++) {
-        const double t = block_sum(v[q], red);
-        if (threadIdx.x == 0) s.partials[(size_t)(slot + q) * s.max_blocks + blk] = t;
+    for (int q = 0; q < NV; q++) acc[q] = v[q];
+    wave_sum<NV>(acc);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0)
+#pragma unroll
+        for (int q = 0; q < NV; q++) red[q][w] = acc[q];
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; k++) t += red[threadIdx.x][k];
+        s.partials[(size_t)(slot + threadIdx.x) * s.max_blocks + blk] = t;
     }
 }
 

@@ -1117,7 +1117,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_post(const SceneDev* scenes, cons
 // k_mg_step0's and k_pcg_dir's, in their order, so what one writes the
 // other reads through the same XCD's L2.  Per-cell form (each cell its
 // neighbours' z0) 8.3 us at 128^2, 10.1 us at 1024^2; an LDS window of whole
-// rows over linear chunks 97 us at 4096^2; this form 5.7, 8.2 and 39 us.
+// rows over linear chunks 97 us at 4096^2; this form 4.8, 7.3 and 36 us.
 constexpr int kUpR = kUpTile + 2;        // cells a side with the halo
 constexpr int kUpY = kUpTile / 2 + 2;    // level-1 cells a side that the halo's cells prolong from
 static_assert(kUpTile % 2 == 0 && kUpTile * kUpTile % kBlock == 0 && kBlock % kUpTile == 0, "whole rows of a tile a pass");

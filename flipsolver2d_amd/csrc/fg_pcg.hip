@@ -265,7 +265,8 @@ __device__ __forceinline__ double pcg_row(uint8_t cc, const float (&P)[5])
 // that wrote it.  The halo is addressed linearly, so a row's end couples to
 // the next row's first cell where the reference's matrix does.
 // Per cell over linear chunks 7.3 us at 128^2, 11.1 at 1024^2, 56 at 4096^2;
-// this form 6.7, 10.6 and 46 us.
+// this form 5.7, 9.1 and 42 us (6.7, 10.6 and 46 with the loads behind the flags and
+// the sums through LDS permutes).
 __global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, const int2* map, int it)
 {
     constexpr int R = kUpTile + 2;
@@ -273,9 +274,7 @@ __global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, cons
     const SceneBlock sb = scene_block(map, true);
     const SceneDev& s = scenes[sb.scene];
     cptr<SceneScalars> scr = cst(s.sc);
-    // one test after the uniform loads, so that they issue together
-    if (!s.active | (s.precond != kPrecondMG) | (scr->outer_done != 0) | (scr->inner_done != 0) | (sb.block >= s.up_blocks))
-        return;
+    if (!s.active | (s.precond != kPrecondMG) | (sb.block >= s.up_blocks)) return;
     const int I = s.I, J = s.J, C = I * J;
     const bool first = it == 0;
     gptr<const float> z = gbl<const float>(s.cu);
@@ -305,6 +304,10 @@ __global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, cons
         for (int u = 0; u < N; u++)
             cc[u] = code[min((i0 + a0 + u * (kBlock / kUpTile)) * J + min(j0 + b, J - 1), C - 1)];
         if (tile == t0) {
+            // the first tile's loads are on their way before the stop flags are read
+#pragma unroll
+            for (int u = 0; u < Q; u++) asm volatile("" : "+v"(zq[u]), "+v"(oq[u]));
+            if ((scr->outer_done != 0) | (scr->inner_done != 0)) return;
             if (!pcg_a_scalars(s, s.up_blocks, it, sb.block == 0 && threadIdx.x == 0, beta)) return;
         } else {
             __syncthreads();   // the tile before is done with the LDS
