@@ -1649,17 +1649,23 @@ int levelset_bands(Group& G, bool outside)
     // outside chain (NB-FLIP, far longer) keeps the count it launched
     int hint = 0;
     for (fg_scene* s : G.sc) hint = std::max(hint, outside ? s->ls_hint_out : (s->ls_hint > 0 ? s->ls_hint + 1 : 0));
+    // a band after the last one costs 2 us of launch, a poll 25 us of an idle
+    // device: where few bands can be left, all are launched and none polled
+    constexpr int kNoPoll = 10;
     int chunk = hint > 0 ? hint : kChunk;
+    const bool all = G.max_bands - (hint > 0 ? hint - 1 : 0) <= kNoPoll;
+    if (all) chunk = G.max_bands;
     int32_t flags[3];
     int launched = 0;
     for (int band = 0; band < G.max_bands; band += chunk, chunk = kChunk) {
         const int end = std::min(G.max_bands, band + chunk);
         for (int k = band; k < end; k++) launch_levelset_band(G.g.ls, G.L->stream, G.d, k, outside);
         launched = end;
+        if (all) break;
         FGCHK(poll_group(G, end - 1, flags));
         if (!flags[2]) break;
     }
-    if (outside)
+    if (outside && !all)
         for (fg_scene* s : G.sc) s->ls_hint_out = launched;
     return FG_OK;
 }
