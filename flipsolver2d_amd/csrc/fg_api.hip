@@ -1444,8 +1444,7 @@ int run_solve(Group& G, bool rhs_from_grid)
     // the next level's activity marks
     if (G.mg_levels > 1) launch_mg_mark(dim3(G.mg_grid[1], (unsigned)G.n), st, G.d, 1);
     for (int l = 1; l < G.mg_levels; l++) {
-        const dim3 gl(G.mg_grid[l], (unsigned)G.n);
-        launch_mg_galerkin(gl, st, G.d, l);
+        launch_mg_galerkin(dim3((unsigned)cdiv((int64_t)G.mg_grid[l] * kBlock, kGalCells), (unsigned)G.n), st, G.d, l);
         if (l + 1 < G.mg_levels)
             launch_mg_symmark(dim3(G.sym_grid[l] + G.mg_grid[l + 1], (unsigned)G.n), st, G.d, l, (int)G.sym_grid[l]);
         else

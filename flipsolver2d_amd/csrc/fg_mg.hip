@@ -220,131 +220,157 @@ __device__ __forceinline__ void static_for(F&& f)
 }
 
 template <int DI, int DJ>
-__device__ __forceinline__ void galerkin_add(double (&acc)[kMgStencil], uint32_t am, double w)
+__device__ __forceinline__ void galerkin_add(double (&acc)[kMgStencil], double w, double v)
 {
     if constexpr (DI >= -2 && DI <= 2 && DJ >= -2 && DJ <= 2) {
         constexpr int k = (DI + 2) * 5 + (DJ + 2);
-        acc[k] += ((am >> k) & 1u) ? w : 0.0;   // a select, not a branch
+        acc[k] = __builtin_fma(w, v, acc[k]);
     }
 }
 
 // One entry (value v) of fine row f = (2ci-1+A, 2cj-1+B) coupling it to
-// g = f + (EI, EJ): spread R_f v P_g over g's coarse parents.
+// g = f + (EI, EJ): spread R_f v P_g over g's coarse parents.  A weight has
+// 7 significant bits and v 24 (a float), so each product is exact in FP64
+// and the fused multiply-add rounds as the product and the sum would.
 template <int A, int B, int EI, int EJ>
-__device__ __forceinline__ void galerkin_spread(double (&acc)[kMgStencil], uint32_t am, double v)
+__device__ __forceinline__ void galerkin_spread(double (&acc)[kMgStencil], double v)
 {
     constexpr int ti = -1 + A + EI, tj = -1 + B + EJ;   // g - 2C
     constexpr int pi0 = half_floor(ti), pj0 = half_floor(tj);
     constexpr int pi1 = (ti & 1) ? pi0 + 1 : pi0 - 1, pj1 = (tj & 1) ? pj0 + 1 : pj0 - 1;
     constexpr double wc = w1c(A) * w1c(B);
-    galerkin_add<pi0, pj0>(acc, am, (wc * 0.5625) * v);
-    galerkin_add<pi0, pj1>(acc, am, (wc * 0.1875) * v);
-    galerkin_add<pi1, pj0>(acc, am, (wc * 0.1875) * v);
-    galerkin_add<pi1, pj1>(acc, am, (wc * 0.0625) * v);
+    galerkin_add<pi0, pj0>(acc, wc * 0.5625, v);
+    galerkin_add<pi0, pj1>(acc, wc * 0.1875, v);
+    galerkin_add<pi1, pj0>(acc, wc * 0.1875, v);
+    galerkin_add<pi1, pj1>(acc, wc * 0.0625, v);
 }
 
-// A_l = R A_{l-1} P, one coarse row C = (ci, cj) per thread: the fine cells
-// f, their stencil entries g and g's coarse parents sit at compile-time
-// offsets from C, so the 25 FP64 accumulators stay in registers.
-template <bool FINE0, typename MT>
-__device__ __forceinline__ void galerkin_row(const SceneDev& s, const MT& M, int l, int c, int ci, int cj)
+// The fine row A's (2ci - 1 + A) part of coarse row C = (ci, cj): its four
+// fine cells, their stencil entries and those entries' coarse parents sit at
+// compile-time offsets from C, so the 25 FP64 accumulators stay in registers.
+// Every load is unconditional (clamped fine index; a fine cell outside the
+// grid contributes zero).  Inactive fine rows hold all-zero coefficients
+// (level >= 1) or a non-fluid code (level 0): they add nothing.
+template <bool FINE0, int A, typename MT>
+__device__ __forceinline__ void galerkin_part(const SceneDev& s, const MT& M, int l, int ci, int cj,
+                                              double (&acc)[kMgStencil])
 {
-    const auto& L = M.lv[l];
-    const int CL = L.I * L.J;
-    // activity of the 5x5 coarse neighbourhood, bit (di+2)*5 + (dj+2)
-    uint32_t am = 0;
-    gptr<const uint8_t> act = gbl<const uint8_t>(L.act);
-#pragma unroll
-    for (int k = 0; k < kMgStencil; k++) {   // clamped loads, all issued together
-        const int ni = ci + k / 5 - 2, nj = cj + k % 5 - 2;
-        const bool in = ni >= 0 && ni < L.I && nj >= 0 && nj < L.J;
-        const uint8_t v = act[min(max(ni, 0), L.I - 1) * L.J + min(max(nj, 0), L.J - 1)];
-        am |= (in && v) ? 1u << k : 0u;
-    }
-    double acc[kMgStencil];
-#pragma unroll
-    for (int k = 0; k < kMgStencil; k++) acc[k] = 0.0;
     const int FI = FINE0 ? s.I : M.lv[l - 1].I, FJ = FINE0 ? s.J : M.lv[l - 1].J;
-    const int CF = FI * FJ;
-    // Every load is unconditional (clamped fine index; a fine cell outside
-    // the grid contributes zero), so the loads of all 16 fine rows can be in
-    // flight together instead of one branch-guarded batch after another.
-    // Inactive fine rows hold all-zero coefficients (level >= 1) or a
-    // non-fluid code (level 0): they add nothing.
+    const int fi = 2 * ci - 1 + A;
+    const bool row = fi >= 0 && fi < FI;
+    const int fr = min(max(fi, 0), FI - 1) * FJ;
     if constexpr (FINE0) {
         gptr<const uint8_t> code = gbl<const uint8_t>(s.stencil);
-        uint8_t cd[16];
-        static_for<16>([&](auto ab) {
-            constexpr int a = decltype(ab)::value / 4, b = decltype(ab)::value % 4;
-            const int fi = 2 * ci - 1 + a, fj = 2 * cj - 1 + b;
-            const bool in = fi >= 0 && fi < FI && fj >= 0 && fj < FJ;
-            const uint8_t k = code[min(max(fi, 0), FI - 1) * FJ + min(max(fj, 0), FJ - 1)];
-            cd[decltype(ab)::value] = in ? k : 0;
-        });
-        static_for<16>([&](auto ab) {
-            constexpr int a = decltype(ab)::value / 4, b = decltype(ab)::value % 4;
+        uint8_t cd[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) {
             const int fj = 2 * cj - 1 + b;
-            const uint8_t k = cd[decltype(ab)::value];
+            const uint8_t k = code[fr + min(max(fj, 0), FJ - 1)];
+            cd[b] = row && fj >= 0 && fj < FJ ? k : 0;
+        }
+        static_for<4>([&](auto bb) {
+            constexpr int b = decltype(bb)::value;
+            const int fj = 2 * cj - 1 + b;
+            const uint8_t k = cd[b];
             const double on = (k & 0x80) ? 1.0 : 0.0;
-            galerkin_spread<a, b, 0, 0>(acc, am, on * (double)((k >> 4) & 7));
-            galerkin_spread<a, b, -1, 0>(acc, am, (k & 1) ? -on : 0.0);
-            galerkin_spread<a, b, 1, 0>(acc, am, (k & 2) ? -on : 0.0);
-            galerkin_spread<a, b, 0, -1>(acc, am, ((k & 4) && fj > 0) ? -on : 0.0);   // not the row-wrapping coupling
-            galerkin_spread<a, b, 0, 1>(acc, am, ((k & 8) && fj < FJ - 1) ? -on : 0.0);
+            galerkin_spread<A, b, 0, 0>(acc, on * (double)((k >> 4) & 7));
+            galerkin_spread<A, b, -1, 0>(acc, (k & 1) ? -on : 0.0);
+            galerkin_spread<A, b, 1, 0>(acc, (k & 2) ? -on : 0.0);
+            galerkin_spread<A, b, 0, -1>(acc, ((k & 4) && fj > 0) ? -on : 0.0);   // not the row-wrapping coupling
+            galerkin_spread<A, b, 0, 1>(acc, ((k & 8) && fj < FJ - 1) ? -on : 0.0);
         });
     } else {
         gptr<const float> fc = gbl<const float>(M.lv[l - 1].coef);
-        gptr<const char> fb = (gptr<const char>)fc;
-        static_for<8>([&](auto hh) {   // two fine cells at a time: 50 loads in flight
-            constexpr int a = decltype(hh)::value / 2, b0 = 2 * (decltype(hh)::value % 2);
-            float v[2][kMgStencil];
-            bool in[2];
+        float v[4][kMgStencil];
+        float in[4];
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int fi = 2 * ci - 1 + a, fj = 2 * cj - 1 + b0 + h;
-                in[h] = fi >= 0 && fi < FI && fj >= 0 && fj < FJ;
-                const uint32_t f = (uint32_t)(min(max(fi, 0), FI - 1) * FJ + min(max(fj, 0), FJ - 1));
-#pragma unroll
-                for (int e = 0; e < kMgStencil; e++)
-                    v[h][e] = *(gptr<const float>)(fb + (f * (uint32_t)kMgRowStride + (uint32_t)e) * 4u);
-            }
-            static_for<2>([&](auto h2) {
-                constexpr int h = decltype(h2)::value, b = b0 + h;
-                static_for<kMgStencil>([&](auto ee) {
-                    constexpr int e = decltype(ee)::value;
-                    galerkin_spread<a, b, e / 5 - 2, e % 5 - 2>(acc, am, in[h] ? (double)v[h][e] : 0.0);
-                });
+        for (int b = 0; b < 4; b++) {
+            const int fj = 2 * cj - 1 + b;
+            in[b] = mask01(row && fj >= 0 && fj < FJ);
+            load_coef_row(fc, fr + min(max(fj, 0), FJ - 1), v[b]);
+        }
+        static_for<4>([&](auto bb) {
+            constexpr int b = decltype(bb)::value;
+            static_for<kMgStencil>([&](auto ee) {
+                constexpr int e = decltype(ee)::value;
+                galerkin_spread<A, b, e / 5 - 2, e % 5 - 2>(acc, (double)(v[b][e] * in[b]));
             });
         });
     }
-#pragma unroll
-    for (int k = 0; k < kMgStencil; k++) L.coef[(size_t)c * kMgRowStride + k] = (float)(0.25 * acc[k]);
 }
 
+// A_l = R A_{l-1} P: kGalCells coarse rows a block, wave a summing fine row
+// a's part of each (lane = coarse row), the four parts added in LDS, entries
+// of inactive coarse neighbours dropped, and the row written as 16-byte
+// stores.  The parts are sums of products of few bits, exact in FP64 on the
+// upper levels, so where the order of the sums changed, they hardly do.
+// Bound by instruction issue: 1,600 multiply-adds and 400 conversions a row
+// (a wave a quarter of them, since the small levels have a few waves for the
+// whole chip).  A thread a row, with the activity selected at every addition
+// (10 us at any size below 128^2), took 11.1 us a launch at 128^2 and 100 us
+// at 4096^2; this form 7.7 and 105 us (the large one is the coefficients' traffic: 1.4 GB
+// over its eight levels), 14.4 and 12.6 us at 1024^2.
 // An inactive row must hold zeros; its dinv, not yet rewritten for this
 // hierarchy, says whether it held any: +0 (bit pattern 0) only on a row that
 // was inactive before (or never set: the arena starts zeroed), whose
 // coefficients are zero already -- most of the level, and most of its writes.
 __global__ void __launch_bounds__(kBlock) k_mg_galerkin(const SceneDev* scenes, int l)
 {
+    static_assert(kGalCells == 64 && kBlock == 256, "a coarse row a lane, a fine row a wave");
+    __shared__ double part[4][kMgStencil][kGalCells];
     const SceneDev& s = scenes[blockIdx.y];
     if (!s.active || s.precond != kPrecondMG) return;
     const auto& M = *cst(s.mg);
     if (l >= M.n) return;
     const auto& L = M.lv[l];
-    const int CL = L.I * L.J;
-    const int c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= CL) return;
-    if (!L.act[c]) {
-        if (__float_as_uint(gbl<const float>(L.dinv)[c]) != 0u) {
-#pragma unroll
-            for (int k = 0; k < kMgStencil; k++) L.coef[(size_t)c * kMgRowStride + k] = 0.f;
-        }
-        return;
-    }
+    const int CL = L.I * L.J, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if ((int)blockIdx.x * kGalCells >= CL) return;
+    const int c0 = blockIdx.x * kGalCells + lane, c = min(c0, CL - 1);
+    gptr<const uint8_t> act = gbl<const uint8_t>(L.act);
+    const bool on = c0 < CL && act[c] != 0;
+    const bool clear = c0 < CL && !on && __float_as_uint(gbl<const float>(L.dinv)[c]) != 0u;
     const int ci = c / L.J, cj = c - ci * L.J;
-    if (l == 1) galerkin_row<true>(s, M, l, c, ci, cj);
-    else galerkin_row<false>(s, M, l, c, ci, cj);
+    const bool any = __any(on);   // the block's rows: the same in every wave
+    if (any) {
+        double acc[kMgStencil];
+#pragma unroll
+        for (int k = 0; k < kMgStencil; k++) acc[k] = 0.0;
+        if (l == 1) {
+            if (w == 0) galerkin_part<true, 0>(s, M, l, ci, cj, acc);
+            else if (w == 1) galerkin_part<true, 1>(s, M, l, ci, cj, acc);
+            else if (w == 2) galerkin_part<true, 2>(s, M, l, ci, cj, acc);
+            else galerkin_part<true, 3>(s, M, l, ci, cj, acc);
+        } else {
+            if (w == 0) galerkin_part<false, 0>(s, M, l, ci, cj, acc);
+            else if (w == 1) galerkin_part<false, 1>(s, M, l, ci, cj, acc);
+            else if (w == 2) galerkin_part<false, 2>(s, M, l, ci, cj, acc);
+            else galerkin_part<false, 3>(s, M, l, ci, cj, acc);
+        }
+#pragma unroll
+        for (int k = 0; k < kMgStencil; k++) part[w][k][lane] = acc[k];
+    }
+    __syncthreads();
+    if (!on && !clear) return;
+    // wave w: entries 4w .. 4w+3 and 16+4w .. 19+4w (the row has 25)
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    gptr<float> out = gbl(L.coef) + (size_t)c * kMgRowStride;
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int k0 = 16 * h + 4 * w;
+        if (k0 >= kMgStencil) break;
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int k = min(k0 + e, kMgStencil - 1), ni = ci + k / 5 - 2, nj = cj + k % 5 - 2;
+            const bool in = ni >= 0 && ni < L.I && nj >= 0 && nj < L.J;
+            const bool use = act[min(max(ni, 0), L.I - 1) * L.J + min(max(nj, 0), L.J - 1)] != 0 && in && on;
+            double t = 0.0;
+            if (any) t = ((part[0][k][lane] + part[1][k][lane]) + part[2][k][lane]) + part[3][k][lane];
+            x[e] = use ? (float)(0.25 * t) : 0.f;
+        }
+        if (k0 + 4 <= kMgStencil) *(gptr<v4>)(out + k0) = v4{x[0], x[1], x[2], x[3]};
+        else out[k0] = x[0];   // entry 24
+    }
 }
 
 // Mirror the upper entries into the lower ones (exact symmetry) and form the
