@@ -1669,6 +1669,11 @@ int levelset_bands(Group& G, bool outside)
     return FG_OK;
 }
 
+// Whether k_sdf_materials takes more lanes a bin: the group's bins, a wave
+// for 16 of them, would leave SIMDs without one (see kSdfLanesFew).
+bool few_bins(const Group& G) { return (int64_t)G.g.bins.x * (kBlock / kSdfLanes) * G.n <= kSdfFewBins; }
+dim3 few_bins_grid(const Group& G) { return dim3(G.g.bins.x * (kSdfLanesFew / kSdfLanes), (unsigned)G.n); }
+
 int run_stage(Group& G, int stage)
 {
     fg_ctx* ctx = G.ctx;
@@ -1691,7 +1696,7 @@ int run_stage(Group& G, int stage)
         launch_scatter(g.parts, st, d);
         launch_fixup(g.cells, st, d);
         launch_gather(g.parts, st, d);
-        launch_finalize(g.one, st, d, 1);
+        launch_finalize(g.one, st, d, 1, g.parts.x);
         kp.done(G.parts);
         break;
     }
@@ -1720,7 +1725,7 @@ int run_stage(Group& G, int stage)
         launch_scatter(D.g.parts, st, D.d);
         launch_fixup(D.g.cells, st, D.d);
         launch_gather(D.g.parts, st, D.d);
-        launch_finalize(D.g.one, st, D.d, 4);
+        launch_finalize(D.g.one, st, D.d, 4, D.g.parts.x);
         break;
     }
     case FG_STAGE_P2G: {
@@ -1736,7 +1741,7 @@ int run_stage(Group& G, int stage)
     case FG_STAGE_SDF: {
         {
             KProf kp(G, FG_K_SDF, true);
-            launch_sdf_materials(g.bins, st, d);
+            launch_sdf_materials(few_bins(G) ? few_bins_grid(G) : g.bins, st, d, few_bins(G));
             kp.done(0);
         }
         // afterTransfer (flipsolver2d.cpp:390-410), before the level set and
@@ -1793,7 +1798,7 @@ int run_stage(Group& G, int stage)
         KProf kp(G, FG_K_G2P, true);
         launch_g2p_count(g.parts, st, d);
         kp.done(G.parts);
-        launch_finalize(g.one, st, d, 2);
+        launch_finalize(g.one, st, d, 2, g.parts.x);
         break;
     }
     case FG_STAGE_COUNT:
@@ -1898,7 +1903,7 @@ int run_nb_substep(Group& G, Timer& tm)
         launch_scatter(g.parts, st, d);
         launch_fixup(g.cells, st, d);
         launch_gather(g.parts, st, d);
-        launch_finalize(g.one, st, d, 1);
+        launch_finalize(g.one, st, d, 1, g.parts.x);
         kp.done(G.parts);
     }
     tm.lap(FG_STAGE_REBIN);
@@ -1920,7 +1925,7 @@ int run_nb_substep(Group& G, Timer& tm)
     // combination), extrapolateLevelsetInside, updateMaterials, body forces
     {
         KProf kp(G, FG_K_SDF, true);
-        launch_sdf_materials(g.bins, st, d);
+        launch_sdf_materials(few_bins(G) ? few_bins_grid(G) : g.bins, st, d, few_bins(G));
         kp.done(0);
     }
     tm.lap(FG_STAGE_SDF);
@@ -2012,7 +2017,7 @@ int ensure_vmax(fg_ctx* ctx, Lane* L, const std::vector<fg_scene*>& scenes)
     Group G;
     FGCHK(make_group(ctx, need, {}, G, false, L));
     launch_max_v2(G.g.parts, G.L->stream, G.d);
-    launch_finalize(G.g.one, G.L->stream, G.d, 2);
+    launch_finalize(G.g.one, G.L->stream, G.d, 2, G.g.parts.x);
     FGCHK(read_group_scalars(G));
     for (fg_scene* s : need) s->vmax_ready = true;
     return FG_OK;

@@ -239,28 +239,37 @@ __global__ void __launch_bounds__(kBlock) k_p2g(const SceneDev* scenes)
 // lane needs besides the particles is issued at the top, in one round: the
 // window rows' bounds, the bin's 3 x 4 cell boundaries (its cells' particle
 // counts) and the materials of the cells the lane writes.
-template <bool kExact>
+// A bin has LANES lanes: 4, two or three whole window rows each, or 32, of
+// which 27 take a third of a row each (every kSplit-th run of U particles).
+// With a wave a SIMD or less (a 128^2 scene is 116 waves of 4-lane bins) the
+// kernel is one lane's chain of loads, six rounds long with 4 lanes and one
+// with 32: 36.5 -> 10.7 us at 128^2.  Once the chip is full the rounds overlap
+// and the 32 lanes' reductions cost more (8 lanes: no gain at 1024^2, 8 % lost
+// on 256 mixed scenes).
+template <int LANES, bool kExact>
 __device__ __forceinline__ void sdf_bins(const SceneDev& s)
 {
-    static_assert(kSdfLanes >= 4 && kSdfLanes <= 64 && (kSdfLanes & (kSdfLanes - 1)) == 0,
-                  "a bin's lanes are a power-of-two group inside one wave");
+    static_assert(LANES == 4 || LANES == 32, "a bin's lanes are a power-of-two group inside one wave");
+    constexpr int kSplit = LANES == 32 ? 3 : 1;          // lanes a window row
+    constexpr int kRowLanes = LANES == 32 ? 9 : LANES;   // window rows taken at once
     const int I = s.I, J = s.J;
     const int nbI = (I + 2) / 3, nbJ = (J + 2) / 3;
-    const int sub = threadIdx.x & (kSdfLanes - 1);
-    const int bin = xcd_tile(blockIdx.x, gridDim.x) * (kBlock / kSdfLanes) + threadIdx.x / kSdfLanes;
+    const int sub = threadIdx.x & (LANES - 1);
+    const int bin = xcd_tile(blockIdx.x, gridDim.x) * (kBlock / LANES) + threadIdx.x / LANES;
     if (bin >= nbI * nbJ) return;   // all lanes of a bin leave together
     const int bi = bin / nbJ, bj = bin - (bin / nbJ) * nbJ;
     const int r0 = max(0, 3 * bi - 3), r1 = min(I, 3 * bi + 6);
     const int c0 = max(0, 3 * bj - 3), c1 = min(J, 3 * bj + 6);
     const int i0 = 3 * bi, j0 = 3 * bj;
-    // this lane's window rows r0+sub, r0+sub+kSdfLanes, ... and cells
-    // q = sub, sub+kSdfLanes, ... of the bin (q = 3a + b)
-    constexpr int NR = (9 + kSdfLanes - 1) / kSdfLanes;
+    // this lane's window rows r0+row, r0+row+kRowLanes, ... (its share of each)
+    // and cells q = sub, sub+LANES, ... of the bin (q = 3a + b)
+    constexpr int NR = (9 + kRowLanes - 1) / kRowLanes, NQ = (9 + LANES - 1) / LANES;
+    const int row = sub / kSplit, share = sub - row * kSplit;
     gptr<const int32_t> cs = gbl<const int32_t>(s.cellStart);
     int rb[NR], re[NR];
 #pragma unroll
     for (int q = 0; q < NR; q++) {   // clamped rows: every load unconditional
-        const int r = r0 + sub + q * kSdfLanes, rc = min(r, r1 - 1);
+        const int r = r0 + row + q * kRowLanes, rc = min(r, r1 - 1);
         rb[q] = cs[rc * J + c0];
         re[q] = cs[rc * J + c1];
     }
@@ -269,19 +278,19 @@ __device__ __forceinline__ void sdf_bins(const SceneDev& s)
     for (int a = 0; a < 3; a++)
 #pragma unroll
         for (int k = 0; k < 4; k++) bnd[a][k] = cs[min(i0 + a, I - 1) * J + min(j0 + k, J)];
-    int8_t mq[NR];
+    int8_t mq[NQ];
     if (!kExact) {
         gptr<const int8_t> mat = gbl<const int8_t>(s.mat);
 #pragma unroll
-        for (int q = 0; q < NR; q++) {   // cell sub + q kSdfLanes (clamped: loads unconditional)
-            const int cq = min(sub + q * kSdfLanes, 8), a = cq / 3, b = cq - a * 3;
+        for (int q = 0; q < NQ; q++) {   // cell sub + q LANES (clamped: loads unconditional)
+            const int cq = min(sub + q * LANES, 8), a = cq / 3, b = cq - a * 3;
             mq[q] = mat[min(i0 + a, I - 1) * J + min(j0 + b, J - 1)];
         }
     }
 #pragma unroll
     for (int q = 0; q < NR; q++) {
-        const int r = r0 + sub + q * kSdfLanes;
-        if (r >= r1) re[q] = rb[q];
+        const int r = r0 + row + q * kRowLanes;
+        if (r >= r1 || row >= kRowLanes) re[q] = rb[q];
     }
     float cx[3], cy[3];
 #pragma unroll
@@ -318,8 +327,8 @@ __device__ __forceinline__ void sdf_bins(const SceneDev& s)
 #pragma unroll
     for (int q = 0; q < NR; q++) {
         const int e = re[q];
-        constexpr int U = 24;   // loads in flight per lane (a row segment holds ~9 ppc)
-        for (int k0 = rb[q]; k0 < e; k0 += U) {
+        constexpr int U = LANES == 32 ? 12 : 24;   // loads in flight per lane (a row segment holds ~9 ppc)
+        for (int k0 = rb[q] + share * U; k0 < e; k0 += kSplit * U) {
             // past the row's end a lane re-reads its last particle: the
             // minimum of a value with itself changes nothing, so no branch
             float2 pp[U];
@@ -346,16 +355,16 @@ __device__ __forceinline__ void sdf_bins(const SceneDev& s)
 #pragma unroll
         for (int b = 0; b < 3; b++) {
 #pragma unroll
-            for (int o = 1; o < kSdfLanes; o <<= 1) {
+            for (int o = 1; o < LANES; o <<= 1) {
                 const float t = __shfl_xor(d2[a][b], o, 64);
                 if (t < d2[a][b]) d2[a][b] = t;
             }
         }
-    // cell q of the bin is written by lane q mod kSdfLanes (q, a, b
+    // cell q of the bin is written by lane q mod LANES (q, a, b
     // compile-time, so the arrays stay in registers)
 #pragma unroll
     for (int q = 0; q < 9; q++) {
-        if ((q & (kSdfLanes - 1)) != sub) continue;
+        if ((q & (LANES - 1)) != sub) continue;
         const int a = q / 3, b = q - (q / 3) * 3;
         const int i = i0 + a, j = j0 + b;
         if (i >= I || j >= J) continue;
@@ -370,7 +379,7 @@ __device__ __forceinline__ void sdf_bins(const SceneDev& s)
         s.fsdf[c] = sdf;
         s.pcount[c] = min(n, 2 * s.ppc);
         if (s.nb) continue;   // NB-FLIP updates the materials from its final level set
-        int8_t m = mq[q / kSdfLanes];
+        int8_t m = mq[q / LANES];
         if (sdf < 0.f) {
             if (is_empty(m)) m = M_FLUID;
         } else {
@@ -380,11 +389,12 @@ __device__ __forceinline__ void sdf_bins(const SceneDev& s)
     }
 }
 
+template <int LANES>
 __global__ void __launch_bounds__(kBlock) k_sdf_materials(const SceneDev* scenes)
 {
     const SceneDev& s = scenes[blockIdx.y];
     if (!s.active) return;
-    sdf_bins<false>(s);
+    sdf_bins<LANES, false>(s);
 }
 
 // The exact SDF of every cell that holds particles, for a scene in which no
@@ -395,7 +405,7 @@ __global__ void __launch_bounds__(kBlock) k_sdf_exact(const SceneDev* scenes)
 {
     const SceneDev& s = scenes[blockIdx.y];
     if (!s.active || !s.sdf_short || cst(s.sc)->sdf_known) return;
-    sdf_bins<true>(s);
+    sdf_bins<kSdfLanes, true>(s);
 }
 
 // ---------------------------------------------------------------------------
@@ -1026,7 +1036,11 @@ namespace fg {
     void launch_##name(dim3 g, hipStream_t st, const SceneDev* sc, T a) { fg_launch(k_##name, g, dim3(kBlock), st, sc, a); }
 FG_LAUNCH0(stencil)
 FG_LAUNCH0(p2g)
-FG_LAUNCH0(sdf_materials)
+void launch_sdf_materials(dim3 g, hipStream_t st, const SceneDev* sc, bool few)
+{
+    if (few) fg_launch(k_sdf_materials<kSdfLanesFew>, g, dim3(kBlock), st, sc);
+    else fg_launch(k_sdf_materials<kSdfLanes>, g, dim3(kBlock), st, sc);
+}
 FG_LAUNCH0(sdf_exact)
 FG_LAUNCH1(extrapolate, int, which)
 void launch_levelset_init(dim3 g, hipStream_t st, const SceneDev* sc, bool outside)

@@ -76,13 +76,15 @@ FG_DECLARE_LAUNCH(scatter);
 FG_DECLARE_LAUNCH(fixup);
 FG_DECLARE_LAUNCH(gather);
 FG_DECLARE_LAUNCH(g2p_count);
-FG_DECLARE_LAUNCH(finalize, int what);
+// pblocks: the most particle blocks of a scene of the launch
+FG_DECLARE_LAUNCH(finalize, int what, unsigned pblocks);
 constexpr int kScanTileCells = kBlock * 16;
 
 // fg_grid.hip
 FG_DECLARE_LAUNCH(stencil);
 FG_DECLARE_LAUNCH(p2g);
-FG_DECLARE_LAUNCH(sdf_materials);
+// few: the launch's bins leave the chip idle (kSdfFewBins), so a bin takes kSdfLanesFew lanes
+FG_DECLARE_LAUNCH(sdf_materials, bool few);
 FG_DECLARE_LAUNCH(sdf_exact);
 FG_DECLARE_LAUNCH(extrapolate, int which);
 // outside: extrapolateLevelsetOutside; else extrapolateLevelsetInside
