@@ -62,7 +62,7 @@ HBM_PEAK_GBS = 8000.0
 #              dinv, y_{l+1}; y) and the 100 B of each stored row
 #   nb_euler   NB-FLIP's Euler pass: U, V and the level set read once and
 #              their advected copies written, 8 (F + C) per substep
-#   visc_cg    the viscosity CG (U and V together): 216 B a cell and iteration,
+#   visc_cg    the viscosity CG (U and V together): 192 B a cell and iteration,
 #              timed over the whole iteration stretch with its polls
 #   mg_coarse  per scene and V-cycle: 4 B per cell of the levels' dinv, of its
 #              input and of its output, once each the 100 B of every row above
@@ -80,7 +80,7 @@ KERNEL_BYTES = {
     "mg_pp": ("K_MG_PP", 1.0, "bytes", ["k_mg_pp"]),
     "mg_coarse": ("K_MG_COARSE", 1.0, "bytes", ["k_mg_coarse"]),
     "nb_euler": ("K_NB_EULER", 1.0, "bytes", ["k_nb_euler"]),
-    "visc_cg": ("K_VISC", 1.0, "bytes", ["k_visc_spmv", "k_visc_update", "k_visc_dir", "k_visc_red"]),
+    "visc_cg": ("K_VISC", 1.0, "bytes", ["k_visc_p", "k_visc_x"]),
 }
 STEP_FAMILIES = ["p2g", "particles", "sdf", "pcg_a", "pcg_b", "mg_down0", "mg_up0", "mg_resid", "mg_pp",
                  "mg_coarse"]

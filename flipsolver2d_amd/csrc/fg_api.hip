@@ -160,6 +160,7 @@ struct fg_scene {
     SceneDev* hpin = nullptr;     // pinned staging for descriptor uploads
     SceneScalars* hsc = nullptr;  // pinned readback of the scalars
     int iters_hint[2] = {0, 0};   // first-sweep PCG iterations of the last solve (pressure, density)
+    int visc_hint = 0;            // iterations of the last viscosity solve
     int ls_hint = 0;              // level-set bands the last substep ran
     int ls_hint_out = 0;          // NB-FLIP: bands the last outside extrapolation launched
     int64_t n_bound = 0;          // upper bound of live particles (host mirror)
@@ -649,7 +650,7 @@ void stats_reset(fg_stats* st)
 // launch geometry
 // --------------------------------------------------------------------------
 struct Geo {
-    dim3 cells, parts, scan, scan1, faces, extrap, ls, one, pcg, bins, p2g, nodes;
+    dim3 cells, parts, scan, scan1, faces, extrap, ls, one, pcg, bins, p2g, nodes, visc;
 };
 
 // x extents of one scene's launches (y is set by the launch group)
@@ -669,6 +670,7 @@ Geo geometry(const fg_scene* s)
     g.pcg = dim3((unsigned)s->pcg_blocks);
     g.bins = dim3((unsigned)cdiv(cdiv(s->I, 3) * cdiv(s->J, 3), kBlock / kSdfLanes));
     g.p2g = dim3((unsigned)(cdiv(s->I, 16) * cdiv(s->J, 16)));
+    g.visc = g.p2g;   // kViscTile = 16
     g.nodes = dim3((unsigned)cdiv((int64_t)(s->I + 1) * (s->J + 1), kBlock));
     return g;
 }
@@ -676,16 +678,16 @@ Geo geometry(const fg_scene* s)
 void geo_max(Geo& a, const Geo& b)
 {
     dim3* pa[] = {&a.cells, &a.parts, &a.scan, &a.scan1, &a.faces, &a.extrap,
-                  &a.ls, &a.one, &a.pcg, &a.bins, &a.p2g, &a.nodes};
+                  &a.ls, &a.one, &a.pcg, &a.bins, &a.p2g, &a.nodes, &a.visc};
     const dim3* pb[] = {&b.cells, &b.parts, &b.scan, &b.scan1, &b.faces, &b.extrap,
-                        &b.ls, &b.one, &b.pcg, &b.bins, &b.p2g, &b.nodes};
-    for (int k = 0; k < 12; k++) pa[k]->x = std::max(pa[k]->x, pb[k]->x);
+                        &b.ls, &b.one, &b.pcg, &b.bins, &b.p2g, &b.nodes, &b.visc};
+    for (int k = 0; k < 13; k++) pa[k]->x = std::max(pa[k]->x, pb[k]->x);
 }
 
 void geo_set_y(Geo& a, int n)
 {
     dim3* pa[] = {&a.cells, &a.parts, &a.scan, &a.scan1, &a.faces, &a.extrap,
-                  &a.ls, &a.one, &a.pcg, &a.bins, &a.p2g, &a.nodes};
+                  &a.ls, &a.one, &a.pcg, &a.bins, &a.p2g, &a.nodes, &a.visc};
     for (dim3* d : pa) d->y = (unsigned)n;
 }
 
@@ -1570,9 +1572,9 @@ int run_solve(Group& G, bool rhs_from_grid)
 // applyViscosity and the second project() of FlipSolver::step
 // (flipsolver2d.cpp:446-453) for the scenes of G with viscosity, as a
 // sub-group: the light model's matrix, its Jacobi-preconditioned CG on U and
-// V together (polled every kViscPoll iterations), the result, then the
+// V together (polled), the result, then the
 // pressure solve again with the substep's matrix and its plain application.
-constexpr int kViscPoll = 8;
+constexpr int kViscFirst = 16, kViscPoll = 4, kViscHintMax = 256;
 constexpr int kViscMaxIters = 20000;
 constexpr double kViscTol = 1e-12;   // relative residual of each system (FP64)
 int run_viscosity(Group& G)
@@ -1587,46 +1589,38 @@ int run_viscosity(Group& G)
     Group V;
     FGCHK(make_group(G.ctx, vs, vst, V, true, G.L));
     hipStream_t st = V.L->stream;
-    const dim3 one(1, V.n);
     const double tol2 = kViscTol * kViscTol;
     launch_visc_setup(V.g.cells, st, V.d);
-    launch_visc_red(one, st, V.d, 0, tol2);
-    int it = 0, open = 1;
+    // the first poll comes after as many iterations as the longest scene took
+    // the last time (and the launch whose sums show the stop), later ones
+    // every kViscPoll
+    int it = 0, open = 1, hint = 0;
+    for (fg_scene* s : vs) hint = std::max(hint, s->visc_hint);
     KProf kp(V, FG_K_VISC);
-    while (open && it < kViscMaxIters) {
-        for (int k = 0; k < kViscPoll; k++) {
-            launch_visc_spmv(V.g.cells, st, V.d);
-            launch_visc_red(one, st, V.d, 1, tol2);
-            launch_visc_update(V.g.cells, st, V.d);
-            launch_visc_red(one, st, V.d, 2, tol2);
-            launch_visc_dir(V.g.cells, st, V.d);
+    for (int chunk = hint > 0 ? hint + 1 : kViscFirst; open && it < kViscMaxIters; chunk = kViscPoll) {
+        for (int k = 0; k < chunk; k++, it++) {
+            launch_visc_p(V.g.visc, st, V.d, it, tol2);
+            launch_visc_x(V.g.cells, st, V.d, it);
         }
-        it += kViscPoll;
         launch_visc_flags(st, V.d, V.n, V.L->bflags);
         HIPCHK(hipMemcpyAsync(V.L->bflags_host, V.L->bflags, sizeof(int32_t), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
         open = V.L->bflags_host[0];
     }
-    // per cell and iteration, U and V together: spmv 24 (d, e, n) + 16 (p)
-    // + 16 (q); update 8 (d) + 16 x 4 read (p, x, r, q) + 16 x 2 written;
-    // direction 8 + 16 x 2 read + 16 written
-    kp.done(216 * V.cells * (int64_t)it);
+    // per cell and iteration, U and V together: p 24 (d, e, n) + 16 x 2 read
+    // (r, p_old) + 16 x 2 written (p, q); x 8 (d) + 16 x 4 read (p, x, r, q)
+    // + 16 x 2 written
+    kp.done(192 * V.cells * (int64_t)it);
     launch_visc_apply(V.g.cells, st, V.d);
-    for (int k = 0; k < V.n; k++) {
-        double sc[kViscScalars];
-        HIPCHK(hipMemcpyAsync(sc, V.sc[k]->h.vsc, sizeof(sc), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        if (fg_stats* stats = V.st[k]) {
-            stats->viscosity_iters = std::max(stats->viscosity_iters, (int32_t)std::max(sc[14], sc[15]));
-            if (sc[12] == 0.0 || sc[13] == 0.0) stats->converged = 0;
-        }
-    }
     // project() again: rhs from the viscous grid, the same matrix snapshot
     const int r = run_solve(V, true);
     for (int k = 0; k < V.n; k++) {
         fg_stats* stats = V.st[k];
-        if (!stats) continue;
         const SceneScalars& sc = *V.sc[k]->hsc;
+        V.sc[k]->visc_hint = std::min(sc.visc_iters, kViscHintMax);
+        if (!stats) continue;
+        stats->viscosity_iters = std::max(stats->viscosity_iters, sc.visc_iters);
+        if (!sc.visc_done) stats->converged = 0;
         stats->pressure_iters = std::max(stats->pressure_iters, sc.total_iters);
         stats->pressure_sweeps = std::max(stats->pressure_sweeps, sc.sweeps);
         stats->pressure_rel_resid = sc.bb > 0 ? std::sqrt(sc.rr64 / sc.bb) : 0.0;

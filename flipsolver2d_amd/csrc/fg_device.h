@@ -96,6 +96,8 @@ struct SceneScalars {
     int32_t mg_stored[kMgMaxLevels];  // active rows per level that read stored coefficients
     int32_t reseeded;       // particles reseedParticles added this substep
     int32_t reseed_dropped; // reseeds beyond the particle capacity
+    int32_t visc_iters;     // iterations of the last viscosity solve (the longer of U and V)
+    int32_t visc_done;      // both met their tolerance
     int32_t sdf_known;      // some cell's fluid SDF is positive (extrapolateLevelsetInside has a known cell)
 };
 
@@ -223,8 +225,8 @@ struct SceneDev {
     float* adv_visc;
     int32_t* src_id;
 };
-// viscosity CG scalars (per system s = 0 (U), 1 (V)): bb, rz, pq, rr, alpha,
-// beta, done at index 2 k + s; the iteration counts at 14, 15
+// viscosity CG scalars (per system s = 0 (U), 1 (V)): bb at s, rz of even and
+// odd iterations at 2 + s and 4 + s, done at 12 + s, the iteration counts at 14 + s
 constexpr int kViscSlots = 4;         // per-block partials: two dots x two systems
 constexpr int kViscScalars = 16;
 constexpr int kMaxEmitters = 256;

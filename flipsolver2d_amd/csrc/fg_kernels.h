@@ -140,14 +140,12 @@ FG_DECLARE_LAUNCH(reseed_count);
 FG_DECLARE_LAUNCH(reseed_write);
 FG_DECLARE_LAUNCH(reseed_commit);
 
-// fg_visc.hip: the light viscosity model (cells; red: one block a scene)
+// fg_visc.hip: the light viscosity model (cells; p: kViscTile x kViscTile tiles)
 FG_DECLARE_LAUNCH(visc_grid);
 FG_DECLARE_LAUNCH(visc_setup);
-FG_DECLARE_LAUNCH(visc_spmv);
-FG_DECLARE_LAUNCH(visc_update);
-FG_DECLARE_LAUNCH(visc_dir);
+FG_DECLARE_LAUNCH(visc_p, int it, double tol2);
+FG_DECLARE_LAUNCH(visc_x, int it);
 FG_DECLARE_LAUNCH(visc_apply);
-FG_DECLARE_LAUNCH(visc_red, int what, double tol2);
 void launch_visc_flags(hipStream_t st, const SceneDev* scenes, int n, int32_t* out);
 
 // fg_nbflip.hip: NBFlipSolver's grid passes (nb_euler over the (I+1) x (J+1)

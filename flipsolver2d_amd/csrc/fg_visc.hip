@@ -14,13 +14,19 @@
 //   for rho U and rho V on the cells' faces (i, j), by Jacobi-preconditioned
 //   CG in FP64 from zero (Eigen's ConjugateGradient with its diagonal
 //   preconditioner), both systems in the same launches:
-//     k_visc_setup    matrix, b, x = 0, r = b, p = r / d; partials bb, rz
-//     k_visc_spmv     q = A p; partials p.q
-//     k_visc_update   x += alpha p, r -= alpha q; partials r.r, r.z
-//     k_visc_dir      p = r / d + beta p
-//     k_visc_red      one block a scene: the sums, alpha, beta, the stop test
-//                     ||r||^2 < tol^2 ||b||^2 (a stopped system keeps alpha 0)
+//     k_visc_setup    matrix, b, x = 0, r = b; partials bb, rz
+//     k_visc_p        the sums of the kernel before: the stop test
+//                     ||r||^2 < tol^2 ||b||^2 and beta; p = r / d + beta p_old;
+//                     q = A p; partials p.q
+//     k_visc_x        the sums of p.q: alpha; x += alpha p, r -= alpha q;
+//                     partials r.r, r.z
 //     k_visc_apply    U = x / rho, V likewise (faces i < I, j < J)
+// Two launches an iteration: every block sums the partials of the kernel
+// before it, in the same order, and p is formed where it is multiplied (in
+// LDS, once a cell and halo cell) and alternates between two buffers.  With
+// the sums in one-block launches and p in one of its own an iteration of
+// eight 256^2 scenes was five launches and 42 us; this form 29 us (k_visc_p 17,
+// k_visc_x 10).
 // The second projection (flipsolver2d.cpp:450-453) reuses the solve.
 #include "fg_kernels.h"
 
@@ -65,18 +71,62 @@ __global__ void __launch_bounds__(kBlock) k_visc_grid(const SceneDev* scenes)
     s.cvisc[c] = v;
 }
 
-// the four per-block partials of one block (thread 0 stores them)
-__device__ __forceinline__ void visc_put(const SceneDev& s, double a, double b, double c, double d)
+// Sums over the block of NV doubles, to out[q * stride + block].
+template <int NV>
+__device__ __forceinline__ void visc_put(double* out, int stride, double (&v)[NV])
 {
-    __shared__ double red[kBlock / 64];
-    const int cb = visc_blocks(s);
-    const double v[4] = {a, b, c, d};
+    __shared__ double red[NV][kBlock / 64];
+    wave_sum<NV>(v);
+    if ((threadIdx.x & 63) == 0)
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const double t = block_sum(v[q], red);
-        if (threadIdx.x == 0) s.vpart[(size_t)q * cb + blockIdx.x] = t;
+        for (int q = 0; q < NV; q++) red[q][threadIdx.x >> 6] = v[q];
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; k++) t += red[threadIdx.x][k];
+        gbl(out)[(size_t)threadIdx.x * stride + blockIdx.x] = t;
     }
 }
+
+// The sums of n partials of NV slots, the same in every thread and block.
+template <int NV>
+__device__ __forceinline__ void visc_sum(const double* part, int stride, int n, double (&out)[NV])
+{
+    __shared__ double red[NV][kBlock / 64];
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        out[q] = 0.0;
+        for (int b = threadIdx.x; b < n; b += kBlock) out[q] += gbl(part)[(size_t)q * stride + b];
+    }
+    wave_sum<NV>(out);
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int q = 0; q < NV; q++) red[q][threadIdx.x >> 6] = out[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        out[q] = 0.0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; k++) out[q] += red[q][k];
+    }
+}
+
+// vsc: bb 0-1, rz of even iterations 2-3 and of odd ones 4-5, done 12-13,
+// iterations 14-15 (system 0 U, 1 V).
+constexpr int kViscTile = 16;
+__device__ __forceinline__ int visc_tiles_j(const SceneDev& s) { return (s.J + kViscTile - 1) / kViscTile; }
+__device__ __forceinline__ int visc_tiles(const SceneDev& s) { return ((s.I + kViscTile - 1) / kViscTile) * visc_tiles_j(s); }
+// The direction of system q at iteration it.  The second buffers are arrays
+// that the pressure solves before and after the viscosity solve leave free
+// (b; the residuals cr and cr2, one after the other: 8 bytes a cell), the
+// partials of p.q those of its z and direction (8 bytes a cell).
+__device__ __forceinline__ gptr<double> visc_p(const SceneDev& s, int q, int it)
+{
+    if ((it & 1) == 0) return gbl(s.vp + (size_t)q * s.I * s.J);
+    return gbl(q == 0 ? s.b : reinterpret_cast<double*>(s.cr));
+}
+__device__ __forceinline__ double* visc_pq(const SceneDev& s) { return reinterpret_cast<double*>(s.cu); }
 
 __global__ void __launch_bounds__(kBlock) k_visc_setup(const SceneDev* scenes)
 {
@@ -111,126 +161,127 @@ __global__ void __launch_bounds__(kBlock) k_visc_setup(const SceneDev* scenes)
         s.vr[c] = bu;
         s.vr[C + c] = bv;
         const double zu = bu / d, zv = bv / d;
-        s.vp[c] = zu;
-        s.vp[C + c] = zv;
         bbu = bu * bu;
         bbv = bv * bv;
         rzu = bu * zu;
         rzv = bv * zv;
     }
-    visc_put(s, bbu, bbv, rzu, rzv);
+    double v[4] = {bbu, bbv, rzu, rzv};
+    visc_put<4>(s.vpart, visc_blocks(s), v);
 }
 
-__global__ void __launch_bounds__(kBlock) k_visc_spmv(const SceneDev* scenes)
+__global__ void __launch_bounds__(kBlock) k_visc_p(const SceneDev* scenes, int it, double tol2)
 {
+    constexpr int R = kViscTile + 2, Q = (R * R + kBlock - 1) / kBlock;
+    static_assert(kViscTile * kViscTile == kBlock, "one cell of the tile per thread");
+    __shared__ double ps[2][R][R + 1];
     const SceneDev& s = scenes[blockIdx.y];
-    if (!s.active || !s.visc_on || (int)blockIdx.x >= visc_blocks(s)) return;
+    if (!s.active || !s.visc_on || (int)blockIdx.x >= visc_tiles(s)) return;
     const int I = s.I, J = s.J, C = I * J;
-    const int c = blockIdx.x * kBlock + threadIdx.x;
+    const int tj = visc_tiles_j(s), i0 = kViscTile * (int)(blockIdx.x / tj), j0 = kViscTile * (int)(blockIdx.x % tj);
+    // loads first (clamped; positions outside the grid are not used)
+    double dq[Q], rq[2][Q], oq[2][Q];
+#pragma unroll
+    for (int u = 0; u < Q; u++) {
+        const int k = min((int)threadIdx.x + u * kBlock, R * R - 1);
+        const int c = min(max(i0 - 1 + k / R, 0), I - 1) * J + min(max(j0 - 1 + k % R, 0), J - 1);
+        dq[u] = gbl(s.vd)[c];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            rq[q][u] = gbl(s.vr)[(size_t)q * C + c];
+            oq[q][u] = it > 0 ? visc_p(s, q, it - 1)[c] : 0.0;
+        }
+    }
+    const int a = 1 + threadIdx.x / kViscTile, b = 1 + threadIdx.x % kViscTile, i = i0 + a - 1, j = j0 + b - 1;
+    const bool in = i < I && j < J;
+    const int c = min(i, I - 1) * J + min(j, J - 1);
+    const double e = gbl(s.ve)[c], n = gbl(s.vn)[c], ew = gbl(s.ve)[max(c - J, 0)], ns = gbl(s.vn)[max(c - 1, 0)];
+    // the sums of k_visc_setup (bb, rz) or of the iteration before (rr, rz)
+    double sum[4];
+    visc_sum<4>(s.vpart, visc_blocks(s), visc_blocks(s), sum);
+    double* const v = s.vsc;
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    bool go[2];
+    double beta[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        // a block that sees the lead's flag of this very launch stops as its own sums would have it
+        const bool done = it > 0 && gbl(v)[12 + q] != 0.0;
+        const bool stop = it == 0 ? sum[q] == 0.0 : sum[q] < tol2 * gbl(v)[q];   // a zero right-hand side: x = 0
+        go[q] = !done && !stop;
+        beta[q] = it == 0 ? 0.0 : sum[2 + q] / gbl(v)[2 + 2 * ((it - 1) & 1) + q];
+        if (lead && !done) {
+            if (it == 0) v[q] = sum[q];
+            v[2 + 2 * (it & 1) + q] = sum[2 + q];
+            v[12 + q] = stop ? 1.0 : 0.0;
+            v[14 + q] = it == 0 ? 0.0 : gbl(v)[14 + q] + 1.0;
+        }
+    }
+    if (!go[0] && !go[1]) return;
+#pragma unroll
+    for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int u = 0; u < Q; u++) {
+            const int k = threadIdx.x + u * kBlock;
+            if (k < R * R) ps[q][k / R][k % R] = it == 0 ? rq[q][u] / dq[u] : rq[q][u] / dq[u] + beta[q] * oq[q][u];
+        }
+    __syncthreads();
+    const double d = gbl(s.vd)[c];
     double pq[2] = {0.0, 0.0};
-    if (c < C) {
-        const int i = c / J, j = c - (c / J) * J;
-        const double d = s.vd[c];
-        const double e = s.ve[c], n = s.vn[c];
-        const double ew = i > 0 ? s.ve[c - J] : 0.0, ns = j > 0 ? s.vn[c - 1] : 0.0;
+    if (in) {
 #pragma unroll
         for (int q = 0; q < 2; q++) {
-            const double* p = s.vp + (size_t)q * C;
-            double v = d * p[c];
-            if (i + 1 < I) v += e * p[c + J];
-            if (i > 0) v += ew * p[c - J];
-            if (j + 1 < J) v += n * p[c + 1];
-            if (j > 0) v += ns * p[c - 1];
-            s.vq[(size_t)q * C + c] = v;
-            pq[q] = p[c] * v;
+            if (!go[q]) continue;
+            const double p = ps[q][a][b];
+            double t = d * p;
+            if (i + 1 < I) t += e * ps[q][a + 1][b];
+            if (i > 0) t += ew * ps[q][a - 1][b];
+            if (j + 1 < J) t += n * ps[q][a][b + 1];
+            if (j > 0) t += ns * ps[q][a][b - 1];
+            visc_p(s, q, it)[c] = p;
+            gbl(s.vq)[(size_t)q * C + c] = t;
+            pq[q] = p * t;
         }
     }
-    visc_put(s, pq[0], pq[1], 0.0, 0.0);
+    visc_put<2>(visc_pq(s), visc_tiles(s), pq);
 }
 
-__global__ void __launch_bounds__(kBlock) k_visc_update(const SceneDev* scenes)
+__global__ void __launch_bounds__(kBlock) k_visc_x(const SceneDev* scenes, int it)
 {
     const SceneDev& s = scenes[blockIdx.y];
     if (!s.active || !s.visc_on || (int)blockIdx.x >= visc_blocks(s)) return;
     const int C = s.I * s.J;
-    const int c = blockIdx.x * kBlock + threadIdx.x;
-    double rr[2] = {0.0, 0.0}, rz[2] = {0.0, 0.0};
+    const int c = blockIdx.x * kBlock + threadIdx.x, cc = min(c, C - 1);
+    const double d = gbl(s.vd)[cc];
+    double p[2], x[2], r[2], t[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const size_t k = (size_t)q * C + cc;
+        p[q] = visc_p(s, q, it)[cc];
+        x[q] = gbl(s.vx)[k];
+        r[q] = gbl(s.vr)[k];
+        t[q] = gbl(s.vq)[k];
+    }
+    cptr<double> v = cst(s.vsc);   // k_visc_p's
+    const bool go[2] = {v[12] == 0.0, v[13] == 0.0};
+    if (!go[0] && !go[1]) return;
+    double pq[2];
+    visc_sum<2>(visc_pq(s), visc_tiles(s), visc_tiles(s), pq);
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};   // rr, rz
     if (c < C) {
-        const double d = s.vd[c];
 #pragma unroll
         for (int q = 0; q < 2; q++) {
-            const double alpha = cst(s.vsc)[8 + q];
+            if (!go[q]) continue;
+            const double alpha = v[2 + 2 * (it & 1) + q] / pq[q];
             const size_t k = (size_t)q * C + c;
-            const double p = s.vp[k];
-            s.vx[k] += alpha * p;
-            const double r = s.vr[k] - alpha * s.vq[k];
-            s.vr[k] = r;
-            rr[q] = r * r;
-            rz[q] = r * (r / d);
+            gbl(s.vx)[k] = x[q] + alpha * p[q];
+            const double rn = r[q] - alpha * t[q];
+            gbl(s.vr)[k] = rn;
+            sum[q] = rn * rn;
+            sum[2 + q] = rn * (rn / d);
         }
     }
-    visc_put(s, rr[0], rr[1], rz[0], rz[1]);
-}
-
-__global__ void __launch_bounds__(kBlock) k_visc_dir(const SceneDev* scenes)
-{
-    const SceneDev& s = scenes[blockIdx.y];
-    if (!s.active || !s.visc_on || (int)blockIdx.x >= visc_blocks(s)) return;
-    const int C = s.I * s.J;
-    const int c = blockIdx.x * kBlock + threadIdx.x;
-    if (c >= C) return;
-    const double d = s.vd[c];
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-        const double beta = cst(s.vsc)[10 + q];
-        const size_t k = (size_t)q * C + c;
-        s.vp[k] = s.vr[k] / d + beta * s.vp[k];
-    }
-}
-
-// what 0: after k_visc_setup; 1: after k_visc_spmv (alpha); 2: after
-// k_visc_update (the stop test, beta).  vsc: bb 0-1, rz 2-3, pq 4-5, rr 6-7,
-// alpha 8-9, beta 10-11, done 12-13, iterations 14-15.
-__global__ void __launch_bounds__(kBlock) k_visc_red(const SceneDev* scenes, int what, double tol2)
-{
-    const SceneDev& s = scenes[blockIdx.y];
-    if (!s.active || !s.visc_on) return;
-    __shared__ double red[kBlock / 64];
-    const int cb = visc_blocks(s);
-    const int nslot = what == 1 ? 2 : 4;
-    double sum[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int q = 0; q < nslot; q++) {
-        double acc = 0.0;
-        for (int b = threadIdx.x; b < cb; b += kBlock) acc += s.vpart[(size_t)q * cb + b];
-        sum[q] = block_sum(acc, red);
-    }
-    if (threadIdx.x != 0) return;
-    double* v = s.vsc;
-    for (int q = 0; q < 2; q++) {
-        if (what == 0) {
-            v[q] = sum[q];
-            v[2 + q] = sum[2 + q];
-            v[6 + q] = sum[q];
-            v[12 + q] = sum[q] == 0.0 ? 1.0 : 0.0;   // a zero right-hand side: x = 0
-            v[14 + q] = 0.0;
-            v[8 + q] = 0.0;
-            v[10 + q] = 0.0;
-        } else if (what == 1) {
-            v[4 + q] = sum[q];
-            v[8 + q] = v[12 + q] != 0.0 ? 0.0 : v[2 + q] / sum[q];
-        } else {
-            v[10 + q] = 0.0;
-            if (v[12 + q] != 0.0) continue;
-            v[6 + q] = sum[q];
-            v[14 + q] += 1.0;
-            if (sum[q] < tol2 * v[q]) {
-                v[12 + q] = 1.0;
-            } else {
-                v[10 + q] = sum[2 + q] / v[2 + q];
-                v[2 + q] = sum[2 + q];
-            }
-        }
-    }
+    visc_put<4>(s.vpart, visc_blocks(s), sum);
 }
 
 __global__ void __launch_bounds__(kBlock) k_visc_apply(const SceneDev* scenes)
@@ -241,6 +292,10 @@ __global__ void __launch_bounds__(kBlock) k_visc_apply(const SceneDev* scenes)
     const int c = blockIdx.x * kBlock + threadIdx.x;
     if (c >= C) return;
     const int i = c / J, j = c - (c / J) * J;
+    if (c == 0) {
+        s.sc->visc_iters = (int32_t)fmax(s.vsc[14], s.vsc[15]);
+        s.sc->visc_done = s.vsc[12] != 0.0 && s.vsc[13] != 0.0;
+    }
     const float rho = (float)s.rho;
     s.u[(size_t)i * J + j] = (float)(s.vx[c] / rho);          // applyResult
     s.v[(size_t)i * (J + 1) + j] = (float)(s.vx[C + c] / rho);
@@ -265,14 +320,12 @@ namespace fg {
     void launch_##name(dim3 g, hipStream_t st, const SceneDev* sc) { fg_launch(k_##name, g, dim3(kBlock), st, sc); }
 FG_VLAUNCH(visc_grid)
 FG_VLAUNCH(visc_setup)
-FG_VLAUNCH(visc_spmv)
-FG_VLAUNCH(visc_update)
-FG_VLAUNCH(visc_dir)
 FG_VLAUNCH(visc_apply)
-void launch_visc_red(dim3 g, hipStream_t st, const SceneDev* sc, int what, double tol2)
+void launch_visc_p(dim3 g, hipStream_t st, const SceneDev* sc, int it, double tol2)
 {
-    fg_launch(k_visc_red, g, dim3(kBlock), st, sc, what, tol2);
+    fg_launch(k_visc_p, g, dim3(kBlock), st, sc, it, tol2);
 }
+void launch_visc_x(dim3 g, hipStream_t st, const SceneDev* sc, int it) { fg_launch(k_visc_x, g, dim3(kBlock), st, sc, it); }
 void launch_visc_flags(hipStream_t st, const SceneDev* sc, int n, int32_t* out)
 {
     hipLaunchKernelGGL(k_visc_flags, dim3(1), dim3(64), 0, st, sc, n, out);
