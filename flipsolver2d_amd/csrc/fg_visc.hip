@@ -45,17 +45,42 @@ __global__ void __launch_bounds__(kBlock) k_visc_grid(const SceneDev* scenes)
     float wt = 1e-10f, vv = 0.0f;
     bool known = false;
     const int j0 = max(0, j - 2), j1 = min(J - 1, j + 1);
-    for (int a = max(0, i - 2); a <= min(I - 1, i + 1); a++) {
-        const int k0 = s.cellStart[a * J + j0], k1 = s.cellStart[a * J + j1 + 1];
-        for (int k = k0; k < k1; k++) {
-            const float2 p = ldg2(s.pos, k);
-            const float w = qbspline(p.x - (float)i, p.y - (float)j);
-            // NBFlipSolver's own (nbflipsolver.cpp:441-504): |w| > 1e-6, and
-            // the sum divided only where some weight counted
-            if (s.nb ? fabsf(w) > 1e-6f : w > 1e-9f) {
-                wt += w;
-                vv += w * s.pvisc[k];
-                known = true;
+    // the four rows' bounds at once, then kVgItems particles a step whose
+    // loads issue together (clamped; summed in order): with a load, its test
+    // and the next particle in turn the loop ran at a load's latency a
+    // particle, 95 us at eight 256^2 scenes; this 56
+    constexpr int kVgItems = 4;
+    int kb[4], ke[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int a = i - 2 + q;
+        const bool row = a >= 0 && a < I;
+        const int ac = min(max(a, 0), I - 1);
+        kb[q] = gbl(s.cellStart)[ac * J + j0];
+        ke[q] = row ? gbl(s.cellStart)[ac * J + j1 + 1] : kb[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        for (int k = kb[q]; k < ke[q]; k += kVgItems) {
+            float2 p[kVgItems];
+            float nu[kVgItems];
+#pragma unroll
+            for (int u = 0; u < kVgItems; u++) {
+                const int ku = min(k + u, ke[q] - 1);
+                p[u] = ldg2(s.pos, ku);
+                nu[u] = gbl(s.pvisc)[ku];
+            }
+#pragma unroll
+            for (int u = 0; u < kVgItems; u++) {
+                if (k + u >= ke[q]) continue;
+                const float w = qbspline(p[u].x - (float)i, p[u].y - (float)j);
+                // NBFlipSolver's own (nbflipsolver.cpp:441-504): |w| > 1e-6, and
+                // the sum divided only where some weight counted
+                if (s.nb ? fabsf(w) > 1e-6f : w > 1e-9f) {
+                    wt += w;
+                    vv += w * nu[u];
+                    known = true;
+                }
             }
         }
     }
