@@ -569,6 +569,12 @@ __device__ bool bfs_band(int tile, const float* gin, const uint8_t* vin, const i
         }
         if (g * NW + NW == H) last = f;
         const int st = g * NW + (w ? w : NW);
+        // a level-st cell d cells outside the tile reaches the tile's cells of
+        // level st + d and up alone: past st + d = H it is not listed.  What a
+        // listed cell reads is listed: one level less, one cell further out.
+        // Velocities of the 1024^2 dam break (half its tiles work): 58.5 us a
+        // launch with the whole halo, 52.4 so; the level set's bands 15.6, 15.1.
+        m &= (lane >= st && lane < R - st) ? (~0ull >> (64 - (R - 2 * st))) << st : 0ull;
         if (!__any(m != 0)) {
             if (!__any(f != 0)) break;
             continue;
