@@ -275,6 +275,8 @@ __global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, cons
     const SceneDev& s = scenes[sb.scene];
     cptr<SceneScalars> scr = cst(s.sc);
     if (!s.active | (s.precond != kPrecondMG) | (sb.block >= s.up_blocks)) return;
+    // of several scenes some have stopped (see k_mg_rr): their loads are not issued
+    if (map && ((scr->outer_done != 0) | (scr->inner_done != 0))) return;
     const int I = s.I, J = s.J, C = I * J;
     const bool first = it == 0;
     gptr<const float> z = gbl<const float>(s.cu);
