@@ -92,16 +92,16 @@ SOLVE_FAMILIES = ["pcg_a", "pcg_b", "mg_down0", "mg_up0", "mg_resid", "mg_pp", "
 # algorithmic bytes over the same launches (profiles/hbm_traffic.md; on a
 # 1 GiB copy kernel the same counters read 1.000 GiB each way).
 MEASURED_TRAFFIC_PER_UNIT = {
-    "mixed256": {"p2g": 1.367, "particles": 0.655, "sdf": 2.114, "pcg_a": 1.089, "pcg_b": 1.012,
-                 "mg_down0": 1.063, "mg_up0": 0.948, "mg_resid": 1.306, "mg_pp": 1.143, "mg_coarse": 1.243},
-    "dam1024": {"p2g": 1.107, "particles": 2.041, "sdf": 0.63, "pcg_a": 1.022, "pcg_b": 1.003,
-                "mg_down0": 1.029, "mg_up0": 0.939, "mg_resid": 1.21, "mg_pp": 1.113, "mg_coarse": 1.513},
-    "nb1024": {"p2g": 1.3, "particles": 0.261, "sdf": 2.155, "pcg_a": 1.022, "pcg_b": 1.003, "mg_down0": 1.018,
-               "mg_up0": 0.939, "mg_resid": 1.211, "mg_pp": 1.114, "mg_coarse": 1.516, "nb_euler": 1.646},
-    "visc256": {"p2g": 1.224, "particles": 1.704, "sdf": 1.285, "pcg_a": 1.054, "pcg_b": 1.005, "mg_down0": 1.024,
-                "mg_up0": 0.937, "mg_resid": 1.203, "mg_pp": 1.093, "mg_coarse": 1.311, "visc_cg": 1.193},
-    "proj4096": {"pcg_a": 1.863, "pcg_b": 1.0, "mg_down0": 1.006, "mg_up0": 1.983, "mg_resid": 1.259,
-                 "mg_pp": 1.222, "mg_coarse": 1.386},
+    "mixed256": {"p2g": 1.367, "particles": 0.659, "sdf": 2.115, "pcg_a": 1.075, "mg_down0": 1.017, "mg_up0": 1.041,
+                 "mg_resid": 1.369, "mg_pp": 1.139, "mg_coarse": 1.211},
+    "dam1024": {"p2g": 1.107, "particles": 2.041, "sdf": 0.629, "pcg_a": 1.064, "mg_down0": 1.009, "mg_up0": 1.017,
+                "mg_resid": 1.353, "mg_pp": 1.19, "mg_coarse": 1.318},
+    "nb1024": {"p2g": 1.296, "particles": 0.261, "sdf": 2.155, "pcg_a": 1.093, "mg_down0": 1.009, "mg_up0": 1.017,
+               "mg_resid": 1.404, "mg_pp": 1.228, "mg_coarse": 1.321, "nb_euler": 1.646},
+    "visc256": {"p2g": 1.223, "particles": 1.704, "sdf": 1.264, "pcg_a": 1.054, "mg_down0": 1.006, "mg_up0": 1.019,
+                "mg_resid": 1.236, "mg_pp": 1.093, "mg_coarse": 1.228, "visc_cg": 1.339},
+    "proj4096": {"pcg_a": 1.637, "mg_down0": 1.007, "mg_up0": 1.152, "mg_resid": 1.396, "mg_pp": 1.372,
+                 "mg_coarse": 1.309},
 }
 
 
