@@ -1325,6 +1325,11 @@ struct KProf {
 // scenes of the group run the same sweep and iteration index in lock step;
 // a scene whose solve has stopped skips the launches that remain.
 // ---------------------------------------------------------------------------
+// Whether some scene of S uses the V-cycle.  In a group that has such scenes
+// the ones that go on iterating may all use the IPP (a side over 32,768 cells):
+// the V-cycle kernels then have no block, and an empty grid is an error.
+bool any_vcycle(const SolveLaunch& S) { return S.blocks[kUpKind] > 0; }
+
 // One V-cycle z = M r over the scenes of S whose solve uses it; it < 0: of
 // the residual that starts a sweep (cr), else of iteration it's, whose step
 // its first launch takes.  Level-l launches cover the scenes that have level
@@ -1336,7 +1341,7 @@ void launch_vcycle(const Group& G, hipStream_t st, const SolveLaunch& S, int it)
     // (t per scene; the maps and grids hold a level's blocks only for the
     // scenes that launch it)
     const int top = G.mg_top;
-    if (S.blocks[1]) {
+    {
         KProf kp(G, FG_K_MG_DOWN0, true);
         if (it < 0) launch_mg_down0(S.grid(1), st, S.d, S.map[1], 0);
         else launch_mg_step0(S.grid(1), st, S.d, S.map[1], it);
@@ -1391,7 +1396,7 @@ void launch_vcycle(const Group& G, hipStream_t st, const SolveLaunch& S, int it)
 // kernel; the others: the V-cycle, whose first launch makes r and x).
 void launch_iteration(const Group& G, hipStream_t st, const SolveLaunch& S, int it)
 {
-    if (G.mg_levels) {
+    if (any_vcycle(S)) {
         KProf kp(G, FG_K_PCG_A, true);
         launch_pcg_dir(S.grid(kUpKind), st, S.d, S.map[kUpKind], it);
         kp.done(0);   // units: at the end of the solve
@@ -1406,7 +1411,7 @@ void launch_iteration(const Group& G, hipStream_t st, const SolveLaunch& S, int 
         launch_pcg_b(S.grid(0), st, S.d, S.map[0], it);
         kp.done(0);
     }
-    if (G.mg_levels) {
+    if (any_vcycle(S)) {
         KProf kp(G, FG_K_VCYCLE);
         launch_vcycle(G, st, S, it);
         kp.done(0);
@@ -1494,7 +1499,7 @@ int run_solve(Group& G, bool rhs_from_grid)
             S = group_launch(G, G.d, 1);
         }
         if (count == 0) break;
-        if (G.mg_levels) {
+        if (any_vcycle(S)) {
             KProf kp(G, FG_K_VCYCLE);
             launch_vcycle(G, st, S, -1);
             kp.done(0);

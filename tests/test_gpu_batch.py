@@ -142,3 +142,38 @@ def test_tiling_autotune_sets_the_fastest_and_keeps_batch_equal_to_solo(fg, ctx)
             sc.close()
     with pytest.raises(fg.FgError):
         fg.batch_autotune_tiling(ctx, [], rounds=1)
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_batch_of_both_preconditioners_equals_solo(fg, ctx, fused):
+    """4 x 70000 has too many levels for the V-cycle and solves with the IPP; the ordinary scenes beside it stop first,
+    so the solve's launches go on with no block of a V-cycle kernel."""
+    def scenes():
+        out = []
+        for n in (64, 33):
+            walls, fluids = fg.dam_break_geometry(n)
+            out.append(fg.Scene(ctx, fg.make_params(n, ppc=4)))
+            out[-1].init_geometry(walls, fluids, friction=np.zeros(len(walls), np.float32), seed=n)
+        dx, J = 1.0 / 64, 70000
+        walls = [fg.box(0, dx, 0, J * dx), fg.box(3 * dx, 4 * dx, 0, J * dx), fg.box(0, 4 * dx, 0, dx)]
+        out.insert(1, fg.Scene(ctx, fg.make_params(4, J, dx=dx, ppc=4, max_particles=20000, gravity=(2.0, 9.0))))
+        out[1].init_geometry(walls, [fg.box(dx, 3 * dx, 20 * dx, 420 * dx)], friction=np.zeros(3, np.float32), seed=5)
+        return out
+
+    solo, batch = scenes(), scenes()
+    try:
+        ctx.set_vcycle_fused(fused)
+        for f in range(2):
+            want = [sc.step_frame() for sc in solo]
+            got = fg.batch_step_frame(ctx, batch)
+            _log(f"frame {f}: pressure iterations {[s.pressure_iters for s in got]}")
+            assert want[1].pressure_iters > max(want[0].pressure_iters, want[2].pressure_iters)   # the IPP scene ends alone
+            for k in range(3):
+                assert (want[k].substeps, want[k].pressure_iters) == (got[k].substeps, got[k].pressure_iters), (f, k)
+                assert got[k].converged == 1
+        for k in range(3):
+            _same(solo[k].get_state(), batch[k].get_state(), k)
+    finally:
+        ctx.set_vcycle_fused(True)
+        for sc in solo + batch:
+            sc.close()
