@@ -2176,7 +2176,12 @@ int step_frames_split(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const s
             st.push_back(stats[k]);
         }
         rc[li] = step_frames_lane(ctx, ctx->lanes[li], sc, st, t0);
-        if (rc[li] != FG_OK) msg[li] = g_err;
+        if (rc[li] != FG_OK) {
+            msg[li] = g_err;
+            // a call that fails leaves nothing queued: a scene that is destroyed
+            // next hands its memory on (fg_scene_destroy waits for lane 0 alone)
+            hipStreamSynchronize(ctx->lanes[li]->stream);
+        }
     };
     std::vector<std::thread> workers;
     for (size_t li = 1; li < plan.size(); li++) workers.emplace_back(run, li);
@@ -2698,7 +2703,7 @@ int fg_scene_destroy(fg_scene* s)
 {
     if (!s) return FG_OK;
     fg_ctx* ctx = s->ctx;
-    hipStreamSynchronize(ctx->stream);   // the other lanes' work ended with the calls that queued it
+    hipStreamSynchronize(ctx->stream);   // the other lanes' work ends with the calls that queue it (step_frames_split)
     ctx->used -= s->bytes;
     SceneMem m;
     m.arena = s->arena;
