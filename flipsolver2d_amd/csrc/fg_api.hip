@@ -555,13 +555,16 @@ void trim_pool(fg_ctx* ctx, uint64_t bytes, size_t blocks = kPoolBlocks)
 }
 
 // Memory for a scene of `need` bytes: the pooled block that fits best, if it
-// is at most a quarter (or 16 MiB) too large, else a new one.
+// is at most a quarter (or 16 MiB) too large, else a new one.  Under a budget,
+// which admits scenes by the bytes they need, a block must be of just that
+// size: what scenes hold then never passes what was admitted.
 hipError_t take_block(fg_ctx* ctx, uint64_t need, SceneMem* out)
 {
+    const uint64_t slack = ctx->budget ? 0 : std::max<uint64_t>(need / 4, 16ull << 20);
     size_t best = ctx->pool.size();
     for (size_t k = 0; k < ctx->pool.size(); k++) {
         const uint64_t b = ctx->pool[k].bytes;
-        if (b >= need && b <= need + std::max<uint64_t>(need / 4, 16ull << 20) &&
+        if (b >= need && b <= need + slack &&
             (best == ctx->pool.size() || b < ctx->pool[best].bytes))
             best = k;
     }
@@ -629,7 +632,7 @@ int create_scene(fg_ctx* ctx, const fg_scene_params* p, bool solver_only, fg_sce
     s->d = m.d;
     s->hpin = m.hpin;
     s->hsc = m.hsc;
-    ctx->used += s->bytes;
+    ctx->used += s->block_bytes;
     const int rc = setup_scene_memory(s);
     if (rc != FG_OK) {
         fg_scene_destroy(s);
@@ -2704,7 +2707,7 @@ int fg_scene_destroy(fg_scene* s)
     if (!s) return FG_OK;
     fg_ctx* ctx = s->ctx;
     hipStreamSynchronize(ctx->stream);   // the other lanes' work ends with the calls that queue it (step_frames_split)
-    ctx->used -= s->bytes;
+    ctx->used -= s->block_bytes;
     SceneMem m;
     m.arena = s->arena;
     m.bytes = s->block_bytes;

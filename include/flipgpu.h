@@ -201,6 +201,9 @@ int32_t fg_abi_version(void);
 
 int fg_ctx_create(int32_t device, uint64_t hbm_budget_bytes, fg_ctx** out);
 int fg_ctx_destroy(fg_ctx* ctx);
+/* Device memory that the context's live scenes hold (their fg_scene_bytes; a
+ * context without a budget may give a scene a larger block of its pool, which
+ * counts whole).  The pool itself (see fg_scene_destroy) is not in it. */
 int fg_ctx_bytes_in_use(fg_ctx* ctx, uint64_t* out);
 /* Per-stage HIP-event timing for later calls (adds synchronisation). */
 int fg_ctx_set_timing(fg_ctx* ctx, int32_t enabled);

@@ -2,6 +2,7 @@
 counts where.  Each scenario runs in a process of its own, with the stand-in's symbols ahead of the runtime's."""
 import ctypes as C
 import os
+import random
 import subprocess
 import sys
 
@@ -40,7 +41,40 @@ def failed_launch_leaves_no_lane_busy(fg, stub):
     assert failures > 10
 
 
-SCENARIOS = [failed_launch_leaves_no_lane_busy]
+def _need(fg, params):
+    n = C.c_uint64()
+    fg._check(fg.lib().fg_scene_bytes(C.byref(params), C.byref(n)))
+    return n.value
+
+
+def pool_keeps_the_budget(fg, stub):
+    """Scenes made and destroyed in turn, their sizes close enough that one could live in another's memory: the device
+    memory stays within the budget, and what fits the budget is not refused."""
+    rng = random.Random(5)
+    sizes = {n: _need(fg, fg.make_params(n, ppc=4)) for n in (32, 40, 48, 56, 60, 62, 64)}
+    budget = 5 * sizes[64]
+    with fg.Context(0, hbm_budget=budget) as ctx:
+        base, live, refused = stub.stub_device_bytes(), [], 0
+        for step in range(600):
+            n = rng.choice(list(sizes))
+            if rng.random() < 0.45 and live:
+                live.pop(rng.randrange(len(live)))[0].close()
+            else:
+                held = sum(b for _, b in live)
+                try:
+                    live.append((fg.Scene(ctx, fg.make_params(n, ppc=4)), sizes[n]))
+                except fg.FgError as e:
+                    assert e.code == fg.E_BUDGET and held + sizes[n] > budget, (step, held, sizes[n])
+                    refused += 1
+            assert ctx.bytes_in_use() == sum(b for _, b in live), step
+            # the arenas; a descriptor of a few KB a block lies beside each
+            assert stub.stub_device_bytes() - base <= budget + 64 * 4096, (step, stub.stub_device_bytes() - base, budget)
+        assert refused > 20
+        for sc, _ in live:
+            sc.close()
+
+
+SCENARIOS = [failed_launch_leaves_no_lane_busy, pool_keeps_the_budget]
 
 
 @pytest.fixture(scope="module")
