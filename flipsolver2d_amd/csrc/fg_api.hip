@@ -25,6 +25,9 @@ using namespace fg;
 
 namespace fg {
 LaunchEvents& next_launch_events();
+// fg_serve.cpp: what a server's budget leaves for the memory of destroyed scenes
+void set_pool_room(fg_ctx* ctx, const void* owner, uint64_t bytes);
+void drop_pool_room(fg_ctx* ctx, const void* owner);
 }
 
 namespace {
@@ -101,9 +104,10 @@ struct Lane {
 // destroyed scene's goes to its context's pool and serves the next one that
 // fits, since allocating and freeing it costs 0.3 + 0.5 ms (and a device
 // synchronisation) whatever its size -- ten times a 64^2 substep.  The pool
-// holds at most kPoolBytes and kPoolBlocks, leaves room for live scenes under
-// the context's budget, gives everything back when an allocation fails and
-// when the context goes, and is the context's alone (one host thread).
+// holds at most kPoolBytes and kPoolBlocks and what the context's budget and
+// its servers' budgets leave beside their scenes, gives everything back when
+// an allocation fails and when the context goes, and is the context's alone
+// (one host thread).
 struct SceneMem {
     void* arena = nullptr;
     uint64_t bytes = 0;
@@ -138,6 +142,7 @@ struct fg_ctx {
     int64_t* totals = nullptr;      // pinned: counts the device reports
     std::vector<SceneMem> pool;   // memory of destroyed scenes, oldest first
     uint64_t pooled = 0;
+    std::vector<std::pair<const void*, uint64_t>> rooms;   // by server: what its budget leaves
 };
 
 struct fg_scene {
@@ -535,6 +540,10 @@ int setup_scene_memory(fg_scene* s)
     return FG_OK;
 }
 
+// The process's contexts (a server may outlive its own).
+std::mutex g_contexts_mu;
+std::vector<fg_ctx*> g_contexts;
+
 void free_block(const SceneMem& m)
 {
     if (m.arena) hipFree(m.arena);
@@ -554,13 +563,23 @@ void trim_pool(fg_ctx* ctx, uint64_t bytes, size_t blocks = kPoolBlocks)
     ctx->pool.erase(ctx->pool.begin(), ctx->pool.begin() + (ptrdiff_t)k);
 }
 
+// What the pool may hold while a scene of `need` more bytes is made.
+uint64_t pool_room(const fg_ctx* ctx, uint64_t need)
+{
+    uint64_t room = kPoolBytes;
+    if (ctx->budget) room = std::min(room, ctx->budget - std::min(ctx->budget, ctx->used + need));
+    for (const auto& r : ctx->rooms) room = std::min(room, r.second - std::min(r.second, need));
+    return room;
+}
+
 // Memory for a scene of `need` bytes: the pooled block that fits best, if it
-// is at most a quarter (or 16 MiB) too large, else a new one.  Under a budget,
-// which admits scenes by the bytes they need, a block must be of just that
-// size: what scenes hold then never passes what was admitted.
+// is at most a quarter (or 16 MiB) too large, else a new one.  Under a budget
+// (the context's or a server's), which admits scenes by the bytes they need, a
+// block must be of just that size: what scenes hold then never passes what was
+// admitted.
 hipError_t take_block(fg_ctx* ctx, uint64_t need, SceneMem* out)
 {
-    const uint64_t slack = ctx->budget ? 0 : std::max<uint64_t>(need / 4, 16ull << 20);
+    const uint64_t slack = ctx->budget || !ctx->rooms.empty() ? 0 : std::max<uint64_t>(need / 4, 16ull << 20);
     size_t best = ctx->pool.size();
     for (size_t k = 0; k < ctx->pool.size(); k++) {
         const uint64_t b = ctx->pool[k].bytes;
@@ -574,8 +593,7 @@ hipError_t take_block(fg_ctx* ctx, uint64_t need, SceneMem* out)
         ctx->pool.erase(ctx->pool.begin() + (ptrdiff_t)best);
         return hipSuccess;
     }
-    // under a budget the pool takes only what live scenes leave
-    if (ctx->budget) trim_pool(ctx, ctx->budget - std::min(ctx->budget, ctx->used + need));
+    trim_pool(ctx, pool_room(ctx, need));
     for (int attempt = 0;; attempt++) {
         SceneMem m;
         m.bytes = need;
@@ -602,9 +620,7 @@ void give_block(fg_ctx* ctx, const SceneMem& m)
     }
     ctx->pool.push_back(m);
     ctx->pooled += m.bytes;
-    uint64_t limit = kPoolBytes;
-    if (ctx->budget) limit = std::min(limit, ctx->budget - std::min(ctx->budget, ctx->used));
-    trim_pool(ctx, limit);
+    trim_pool(ctx, pool_room(ctx, 0));
 }
 
 int create_scene(fg_ctx* ctx, const fg_scene_params* p, bool solver_only, fg_scene** out)
@@ -2496,6 +2512,21 @@ int set_emitters(fg_scene* s, int32_t n, const float* velocity, const uint8_t* t
 fg::LaunchEvents& fg::next_launch_events() { return g_next_events; }
 int fg::report_error(int code, const std::string& msg) { return fail(code, msg); }
 
+void fg::set_pool_room(fg_ctx* ctx, const void* owner, uint64_t bytes)
+{
+    auto it = std::find_if(ctx->rooms.begin(), ctx->rooms.end(), [&](const auto& r) { return r.first == owner; });
+    if (it == ctx->rooms.end()) it = ctx->rooms.insert(it, {owner, 0});
+    it->second = bytes;
+    trim_pool(ctx, pool_room(ctx, 0));
+}
+void fg::drop_pool_room(fg_ctx* ctx, const void* owner)
+{
+    std::lock_guard<std::mutex> lock(g_contexts_mu);
+    if (std::find(g_contexts.begin(), g_contexts.end(), ctx) == g_contexts.end()) return;
+    auto& r = ctx->rooms;
+    r.erase(std::remove_if(r.begin(), r.end(), [&](const auto& e) { return e.first == owner; }), r.end());
+}
+
 // ============================================================================
 // C-ABI
 // ============================================================================
@@ -2528,6 +2559,10 @@ int fg_ctx_create(int32_t device, uint64_t hbm_budget_bytes, fg_ctx** out)
         fg_ctx_destroy(c);
         return fail(FG_E_DEVICE, std::string("hipHostMalloc: ") + hipGetErrorString(e));
     }
+    {
+        std::lock_guard<std::mutex> lock(g_contexts_mu);
+        g_contexts.push_back(c);
+    }
     *out = c;
     return FG_OK;
 }
@@ -2535,6 +2570,10 @@ int fg_ctx_create(int32_t device, uint64_t hbm_budget_bytes, fg_ctx** out)
 int fg_ctx_destroy(fg_ctx* ctx)
 {
     if (!ctx) return FG_OK;
+    {
+        std::lock_guard<std::mutex> lock(g_contexts_mu);
+        g_contexts.erase(std::remove(g_contexts.begin(), g_contexts.end(), ctx), g_contexts.end());
+    }
     for (Lane* L : ctx->lanes) lane_destroy(L);
     trim_pool(ctx, 0, 0);
     for (int k = 0; k < 2; k++) {

@@ -18,6 +18,9 @@
 
 namespace fg {
 int report_error(int code, const std::string& msg);
+// what a server's budget leaves for the memory that its context keeps of destroyed scenes
+void set_pool_room(fg_ctx* ctx, const void* owner, uint64_t bytes);
+void drop_pool_room(fg_ctx* ctx, const void* owner);
 }
 
 namespace {
@@ -76,12 +79,18 @@ struct fg_server {
 
 namespace {
 
+void count_bytes(fg_server* srv, int64_t bytes)
+{
+    srv->resident_bytes += bytes;
+    fg::set_pool_room(srv->ctx, srv, srv->budget - srv->resident_bytes);
+}
+
 void drop_scene(fg_server* srv, Req& r)
 {
     if (!r.scene) return;
+    count_bytes(srv, -(int64_t)r.bytes);
     fg_scene_destroy(r.scene);
     r.scene = nullptr;
-    srv->resident_bytes -= r.bytes;
 }
 
 // The head request cannot be admitted, for good: it leaves the queue as
@@ -138,7 +147,7 @@ int admit(fg_server* srv, int* admitted)
             continue;
         }
         r.scene = sc;
-        srv->resident_bytes += r.bytes;
+        count_bytes(srv, (int64_t)r.bytes);
         r.status.state = FG_REQ_RESIDENT;
         r.status.admit_ms = srv->now_ms();
         fg_scene_particle_count(sc, &r.status.particles);
@@ -163,6 +172,7 @@ int fg_server_create(fg_ctx* ctx, uint64_t hbm_budget_bytes, int32_t max_residen
     s->budget = hbm_budget_bytes;
     s->max_resident = max_resident;
     s->t0 = std::chrono::steady_clock::now();
+    count_bytes(s, 0);
     *out = s;
     return FG_OK;
 }
@@ -171,6 +181,7 @@ int fg_server_destroy(fg_server* srv)
 {
     if (!srv) return FG_OK;
     for (auto& kv : srv->reqs) drop_scene(srv, kv.second);
+    fg::drop_pool_room(srv->ctx, srv);
     delete srv;
     return FG_OK;
 }

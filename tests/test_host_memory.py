@@ -74,7 +74,36 @@ def pool_keeps_the_budget(fg, stub):
             sc.close()
 
 
-SCENARIOS = [failed_launch_leaves_no_lane_busy, pool_keeps_the_budget]
+def server_keeps_its_budget(fg, stub):
+    """A server's budget bounds the device memory of its scenes and of the memory kept from those that ended, on a context
+    that has no budget of its own and whose own scenes left memory in the pool."""
+    rng = random.Random(7)
+    walls, fluids = fg.dam_break_geometry(32)
+    with fg.Context(0) as ctx:
+        base = stub.stub_device_bytes()
+        for sc in [fg.Scene(ctx, fg.make_params(64, ppc=4)) for _ in range(12)]:
+            sc.close()
+        largest = _need(fg, fg.make_params(96, ppc=4))
+        with fg.Server(ctx, hbm_budget=3 * largest, max_resident=16) as srv:
+            kept, waits = [], 0
+            for tick in range(200):
+                for _ in range(rng.randint(0, 3)):
+                    n, keep = rng.choice((40, 56, 64, 72, 88, 90, 96)), rng.random() < 0.3
+                    p = fg.make_params(n, ppc=4)
+                    rid = srv.submit(p, walls, fluids, rng.randint(1, 4), keep=keep)
+                    if keep:
+                        kept.append(rid)
+                t = srv.tick()
+                waits += t.queued > 0
+                held = stub.stub_device_bytes() - base
+                # beside the scenes: the lane's descriptors and block maps
+                assert held <= 3 * largest + (1 << 20), (tick, held, 3 * largest)
+                if kept and rng.random() < 0.3 and srv.status(kept[0]).state == fg.REQ_DONE:
+                    srv.release(kept.pop(0))
+            assert waits > 20
+
+
+SCENARIOS = [failed_launch_leaves_no_lane_busy, pool_keeps_the_budget, server_keeps_its_budget]
 
 
 @pytest.fixture(scope="module")
