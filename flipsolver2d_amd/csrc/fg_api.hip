@@ -76,6 +76,7 @@ constexpr int kFlagWords = 4 + kMapKinds;
 // stepped by its own host thread, so the scenes of one lane overlap on the
 // device with those of the others.
 struct Lane {
+    int device = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
     int bcap = 0;
@@ -105,9 +106,9 @@ struct Lane {
 // fits, since allocating and freeing it costs 0.3 + 0.5 ms (and a device
 // synchronisation) whatever its size -- ten times a 64^2 substep.  The pool
 // holds at most kPoolBytes and kPoolBlocks and what the context's budget and
-// its servers' budgets leave beside their scenes, gives everything back when
-// an allocation fails and when the context goes, and is the context's alone
-// (one host thread).
+// its servers' budgets leave beside their scenes, and gives everything back
+// when a device allocation of this library fails (dev_alloc) and when the
+// context goes.
 struct SceneMem {
     void* arena = nullptr;
     uint64_t bytes = 0;
@@ -143,6 +144,7 @@ struct fg_ctx {
     std::vector<SceneMem> pool;   // memory of destroyed scenes, oldest first
     uint64_t pooled = 0;
     std::vector<std::pair<const void*, uint64_t>> rooms;   // by server: what its budget leaves
+    std::mutex pool_mu;           // of the three above: an allocation on any thread may empty the pool
 };
 
 struct fg_scene {
@@ -188,6 +190,57 @@ constexpr uint64_t kNoAllocScratchBytes = 48ull << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
+
+// The process's contexts (a server may outlive its own, and a context whose
+// allocation fails has the others give back what they pooled).
+std::mutex g_contexts_mu;
+std::vector<fg_ctx*> g_contexts;
+
+void free_block(const SceneMem& m)
+{
+    if (m.arena) hipFree(m.arena);
+    if (m.d) hipFree(m.d);
+    if (m.hpin) hipHostFree(m.hpin);
+    if (m.hsc) hipHostFree(m.hsc);
+}
+
+// Give back pooled memory, oldest first, until at most `bytes` are pooled
+// (pool_mu held).
+void trim_pool(fg_ctx* ctx, uint64_t bytes, size_t blocks = kPoolBlocks)
+{
+    size_t k = 0;
+    while (k < ctx->pool.size() && (ctx->pooled > bytes || ctx->pool.size() - k > blocks)) {
+        ctx->pooled -= ctx->pool[k].bytes;
+        free_block(ctx->pool[k++]);
+    }
+    ctx->pool.erase(ctx->pool.begin(), ctx->pool.begin() + (ptrdiff_t)k);
+}
+
+// Give back everything that the contexts of `device` have pooled (from any
+// host thread), after a failed allocation, whose error is answered here; false
+// if there was nothing.
+bool give_back_pools(int device)
+{
+    bool any = false;
+    std::lock_guard<std::mutex> lock(g_contexts_mu);
+    for (fg_ctx* c : g_contexts) {
+        if (c->device != device) continue;
+        std::lock_guard<std::mutex> pool(c->pool_mu);
+        any = any || !c->pool.empty();
+        trim_pool(c, 0, 0);
+    }
+    if (any) (void)hipGetLastError();
+    return any;
+}
+
+// Device memory beside scenes' own: where the device has none left, the pools
+// are given back and the allocation is tried again.
+template <typename T>
+hipError_t dev_alloc(int device, T** p, uint64_t bytes)
+{
+    const hipError_t e = hipMalloc(p, bytes);
+    return e != hipSuccess && give_back_pools(device) ? hipMalloc(p, bytes) : e;
+}
 
 constexpr int kNoAllocDevices = 64;
 // Per device: the scratch's device address, the host-side scene that lives
@@ -540,29 +593,6 @@ int setup_scene_memory(fg_scene* s)
     return FG_OK;
 }
 
-// The process's contexts (a server may outlive its own).
-std::mutex g_contexts_mu;
-std::vector<fg_ctx*> g_contexts;
-
-void free_block(const SceneMem& m)
-{
-    if (m.arena) hipFree(m.arena);
-    if (m.d) hipFree(m.d);
-    if (m.hpin) hipHostFree(m.hpin);
-    if (m.hsc) hipHostFree(m.hsc);
-}
-
-// Give back pooled memory, oldest first, until at most `bytes` are pooled.
-void trim_pool(fg_ctx* ctx, uint64_t bytes, size_t blocks = kPoolBlocks)
-{
-    size_t k = 0;
-    while (k < ctx->pool.size() && (ctx->pooled > bytes || ctx->pool.size() - k > blocks)) {
-        ctx->pooled -= ctx->pool[k].bytes;
-        free_block(ctx->pool[k++]);
-    }
-    ctx->pool.erase(ctx->pool.begin(), ctx->pool.begin() + (ptrdiff_t)k);
-}
-
 // What the pool may hold while a scene of `need` more bytes is made.
 uint64_t pool_room(const fg_ctx* ctx, uint64_t need)
 {
@@ -579,6 +609,7 @@ uint64_t pool_room(const fg_ctx* ctx, uint64_t need)
 // admitted.
 hipError_t take_block(fg_ctx* ctx, uint64_t need, SceneMem* out)
 {
+    std::unique_lock<std::mutex> lock(ctx->pool_mu);
     const uint64_t slack = ctx->budget || !ctx->rooms.empty() ? 0 : std::max<uint64_t>(need / 4, 16ull << 20);
     size_t best = ctx->pool.size();
     for (size_t k = 0; k < ctx->pool.size(); k++) {
@@ -594,6 +625,7 @@ hipError_t take_block(fg_ctx* ctx, uint64_t need, SceneMem* out)
         return hipSuccess;
     }
     trim_pool(ctx, pool_room(ctx, need));
+    lock.unlock();
     for (int attempt = 0;; attempt++) {
         SceneMem m;
         m.bytes = need;
@@ -606,9 +638,7 @@ hipError_t take_block(fg_ctx* ctx, uint64_t need, SceneMem* out)
             return e;
         }
         free_block(m);
-        if (attempt || ctx->pool.empty()) return e;
-        (void)hipGetLastError();   // the failed allocation's, answered here
-        trim_pool(ctx, 0, 0);
+        if (attempt || !give_back_pools(ctx->device)) return e;
     }
 }
 
@@ -618,6 +648,7 @@ void give_block(fg_ctx* ctx, const SceneMem& m)
         free_block(m);
         return;
     }
+    std::lock_guard<std::mutex> lock(ctx->pool_mu);
     ctx->pool.push_back(m);
     ctx->pooled += m.bytes;
     trim_pool(ctx, pool_room(ctx, 0));
@@ -962,9 +993,10 @@ void lane_destroy(Lane* L)
     delete L;
 }
 
-int lane_create(hipStream_t stream, Lane** out)
+int lane_create(int device, hipStream_t stream, Lane** out)
 {
     auto* L = new Lane();
+    L->device = device;
     hipError_t e = hipSuccess;
     if (stream) {
         L->stream = stream;
@@ -972,7 +1004,7 @@ int lane_create(hipStream_t stream, Lane** out)
         e = hipStreamCreateWithFlags(&L->stream, hipStreamNonBlocking);
         L->own_stream = e == hipSuccess;
     }
-    if (e == hipSuccess) e = hipMalloc(&L->bflags, sizeof(int32_t) * kFlagWords);
+    if (e == hipSuccess) e = dev_alloc(device, &L->bflags, sizeof(int32_t) * kFlagWords);
     if (e == hipSuccess) e = hipHostMalloc((void**)&L->bflags_host, sizeof(int32_t) * kFlagWords, hipHostMallocDefault);
     if (e != hipSuccess) {
         lane_destroy(L);
@@ -1013,12 +1045,12 @@ int ensure_group_buffers(Lane* L, int n)
     const int cap = std::max(n, 2 * L->bcap);
     HIPCHK(hipStreamSynchronize(L->stream));
     lane_free_buffers(L);
-    HIPCHK(hipMalloc(&L->bdesc, sizeof(SceneDev) * cap));
+    HIPCHK(dev_alloc(L->device, &L->bdesc, sizeof(SceneDev) * cap));
     HIPCHK(hipHostMalloc((void**)&L->bdesc_host, sizeof(SceneDev) * cap, hipHostMallocDefault));
-    HIPCHK(hipMalloc(&L->bsub, sizeof(SceneDev) * cap));
+    HIPCHK(dev_alloc(L->device, &L->bsub, sizeof(SceneDev) * cap));
     HIPCHK(hipHostMalloc((void**)&L->bsub_host, sizeof(SceneDev) * cap, hipHostMallocDefault));
-    HIPCHK(hipMalloc(&L->bpack, sizeof(SceneDev) * cap));
-    HIPCHK(hipMalloc(&L->bsc, sizeof(SceneScalars) * cap));
+    HIPCHK(dev_alloc(L->device, &L->bpack, sizeof(SceneDev) * cap));
+    HIPCHK(dev_alloc(L->device, &L->bsc, sizeof(SceneScalars) * cap));
     HIPCHK(hipHostMalloc((void**)&L->bsc_host, sizeof(SceneScalars) * cap, hipHostMallocDefault));
     L->bcap = cap;
     return FG_OK;
@@ -1098,7 +1130,7 @@ int make_group(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const std::vec
             if (L->bmap) hipFree(L->bmap);
             L->bmap = nullptr;
             L->bmap_cap = 0;
-            HIPCHK(hipMalloc(&L->bmap, sizeof(int2) * std::max<int64_t>(total, 1)));
+            HIPCHK(dev_alloc(L->device, &L->bmap, sizeof(int2) * std::max<int64_t>(total, 1)));
             L->bmap_cap = total;
         }
     }
@@ -2120,7 +2152,7 @@ int ensure_lanes(fg_ctx* ctx, int n)
 {
     while ((int)ctx->lanes.size() < n) {
         Lane* L = nullptr;
-        FGCHK(lane_create(nullptr, &L));
+        FGCHK(lane_create(ctx->device, nullptr, &L));
         ctx->lanes.push_back(L);
     }
     return FG_OK;
@@ -2459,7 +2491,7 @@ int upload_geometry(fg_scene* s, const fg_polygons* sets[4], const float* const 
         if (L->bgeo) hipFree(L->bgeo);
         L->bgeo = nullptr;
         L->bgeo_cap = 0;
-        HIPCHK(hipMalloc(&L->bgeo, std::max<size_t>(bytes, 64 << 10)));
+        HIPCHK(dev_alloc(L->device, &L->bgeo, std::max<size_t>(bytes, 64 << 10)));
         L->bgeo_cap = std::max<size_t>(bytes, 64 << 10);
     }
     char* const up = s->ctx->up;
@@ -2514,6 +2546,7 @@ int fg::report_error(int code, const std::string& msg) { return fail(code, msg);
 
 void fg::set_pool_room(fg_ctx* ctx, const void* owner, uint64_t bytes)
 {
+    std::lock_guard<std::mutex> lock(ctx->pool_mu);
     auto it = std::find_if(ctx->rooms.begin(), ctx->rooms.end(), [&](const auto& r) { return r.first == owner; });
     if (it == ctx->rooms.end()) it = ctx->rooms.insert(it, {owner, 0});
     it->second = bytes;
@@ -2523,6 +2556,7 @@ void fg::drop_pool_room(fg_ctx* ctx, const void* owner)
 {
     std::lock_guard<std::mutex> lock(g_contexts_mu);
     if (std::find(g_contexts.begin(), g_contexts.end(), ctx) == g_contexts.end()) return;
+    std::lock_guard<std::mutex> pool(ctx->pool_mu);
     auto& r = ctx->rooms;
     r.erase(std::remove_if(r.begin(), r.end(), [&](const auto& e) { return e.first == owner; }), r.end());
 }
@@ -2547,7 +2581,7 @@ int fg_ctx_create(int32_t device, uint64_t hbm_budget_bytes, fg_ctx** out)
     c->device = device;
     c->budget = hbm_budget_bytes;
     Lane* L = nullptr;
-    const int rc = lane_create(nullptr, &L);
+    const int rc = lane_create(device, nullptr, &L);
     if (rc != FG_OK) {
         delete c;
         return rc;
@@ -2693,8 +2727,8 @@ int fg_ctx_bandwidth_probe(fg_ctx* ctx, uint64_t bytes, int32_t reps, double* gb
 {
     if (!ctx || bytes < 16) return fail(FG_E_INVALID, "bad argument");
     void *a = nullptr, *b = nullptr;
-    HIPCHK(hipMalloc(&a, bytes));
-    hipError_t e = hipMalloc(&b, bytes);
+    HIPCHK(dev_alloc(ctx->device, &a, bytes));
+    hipError_t e = dev_alloc(ctx->device, &b, bytes);
     if (e != hipSuccess) {
         hipFree(a);
         return fail(FG_E_DEVICE, hipGetErrorString(e));

@@ -349,8 +349,9 @@ int fg_ctx_bandwidth_probe(fg_ctx* ctx, uint64_t bytes, int32_t reps, double* gb
 int fg_scene_bytes(const fg_scene_params* p, uint64_t* out);
 int fg_scene_create(fg_ctx* ctx, const fg_scene_params* p, fg_scene** out);
 /* The context may keep a destroyed scene's memory for its next scenes (at
- * most 4 GiB, and never what its budget or a server's leaves no room for); it
- * is given back when an allocation needs it and with the context. */
+ * most 4 GiB, and never what its budget or a server's leaves no room for).  It
+ * is given back with the context, and before an allocation of this library
+ * fails for want of device memory, in whichever context of the process. */
 int fg_scene_destroy(fg_scene* s);
 
 /* Polygons: polygon k has nverts[k] >= 3 vertices, (x, y) pairs in metres

@@ -103,7 +103,47 @@ def server_keeps_its_budget(fg, stub):
             assert waits > 20
 
 
-SCENARIOS = [failed_launch_leaves_no_lane_busy, pool_keeps_the_budget, server_keeps_its_budget]
+def pool_gives_way_to_every_allocation(fg, stub):
+    """Where the device has no memory left, what destroyed scenes left behind is given back: to a batch's buffers (on each
+    lane's own thread), to a set-up's polygons, to a probe, to another context and its scenes."""
+    walls, fluids = fg.dam_break_geometry(32)
+    many = [fg.box(0.2 + 1e-3 * k, 0.21 + 1e-3 * k, 0.1, 0.3) for k in range(600)]
+
+    def batch(ctx, lanes):
+        scenes = [fg.Scene(ctx, fg.make_params(32, ppc=4)) for _ in range(8)]
+        ctx.set_batch_lanes(lanes)
+        return scenes, lambda: fg.batch_step_frame(ctx, scenes)
+
+    def setup(ctx):
+        scenes = [fg.Scene(ctx, fg.make_params(32, ppc=4))]
+        return scenes, lambda: scenes[0].init_geometry(walls, many)
+
+    def other(ctx):
+        def call():
+            with fg.Context(0) as second, fg.Scene(second, fg.make_params(48, ppc=4)) as sc:
+                sc.init_geometry(walls, fluids)
+        return [], call
+
+    def probe(ctx):
+        return [], lambda: ctx.bandwidth_probe(4 << 20, 1)
+
+    def scene(ctx):
+        return [], lambda: fg.Scene(ctx, fg.make_params(96, 64, ppc=4)).close()
+
+    for make in (lambda c: batch(c, 1), lambda c: batch(c, 4), setup, other, probe, scene):
+        with fg.Context(0) as ctx:
+            live, call = make(ctx)
+            for sc in [fg.Scene(ctx, fg.make_params(64, ppc=4)) for _ in range(12)]:
+                sc.close()
+            stub.stub_limit(stub.stub_device_bytes())   # not a byte beyond what is held
+            call()
+            stub.stub_limit(2**63)
+            for sc in live:
+                sc.close()
+
+
+SCENARIOS = [failed_launch_leaves_no_lane_busy, pool_keeps_the_budget, server_keeps_its_budget,
+             pool_gives_way_to_every_allocation]
 
 
 @pytest.fixture(scope="module")
