@@ -944,6 +944,7 @@ struct Group {
     int n = 0;
     Geo g{};
     int64_t cells = 0, faces = 0, parts = 0;
+    int64_t bins = 0;                   // 3 x 3-cell bins of the fluid SDF, of all scenes
     int max_inner = 0;
     int max_bands = 0;
     bool sources = false;               // some scene has SOURCE cells (afterTransfer, reseeding)
@@ -1103,6 +1104,7 @@ int make_group(fg_ctx* ctx, const std::vector<fg_scene*>& scenes, const std::vec
         else geo_max(G.g, gs);
         first = false;
         G.cells += s->C;
+        G.bins += cdiv(s->I, 3) * cdiv(s->J, 3);
         G.faces += s->FU + s->FV;
         G.parts += s->n_bound;
         G.max_inner = std::max(G.max_inner, s->h.max_inner);
@@ -1719,9 +1721,10 @@ int levelset_bands(Group& G, bool outside)
     return FG_OK;
 }
 
-// Whether k_sdf_materials takes more lanes a bin: the group's bins, a wave
-// for 16 of them, would leave SIMDs without one (see kSdfLanesFew).
-bool few_bins(const Group& G) { return (int64_t)G.g.bins.x * (kBlock / kSdfLanes) * G.n <= kSdfFewBins; }
+// Whether k_sdf_materials takes more lanes a bin (see kSdfFewBins).  By the
+// bins that the scenes have, not by the launch's grid, whose blocks beyond a
+// smaller scene's bins exit at once.
+bool few_bins(const Group& G) { return G.bins <= kSdfFewBins; }
 dim3 few_bins_grid(const Group& G) { return dim3(G.g.bins.x * (kSdfLanesFew / kSdfLanes), (unsigned)G.n); }
 
 int run_stage(Group& G, int stage)

@@ -23,7 +23,11 @@ constexpr int kPcgTilingMaxBlocks = 4096;  // finest tiling a context may select
 constexpr int kPcgTilingMinChunk = 256;
 constexpr int kSdfLanes = 4;             // lanes per 3x3-cell bin in the fluid SDF (two or three window rows each)
 constexpr int kSdfLanesFew = 32;         // the same where a launch has few bins: three lanes a window row
-constexpr int kSdfFewBins = 16384;       // a wave a SIMD with kSdfLanes (1,849 bins at 128^2: 36.5 -> 10.7 us; 59,200, eight 256^2 scenes: 38 -> 44)
+// A launch's bins up to which kSdfLanesFew are taken.  Medians with 4 and with 32 lanes:
+// 1,849 bins (128^2) 43 and 11 us, 14,792 (eight of them) 39 and 21, 16,384 (384^2) 33 and 22,
+// 20,000 to 21,000 (mixed scenes) 36 and 23, 24,000 to 33,000 (mixed, 512^2) 31 to 35 and 30 to 42,
+// 59,000 (eight 256^2, 32 of 128^2) 35 to 45 and 53 to 56, 237,000 80 and 200.
+constexpr int kSdfFewBins = 24576;
 // multigrid preconditioner
 constexpr int kPrecondMG = 0, kPrecondIPP = 1;
 constexpr int kMgMaxLevels = 12;

@@ -3,13 +3,14 @@
 // limit), copies and fills done at once, kernels not run (what they would have
 // written stays as it was, zero at first).  A stream counts what was queued on
 // it and what has been waited for.  A chosen launch can be made to fail.
-// Loaded ahead of the library with its symbols global (test_host_memory.py).
+// Launches are counted by kernel.  Loaded ahead of the library with its symbols global (test_host_runtime.py).
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <set>
+#include <string>
 
 namespace {
 struct Stream {
@@ -31,6 +32,8 @@ constexpr int kOutOfMemory = 2, kInvalidConfiguration = 9, kLaunchFailure = 719;
 std::mutex mu;
 std::map<void*, uint64_t> device, pinned;
 std::set<Stream*> streams;
+std::map<const void*, std::string> kernels;
+std::map<const void*, long> launches;
 uint64_t device_bytes = 0, limit = ~0ull;
 long fail_launch = -1;   // launches until one fails
 thread_local int last_error = 0;
@@ -43,10 +46,11 @@ int queue(Stream* s)
     s->queued++;
     return 0;
 }
-int launch(Dim3 g, Dim3 b, Stream* s)
+int launch(const void* f, Dim3 g, Dim3 b, Stream* s)
 {
     {
         std::lock_guard<std::mutex> lock(mu);
+        launches[f]++;
         if (fail_launch >= 0 && fail_launch-- == 0) return error(kLaunchFailure);
     }
     if (!g.x || !g.y || !g.z || !b.x || !b.y || !b.z || b.x * b.y * b.z > 1024) return error(kInvalidConfiguration);
@@ -61,6 +65,16 @@ uint64_t stub_allocations() { return device.size() + pinned.size(); }
 void stub_limit(uint64_t bytes) { limit = bytes; }
 void stub_fail_launch(long n) { fail_launch = n; }
 int stub_launch_failed() { return fail_launch == -1; }
+// launches of the kernels whose (mangled) name holds `part` since the last reset
+long stub_launches(const char* part)
+{
+    std::lock_guard<std::mutex> lock(mu);
+    long n = 0;
+    for (const auto& l : launches)
+        if (kernels[l.first].find(part) != std::string::npos) n += l.second;
+    return n;
+}
+void stub_reset_launches() { launches.clear(); }
 int stub_busy_streams()
 {
     std::lock_guard<std::mutex> lock(mu);
@@ -164,10 +178,10 @@ int hipGetSymbolAddress(void** p, const void*)
     static void* const scratch = std::calloc(1, 64 << 20);
     return *p = scratch, 0;
 }
-int hipLaunchKernel(const void*, Dim3 g, Dim3 b, void**, size_t, Stream* s) { return launch(g, b, s); }
-int hipExtLaunchKernel(const void*, Dim3 g, Dim3 b, void**, size_t, Stream* s, Event* a, Event* z, int)
+int hipLaunchKernel(const void* f, Dim3 g, Dim3 b, void**, size_t, Stream* s) { return launch(f, g, b, s); }
+int hipExtLaunchKernel(const void* f, Dim3 g, Dim3 b, void**, size_t, Stream* s, Event* a, Event* z, int)
 {
-    const int e = launch(g, b, s);
+    const int e = launch(f, g, b, s);
     if (a) hipEventRecord(a, s);
     if (z) hipEventRecord(z, s);
     return e;
@@ -187,6 +201,9 @@ void** __hipRegisterFatBinary(const void*)
     return &handle;
 }
 void __hipUnregisterFatBinary(void**) {}
-void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsigned, void*, void*, void*, void*, int*)
+{
+    kernels[f] = name;
+}
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 }

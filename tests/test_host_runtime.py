@@ -1,5 +1,5 @@
-"""The library's host code over a stand-in for the HIP runtime (hip_host_stub.cpp): what waits for what, and whose memory
-counts where.  Each scenario runs in a process of its own, with the stand-in's symbols ahead of the runtime's."""
+"""The library's host code over a stand-in for the HIP runtime (hip_host_stub.cpp): what waits for what, whose memory counts
+where, and which kernels a rule picks.  Each scenario runs in a process of its own, with the stand-in's symbols ahead of the runtime's."""
 import ctypes as C
 import os
 import random
@@ -142,8 +142,30 @@ def pool_gives_way_to_every_allocation(fg, stub):
                 sc.close()
 
 
+def _batch(fg, ctx, sizes):
+    out = []
+    for n in sizes:
+        walls, fluids = fg.dam_break_geometry(n)
+        out.append(fg.Scene(ctx, fg.make_params(n, ppc=1)))
+        out[-1].init_geometry(walls, fluids)
+    return out
+
+
+def sdf_lanes_by_the_bins_of_the_group(fg, stub):
+    """k_sdf_materials' 32 lanes a bin where the bins of the group's scenes together are few, however uneven their sizes."""
+    for sizes, few in (([64] * 8, True), ([256] + [32] * 40, True), ([256] * 4, False), ([512] + [32], False), ([32] * 250, False)):
+        with fg.Context(0) as ctx:
+            scenes = _batch(fg, ctx, sizes)
+            stub.stub_reset_launches()
+            fg.batch_step_frame(ctx, scenes)
+            wide, plain = (stub.stub_launches(b"k_sdf_materialsILi%dE" % k) for k in (32, 4))
+            assert (wide > 0, plain > 0) == (few, not few), (sizes[0], len(sizes), wide, plain)
+            for sc in scenes:
+                sc.close()
+
+
 SCENARIOS = [failed_launch_leaves_no_lane_busy, pool_keeps_the_budget, server_keeps_its_budget,
-             pool_gives_way_to_every_allocation]
+             pool_gives_way_to_every_allocation, sdf_lanes_by_the_bins_of_the_group]
 
 
 @pytest.fixture(scope="module")
@@ -164,6 +186,8 @@ if __name__ == "__main__":
     _stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
     _stub.stub_device_bytes.restype = _stub.stub_allocations.restype = C.c_uint64
     _stub.stub_limit.argtypes = [C.c_uint64]
+    _stub.stub_launches.argtypes = [C.c_char_p]
+    _stub.stub_launches.restype = C.c_long
     _stub.stub_fail_launch.argtypes = [C.c_long]
     sys.path.insert(0, os.path.dirname(HERE))
     import flipsolver2d_amd as _fg
