@@ -1700,11 +1700,17 @@ int levelset_bands(Group& G, bool outside)
     // outside chain (NB-FLIP, far longer) keeps the count it launched
     int hint = 0;
     for (fg_scene* s : G.sc) hint = std::max(hint, outside ? s->ls_hint_out : (s->ls_hint > 0 ? s->ls_hint + 1 : 0));
-    // a band after the last one costs 2 us of launch, a poll 25 us of an idle
-    // device: where few bands can be left, all are launched and none polled
-    constexpr int kNoPoll = 10;
+    // A poll is 10 us (the hint was right) to 25 us of an idle device; a band
+    // after the last one 2 us of launch up to some 1,000 blocks, 4.5 at 2,000
+    // to 7,000, 9 at 16,000.  Where those that can be left cost no more than a
+    // poll, all are launched and none polled.  A substep (medians, always
+    // polled and so): 64^2 0.446 and 0.437 ms, 0.473 and 0.458 in the first
+    // three frames, 128^2 0.617 and 0.612, eight 64^2 scenes 0.495 and 0.490;
+    // from 192^2 or 100 scenes on the same either way.
+    const int64_t blocks = (int64_t)std::min<unsigned>(G.g.ls.x, kBandBlocks) * G.n;
+    const int spare = blocks <= 1024 ? 10 : blocks <= 8192 ? 5 : 2;
     int chunk = hint > 0 ? hint : kChunk;
-    const bool all = G.max_bands - (hint > 0 ? hint - 1 : 0) <= kNoPoll;
+    const bool all = G.max_bands - (hint > 0 ? hint - 1 : 0) <= spare;
     if (all) chunk = G.max_bands;
     int32_t flags[3];
     int launched = 0;
@@ -2372,7 +2378,9 @@ fg_scene_params solve_params(int32_t size_i, int32_t size_j, double rel_tol, int
 // matrix comes as materials (assembled on the device, k_stencil) or as its
 // bytes (one per cell, the stencil format of fg_scene_state).  staged: a
 // result of kStagedLeast or more comes back through the context's pinned
-// windows, which a caller that may not allocate does without.
+// windows, which a caller that may not allocate does without.  A solve with
+// its result staged and copied by the runtime: 1.19 and 1.16 ms at 2 MiB, 1.59
+// and 1.60 at 4 MiB, 2.43 and 2.55 at 8 MiB, 7.1 and 8.8 at 32 MiB.
 constexpr int64_t kStagedLeast = 4 << 20;
 int solve_on_scene(fg_scene* s, const int8_t* material, const uint8_t* stencil, double scale, const double* b,
                    double* x, fg_solve_stats* stats, bool staged)

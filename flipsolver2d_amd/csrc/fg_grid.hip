@@ -777,7 +777,6 @@ __global__ void __launch_bounds__(kBlock) k_levelset_init(const SceneDev* scenes
 // 1024^2 NB-FLIP dam break's 649 bands of 3 frames: 31.8 us a launch with a
 // block a tile and the search inside the level loop, 14.8 us so.  256 blocks
 // are one a CU.
-constexpr int kBandBlocks = 256;
 template <bool OUT>
 __global__ void __launch_bounds__(kBlock) k_levelset_band(const SceneDev* scenes, int band)
 {

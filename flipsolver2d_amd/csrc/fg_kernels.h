@@ -97,6 +97,7 @@ FG_DECLARE_LAUNCH(apply_solids, int friction);
 FG_DECLARE_LAUNCH(density_rhs);
 FG_DECLARE_LAUNCH(density_adjust);
 constexpr int kBfsTile = 32;
+constexpr int kBandBlocks = 256;   // most blocks a scene of a level-set band's launch (band 0: one a tile)
 
 // fg_init.hip
 // Polygons of a scene's set-up, by set: 0 sinks, 1 sources, 2 solids,

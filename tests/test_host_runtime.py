@@ -164,8 +164,23 @@ def sdf_lanes_by_the_bins_of_the_group(fg, stub):
                 sc.close()
 
 
+def bands_polled_where_empty_ones_cost_more(fg, stub):
+    """A level set of nine bands at most (128^2): a few scenes launch all nine, many look after eight whether any is left
+    (none is here); more than about ten bands are always looked at."""
+    for count, n, want in ((1, 128, 9), (32, 128, 9), (96, 128, 8), (1, 512, 8)):
+        with fg.Context(0) as ctx:
+            scenes = _batch(fg, ctx, [n] * count)
+            stub.stub_reset_launches()
+            fg.batch_step_frame(ctx, scenes)
+            got = stub.stub_launches(b"k_levelset_band")
+            assert got == want, (count, n, got, want)
+            for sc in scenes:
+                sc.close()
+
+
 SCENARIOS = [failed_launch_leaves_no_lane_busy, pool_keeps_the_budget, server_keeps_its_budget,
-             pool_gives_way_to_every_allocation, sdf_lanes_by_the_bins_of_the_group]
+             pool_gives_way_to_every_allocation, sdf_lanes_by_the_bins_of_the_group,
+             bands_polled_where_empty_ones_cost_more]
 
 
 @pytest.fixture(scope="module")
