@@ -1144,13 +1144,16 @@ __global__ void __launch_bounds__(kBlock) k_mg_post(const SceneDev* scenes, cons
 // stages in LDS the tile with a one-cell halo, code and r, and the level-1
 // patch under it, so z0 is formed once per cell (and once more per halo
 // cell) from LDS instead of five times from 30 global loads, which bound
-// the per-cell form by instruction issue.  The quotients by D1, an integer
-// up to 8, are a product with its reciprocal and one step with the exact
-// remainder (correctly rounded, as the division).  A tile is the fine side of
+// the per-cell form by instruction issue.  The quotients by D1, an integer up
+// to kMaxD1, are a product with its reciprocal and one step with the exact
+// remainder: the division's result, but for a remainder that is subnormal
+// (an ulp of it) and an infinite residual (NaN; the solve ends as it does
+// for infinity).  A tile is the fine side of
 // k_mg_step0's and k_pcg_dir's, in their order, so what one writes the
 // other reads through the same XCD's L2.  Per-cell form (each cell its
 // neighbours' z0) 8.3 us at 128^2, 10.1 us at 1024^2; an LDS window of whole
 // rows over linear chunks 97 us at 4096^2; this form 4.8, 7.3 and 36 us.
+constexpr int kMaxD1 = 11;               // a code's count (three bits; 4 where materials made it) and four neighbours
 constexpr int kUpR = kUpTile + 2;        // cells a side with the halo
 constexpr int kUpY = kUpTile / 2 + 2;    // level-1 cells a side that the halo's cells prolong from
 static_assert(kUpTile % 2 == 0 && kUpTile * kUpTile % kBlock == 0 && kBlock % kUpTile == 0, "whole rows of a tile a pass");
@@ -1161,7 +1164,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_up0(const SceneDev* scenes, const
     __shared__ float rs[kUpR][kUpR + 1];
     __shared__ uint8_t cs[kUpR][kUpR + 2];
     __shared__ float ys[kUpY][kUpY + 1];
-    __shared__ float inv[9];                 // 1 / D1
+    __shared__ float inv[kMaxD1 + 1];        // 1 / D1
     const SceneBlock sb = scene_block(map, true);
     const SceneDev& s = scenes[sb.scene];
     const auto& L1 = cst(s.mg)->lv[1];
@@ -1174,7 +1177,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_up0(const SceneDev* scenes, const
     const int tilesJ = (J + kUpTile - 1) / kUpTile, tiles = ((I + kUpTile - 1) / kUpTile) * tilesJ;
     const int per = (tiles + s.up_blocks - 1) / s.up_blocks;
     const int t1 = min(tiles, (sb.block + 1) * per);
-    if (threadIdx.x < 9) inv[threadIdx.x] = threadIdx.x ? 1.0f / (float)threadIdx.x : 0.f;
+    if (threadIdx.x <= kMaxD1) inv[threadIdx.x] = threadIdx.x ? 1.0f / (float)threadIdx.x : 0.f;
     // w x / D1 (0 where D1 is)
     auto over_d = [&](float x, int d) {
         const float n = kMgOmega * x, rd = inv[d], q = n * rd;

@@ -47,3 +47,30 @@ def test_viscosity_tiles(fg, orc, ctx, n_i, n_j):
     assert np.array_equal(g["viscosity"].view(np.uint32), st.viscosity.view(np.uint32))
     e = [rel_l2(g[k], getattr(st, k)) for k in ("pressure", "u", "v")]
     assert max(e) <= 1e-5, e
+
+
+# A caller's own rows: counts up to the 7 that the three bits hold (materials give 4 at most), one to three above the row's
+# neighbours.  The matrix is diagonally dominant by 1 and its norm at most 7 + 4, so its condition is at most 11 and a
+# residual of 1e-10 ||b|| leaves x within 1.1e-9 of the solution; the other 1e-10 is the direct solve's and rounding's.
+@pytest.mark.parametrize("shape", [(33, 65), (97, 129)])
+def test_matrix_with_counts_to_seven(fg, ctx, shape):
+    from scipy.sparse import diags
+    from scipy.sparse.linalg import spsolve
+    rng = np.random.default_rng(shape[0])
+    I, J = shape
+    on = np.zeros((I, J), bool)
+    on[1:-1, 1:-1] = rng.random((I - 2, J - 2)) < 0.85
+    nb = [np.roll(on, s, a) & on for s, a in ((1, 0), (-1, 0), (1, 1), (-1, 1))]   # i-1, i+1, j-1, j+1
+    deg = sum(n.astype(int) for n in nb)
+    count = np.where(on, deg + rng.integers(1, 4, on.shape), 0)
+    assert count.max() == 7 and count.min() == 0
+    code = np.where(on, 0x80 | (count << 4) | sum(n.astype(int) << k for k, n in enumerate(nb)), 0).astype(np.uint8)
+    b = np.where(on, rng.standard_normal(on.shape), 0.0).ravel()
+    A = diags([np.where(on, count, 1).ravel().astype(float), -(nb[1].ravel()[:-J].astype(float)),
+               -(nb[0].ravel()[J:].astype(float)), -(nb[3].ravel()[:-1].astype(float)), -(nb[2].ravel()[1:].astype(float))],
+              [0, J, -J, 1, -1], format="csc")
+    x, st = np.zeros(I * J), fg.SolveStats()
+    fg._check(fg.lib().fg_poisson_solve_matrix(ctx.h, I, J, code.ctypes.data, 1.0, b.ctypes.data, x.ctypes.data, 1e-10, 0,
+                                               C.byref(st)))
+    print(f"{shape}: {st.iterations} iterations", flush=True)
+    assert st.converged and rel_l2(x, spsolve(A, b)) <= 1.2e-9
