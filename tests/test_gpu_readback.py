@@ -18,9 +18,28 @@ def _one(fg, scene, name, like):
     return a[:st.n_particles] if name in PARTICLES else a
 
 
-# one window, ragged sides, viscosity; two; five (a window is 16 MiB); the last two with more particles than 2 ppc a cell
-@pytest.mark.parametrize("I,J,n,visc", [(37, 61, 900, True), (513, 259, 300_001, False), (1021, 767, 1_500_000, False)])
-def test_state_arrays_and_erased_particles(fg, ctx, I, J, n, visc):
+WINDOW = 16 << 20
+
+
+def _stream(I, J, n, visc):
+    """Where the packed state's first plain array and its end lie: each component of n particles (4 bytes), then each array
+    of what Scene.get_state asks for, every one on a 256-byte boundary."""
+    C, U, V = I * J, (I + 1) * J, I * (J + 1)
+    pad = lambda b: (b + 255) // 256 * 256  # noqa: E731
+    arrays = [4 * U, 4 * V, U, V, C, 4 * C, 4 * C, 4 * C, 4 * C, 4 * U, 4 * V, 8 * C, 8 * C, C, 4 * C, 4 * U, 4 * V]
+    first = pad(4 * n) * (6 if visc else 5)
+    return first, first + sum(pad(b) for b in arrays + ([4 * C] if visc else []))
+
+
+# One window, ragged sides, viscosity; two; five (a window is 16 MiB); the plain arrays starting 256 bytes before a window's
+# end, the components filling their sections and not, and 1,024 bytes after it.  The larger ones with more particles than
+# 2 ppc a cell.
+@pytest.mark.parametrize("I,J,n,visc,windows,first", [
+    (37, 61, 900, True, 1, None), (513, 259, 500_001, False, 2, None), (1021, 767, 1_500_000, False, 5, None),
+    (523, 67, 838_848, False, 2, -256), (523, 67, 838_785, False, 2, -256), (523, 67, 838_849, False, 2, 1024)])
+def test_state_arrays_and_erased_particles(fg, ctx, I, J, n, visc, windows, first):
+    at, end = _stream(I, J, n, visc)
+    assert (end + WINDOW - 1) // WINDOW == windows and (first is None or at - WINDOW == first), (at, end)
     rng = np.random.default_rng(I)
     walls, _ = fg.dam_break_geometry(I)
     p = fg.make_params(I, J, ppc=2, viscosity=visc, max_particles=n + 7)
