@@ -720,7 +720,7 @@ Geo geometry(const fg_scene* s)
     g.pcg = dim3((unsigned)s->pcg_blocks);
     g.bins = dim3((unsigned)cdiv(cdiv(s->I, 3) * cdiv(s->J, 3), kBlock / kSdfLanes));
     g.p2g = dim3((unsigned)(cdiv(s->I, 16) * cdiv(s->J, 16)));
-    g.visc = g.p2g;   // kViscTile = 16
+    g.visc = dim3((unsigned)(cdiv(s->I, kViscTile) * cdiv(s->J, kViscTile)));
     g.nodes = dim3((unsigned)cdiv((int64_t)(s->I + 1) * (s->J + 1), kBlock));
     return g;
 }

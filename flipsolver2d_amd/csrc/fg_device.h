@@ -231,6 +231,7 @@ struct SceneDev {
 };
 // viscosity CG scalars (per system s = 0 (U), 1 (V)): bb at s, rz of even and
 // odd iterations at 2 + s and 4 + s, done at 12 + s, the iteration counts at 14 + s
+constexpr int kViscTile = 16;          // k_visc_p: cells a block, per side
 constexpr int kViscSlots = 4;         // per-block partials: two dots x two systems
 constexpr int kViscScalars = 16;
 constexpr int kMaxEmitters = 256;
@@ -464,19 +465,58 @@ __device__ __forceinline__ void wave_sum(double (&v)[NV])
     for (int q = 0; q < NV; q++) v[q] += row_shl<0x101>(v[q]);
 }
 
-// wave64 + block reduction of doubles; result valid in thread 0.
-__device__ __forceinline__ double block_sum(double v, double* lds)
+// Sums of n values each, from NV rows of `part` `stride` apart, in a fixed
+// order (thread t takes values t, t + kBlock, ...; then a fixed wave and LDS
+// tree), in every thread: every block computing them gets identical values.
+// Every thread adds the waves' sums itself, so one barrier serves all NV
+// values; a kernel calls it once for each NV (its LDS is not reused).
+template <int NV>
+__device__ __forceinline__ void sum_rows(const double* part, size_t stride, int n, double (&out)[NV])
 {
-    double w1[1] = {v};
-    wave_sum<1>(w1);
+    __shared__ double red[NV][kBlock / 64];
+    double acc[NV];
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        gptr<const double> row = gbl<const double>(part + q * stride);
+        acc[q] = 0.0;
+        for (int b = threadIdx.x; b < n; b += kBlock) acc[q] += row[b];
+    }
+    wave_sum<NV>(acc);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0)
+#pragma unroll
+        for (int q = 0; q < NV; q++) red[q][w] = acc[q];
     __syncthreads();
-    if (lane == 0) lds[w] = w1[0];
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; k++) t += red[q][k];
+        out[q] = t;
+    }
+}
+
+// The block's sums of NV values a thread, to out[q * stride + blk] (once a
+// kernel for each NV, as above).
+template <int NV>
+__device__ __forceinline__ void put_sums(double* out, size_t stride, int blk, const double (&v)[NV])
+{
+    __shared__ double red[NV][kBlock / 64];
+    double acc[NV];
+#pragma unroll
+    for (int q = 0; q < NV; q++) acc[q] = v[q];
+    wave_sum<NV>(acc);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0)
+#pragma unroll
+        for (int q = 0; q < NV; q++) red[q][w] = acc[q];
     __syncthreads();
-    double t = 0.0;
-    if (threadIdx.x == 0)
-        for (int k = 0; k < (int)(blockDim.x >> 6); k++) t += lds[k];
-    return t;
+    if (threadIdx.x < NV) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; k++) t += red[threadIdx.x][k];
+        gbl(out)[threadIdx.x * stride + blk] = t;
+    }
 }
 
 __device__ __forceinline__ float block_maxf(float v, float* lds)
@@ -520,58 +560,19 @@ __device__ __forceinline__ Chunk my_chunk(const SceneDev& s, int blk)
     return Chunk{beg < C ? beg : C, min(C, beg + s.pcg_chunk)};
 }
 
-// Sum of the nb per-block partials of `slot`, in a fixed order (thread t
-// takes partials t, t+256, ...; then a fixed wave and LDS tree), in every
-// thread.  Every block computing it gets the identical value.  Every thread
-// adds the waves' sums itself, so one barrier serves all NV values; a kernel
-// calls it once (its LDS is not reused).
+// The sums of the nb per-block partials of `slot` and the next ones, in every
+// thread of every block.
 template <int NV>
 __device__ __forceinline__ void sum_partials(const SceneDev& s, int slot, int nb, double (&out)[NV])
 {
-    __shared__ double red[NV][kBlock / 64];
-    double acc[NV];
-#pragma unroll
-    for (int q = 0; q < NV; q++) {
-        gptr<const double> part = gbl<const double>(s.partials + (size_t)(slot + q) * s.max_blocks);
-        acc[q] = 0.0;
-        for (int b = threadIdx.x; b < nb; b += kBlock) acc[q] += part[b];
-    }
-    wave_sum<NV>(acc);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0)
-#pragma unroll
-        for (int q = 0; q < NV; q++) red[q][w] = acc[q];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < NV; q++) {
-        double t = 0.0;
-#pragma unroll
-        for (int k = 0; k < kBlock / 64; k++) t += red[q][k];
-        out[q] = t;
-    }
+    sum_rows<NV>(s.partials + (size_t)slot * s.max_blocks, s.max_blocks, nb, out);
 }
 
-// Block-reduce NV doubles and store them as the partials of solver block blk
-// (once a kernel, as above).
+// The block's sums as the partials of solver block blk.
 template <int NV>
-__device__ __forceinline__ void put_partials(const SceneDev& s, int slot, double (&v)[NV], int blk)
+__device__ __forceinline__ void put_partials(const SceneDev& s, int slot, const double (&v)[NV], int blk)
 {
-    __shared__ double red[NV][kBlock / 64];
-    double acc[NV];
-#pragma unroll
-    for (int q = 0; q < NV; q++) acc[q] = v[q];
-    wave_sum<NV>(acc);
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0)
-#pragma unroll
-        for (int q = 0; q < NV; q++) red[q][w] = acc[q];
-    __syncthreads();
-    if (threadIdx.x < NV) {
-        double t = 0.0;
-#pragma unroll
-        for (int k = 0; k < kBlock / 64; k++) t += red[threadIdx.x][k];
-        s.partials[(size_t)(slot + threadIdx.x) * s.max_blocks + blk] = t;
-    }
+    put_sums<NV>(s.partials + (size_t)slot * s.max_blocks, s.max_blocks, blk, v);
 }
 
 }  // namespace fg

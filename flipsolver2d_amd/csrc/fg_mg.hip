@@ -108,23 +108,33 @@ __device__ __forceinline__ void load_coef_row(gptr<const float> coef, int c, flo
     for (int k = 0; k < kMgStencil; k++) a[k] = q[k >> 2][k & 3];
 }
 
-// sum_k a_k v_k over an active level-l row (dinv != 0) with the level's 25
-// stencil entries: the canonical stencil on canonical rows (dinv < 0), else
-// the stored coefficients, loaded only by the lanes whose rows need them.
+// The 25 entries of an active level-l row (dinv != 0): the canonical stencil
+// on canonical rows (dinv < 0), else the stored coefficients, loaded only by
+// the lanes whose rows need them; and their sum over v.  Two steps, so that a
+// kernel can issue the loads early.
 template <typename MT>
-__device__ __forceinline__ float row_dot(const MT& M, int l, gptr<const float> coef, int CL, int c,
-                                         float dinv_c, const float (&v)[kMgStencil])
+__device__ __forceinline__ void row_load(const MT& M, int l, gptr<const float> coef, int c, float dinv_c,
+                                         float (&a)[kMgStencil])
 {
-    (void)CL;
     const auto& cn = M.canon[l];
-    float a[kMgStencil];
 #pragma unroll
     for (int k = 0; k < kMgStencil; k++) a[k] = cn[k];
     if (dinv_c > 0.f) load_coef_row(coef, c, a);
+}
+__device__ __forceinline__ float row_sum(const float (&a)[kMgStencil], const float (&v)[kMgStencil])
+{
     float ax = 0.f;
 #pragma unroll
     for (int k = 0; k < kMgStencil; k++) ax += a[k] * v[k];
     return ax;
+}
+template <typename MT>
+__device__ __forceinline__ float row_dot(const MT& M, int l, gptr<const float> coef, int c, float dinv_c,
+                                         const float (&v)[kMgStencil])
+{
+    float a[kMgStencil];
+    row_load(M, l, coef, c, dinv_c, a);
+    return row_sum(a, v);
 }
 
 // r at coarse cell (ci, cj) from the finer level's y (FI x FJ): 1-D weights
@@ -664,7 +674,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_resid(const SceneDev* scenes, con
         xv[k] = (rn * fabsf(dn)) * mask01(ok);   // a 0/1 factor, not a select: the load stays unconditional
     }
     const float rc = r[c];
-    const float ax = row_dot(M, l, gbl<const float>(L.coef), CL, c, dc, xv);
+    const float ax = row_dot(M, l, gbl<const float>(L.coef), c, dc, xv);
     gbl(L.y)[c] = rc - ax;
 }
 
@@ -713,15 +723,6 @@ __global__ void __launch_bounds__(kBlock) k_mg_restrict(const SceneDev* scenes, 
 // coefficients read from LDS in every sweep, took 13.8 us a launch at
 // 32 x 32 over 16 x 16 cells; this form 9.7 us (the 128^2 dam break).
 __device__ __forceinline__ bool mg_active(float dinv) { return __float_as_uint(dinv) != 0u; }
-
-// The 25 coefficients of an active level-l row (see row_dot).
-template <typename MT>
-__device__ __forceinline__ void coarse_row(const MT& M, int l, int c, float dinv_c, float (&a)[kMgStencil])
-{
-#pragma unroll
-    for (int k = 0; k < kMgStencil; k++) a[k] = M.canon[l][k];
-    if (dinv_c > 0.f) load_coef_row(gbl<const float>(M.lv[l].coef), c, a);
-}
 
 // sum_k a_k x_k over the 5x5 neighbourhood of x[home], rows w floats apart
 __device__ __forceinline__ float coarse_dot(const float (&a)[kMgStencil], const float* x, int home, int w)
@@ -790,7 +791,7 @@ __global__ void __launch_bounds__(kMgCoarseThreads) k_mg_coarse(const SceneDev* 
     }
     // round 2: this thread's level-t row
     float ct[kMgStencil];
-    if (t < nb) coarse_row(M, t, tc, tin ? dt : 0.f, ct);
+    if (t < nb) row_load(M, t, gbl<const float>(T.coef), tc, tin ? dt : 0.f, ct);
     __syncthreads();
     int ho = 0;   // level l's place in hx and hy
     for (int l = t; l < nb; l++) {   // down: y = r - A x, r_{l+1} = R y, x_{l+1} = r_{l+1} dinv
@@ -806,7 +807,7 @@ __global__ void __launch_bounds__(kMgCoarseThreads) k_mg_coarse(const SceneDev* 
                     ax = coarse_dot(ct, hx, home, w);
                 } else {
                     float a[kMgStencil];
-                    coarse_row(M, l, tid, dc, a);
+                    row_load(M, l, gbl<const float>(L.coef), tid, dc, a);
                     ax = coarse_dot(a, hx, home, w);
                 }
                 y = rs[o + tid] - ax;
@@ -882,7 +883,7 @@ __global__ void __launch_bounds__(kMgCoarseThreads) k_mg_coarse(const SceneDev* 
                     ax = coarse_dot(ct, hx, home, w);
                 } else {
                     float a[kMgStencil];
-                    coarse_row(M, l, tid, dc, a);
+                    row_load(M, l, gbl<const float>(L.coef), tid, dc, a);
                     ax = coarse_dot(a, hx, home, w);
                 }
                 y = x + fabsf(dc) * (rc - ax);
@@ -915,25 +916,6 @@ constexpr int kRRY = 2 * kRRTile + 2;   // fine cells a side whose residual the 
 constexpr int kRRX = kRRY + 4;          // and the x their stencils read
 static_assert(kRRY * kRRY == kBlock, "one fine residual per thread: a second round would be a second chain");
 constexpr int kPPX = kVcTile + 4;       // level-l cells a side whose x the post-smoothing reads
-
-// a[k] and the canonical row cn[k] of an active level-l row, and their sum
-// over v (row_dot in two steps, so that the loads can be issued early)
-template <typename MT>
-__device__ __forceinline__ void row_load(const MT& M, int l, gptr<const float> coef, int c, float dinv_c,
-                                         float (&a)[kMgStencil])
-{
-    const auto& cn = M.canon[l];
-#pragma unroll
-    for (int k = 0; k < kMgStencil; k++) a[k] = cn[k];
-    if (dinv_c > 0.f) load_coef_row(coef, c, a);
-}
-__device__ __forceinline__ float row_sum(const float (&a)[kMgStencil], const float (&v)[kMgStencil])
-{
-    float ax = 0.f;
-#pragma unroll
-    for (int k = 0; k < kMgStencil; k++) ax += a[k] * v[k];
-    return ax;
-}
 
 // Level l (1 <= l < t), down: x = r dinv and y = r - A_l x over the fine
 // patch of a kRRTile x kRRTile tile of level-(l+1) cells, then r_{l+1} = R y
@@ -1132,7 +1114,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_post(const SceneDev* scenes, cons
     float xv[kMgStencil];
     gather25(x, LI, LJ, ci, cj, xv);
     const float rc = gbl<const float>(L.r)[c];
-    const float ax = row_dot(M, l, gbl<const float>(L.coef), CL, c, dc, xv);
+    const float ax = row_dot(M, l, gbl<const float>(L.coef), c, dc, xv);
     gbl(L.y)[c] = xv[12] + fabsf(dc) * (rc - ax);
 }
 

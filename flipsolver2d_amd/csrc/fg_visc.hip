@@ -96,50 +96,8 @@ __global__ void __launch_bounds__(kBlock) k_visc_grid(const SceneDev* scenes)
     s.cvisc[c] = v;
 }
 
-// Sums over the block of NV doubles, to out[q * stride + block].
-template <int NV>
-__device__ __forceinline__ void visc_put(double* out, int stride, double (&v)[NV])
-{
-    __shared__ double red[NV][kBlock / 64];
-    wave_sum<NV>(v);
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int q = 0; q < NV; q++) red[q][threadIdx.x >> 6] = v[q];
-    __syncthreads();
-    if (threadIdx.x < NV) {
-        double t = 0.0;
-#pragma unroll
-        for (int k = 0; k < kBlock / 64; k++) t += red[threadIdx.x][k];
-        gbl(out)[(size_t)threadIdx.x * stride + blockIdx.x] = t;
-    }
-}
-
-// The sums of n partials of NV slots, the same in every thread and block.
-template <int NV>
-__device__ __forceinline__ void visc_sum(const double* part, int stride, int n, double (&out)[NV])
-{
-    __shared__ double red[NV][kBlock / 64];
-#pragma unroll
-    for (int q = 0; q < NV; q++) {
-        out[q] = 0.0;
-        for (int b = threadIdx.x; b < n; b += kBlock) out[q] += gbl(part)[(size_t)q * stride + b];
-    }
-    wave_sum<NV>(out);
-    if ((threadIdx.x & 63) == 0)
-#pragma unroll
-        for (int q = 0; q < NV; q++) red[q][threadIdx.x >> 6] = out[q];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < NV; q++) {
-        out[q] = 0.0;
-#pragma unroll
-        for (int k = 0; k < kBlock / 64; k++) out[q] += red[q][k];
-    }
-}
-
 // vsc: bb 0-1, rz of even iterations 2-3 and of odd ones 4-5, done 12-13,
 // iterations 14-15 (system 0 U, 1 V).
-constexpr int kViscTile = 16;
 __device__ __forceinline__ int visc_tiles_j(const SceneDev& s) { return (s.J + kViscTile - 1) / kViscTile; }
 __device__ __forceinline__ int visc_tiles(const SceneDev& s) { return ((s.I + kViscTile - 1) / kViscTile) * visc_tiles_j(s); }
 // The direction of system q at iteration it.  The second buffers are arrays
@@ -192,7 +150,7 @@ __global__ void __launch_bounds__(kBlock) k_visc_setup(const SceneDev* scenes)
         rzv = bv * zv;
     }
     double v[4] = {bbu, bbv, rzu, rzv};
-    visc_put<4>(s.vpart, visc_blocks(s), v);
+    put_sums<4>(s.vpart, visc_blocks(s), blockIdx.x, v);
 }
 
 __global__ void __launch_bounds__(kBlock) k_visc_p(const SceneDev* scenes, int it, double tol2)
@@ -223,7 +181,7 @@ __global__ void __launch_bounds__(kBlock) k_visc_p(const SceneDev* scenes, int i
     const double e = gbl(s.ve)[c], n = gbl(s.vn)[c], ew = gbl(s.ve)[max(c - J, 0)], ns = gbl(s.vn)[max(c - 1, 0)];
     // the sums of k_visc_setup (bb, rz) or of the iteration before (rr, rz)
     double sum[4];
-    visc_sum<4>(s.vpart, visc_blocks(s), visc_blocks(s), sum);
+    sum_rows<4>(s.vpart, visc_blocks(s), visc_blocks(s), sum);
     double* const v = s.vsc;
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     bool go[2];
@@ -268,7 +226,7 @@ __global__ void __launch_bounds__(kBlock) k_visc_p(const SceneDev* scenes, int i
             pq[q] = p * t;
         }
     }
-    visc_put<2>(visc_pq(s), visc_tiles(s), pq);
+    put_sums<2>(visc_pq(s), visc_tiles(s), blockIdx.x, pq);
 }
 
 __global__ void __launch_bounds__(kBlock) k_visc_x(const SceneDev* scenes, int it)
@@ -291,7 +249,7 @@ __global__ void __launch_bounds__(kBlock) k_visc_x(const SceneDev* scenes, int i
     const bool go[2] = {v[12] == 0.0, v[13] == 0.0};
     if (!go[0] && !go[1]) return;
     double pq[2];
-    visc_sum<2>(visc_pq(s), visc_tiles(s), visc_tiles(s), pq);
+    sum_rows<2>(visc_pq(s), visc_tiles(s), visc_tiles(s), pq);
     double sum[4] = {0.0, 0.0, 0.0, 0.0};   // rr, rz
     if (c < C) {
 #pragma unroll
@@ -306,7 +264,7 @@ __global__ void __launch_bounds__(kBlock) k_visc_x(const SceneDev* scenes, int i
             sum[2 + q] = rn * (rn / d);
         }
     }
-    visc_put<4>(s.vpart, visc_blocks(s), sum);
+    put_sums<4>(s.vpart, visc_blocks(s), blockIdx.x, sum);
 }
 
 __global__ void __launch_bounds__(kBlock) k_visc_apply(const SceneDev* scenes)
