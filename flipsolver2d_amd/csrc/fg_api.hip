@@ -1032,12 +1032,8 @@ void apply_tiling(const fg_ctx* ctx, fg_scene* s)
     s->pcg_blocks = (int)blocks;
     s->h.pcg_chunk = s->pcg_chunk;
     s->h.pcg_blocks = s->pcg_blocks;
-    // k_mg_up0's tiles: as many to a block as the least chunk holds, more
-    // where the blocks or the partials run out
-    const int64_t tiles = cdiv(s->I, kUpTile) * cdiv(s->J, kUpTile);
-    const int64_t least = cdiv(tiles, std::max(1, ctx->pcg_min_chunk / (kUpTile * kUpTile)));
-    const int64_t ub = std::min<int64_t>({least, ctx->pcg_target_blocks, s->max_blocks});
-    s->h.up_blocks = (int)cdiv(tiles, cdiv(tiles, ub));   // every block has a tile
+    s->h.up_blocks = (int)up_block_count(up_tiles(s->I, s->J), ctx->pcg_min_chunk,
+                                         std::min<int64_t>(ctx->pcg_target_blocks, s->max_blocks));
 }
 
 int ensure_group_buffers(Lane* L, int n)

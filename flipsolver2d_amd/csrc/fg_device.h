@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fg_tiles.h"
+
 namespace fg {
 
 constexpr int kBlock = 256;             // threads per block (4 wave64s)
@@ -38,7 +40,6 @@ __host__ __device__ inline int mg_d0_tiles(int I1, int J1)
 {
     return ((I1 + kD0Tile - 1) / kD0Tile) * ((J1 + kD0Tile - 1) / kD0Tile);
 }
-constexpr int kUpTile = 32;              // k_mg_up0: cells a tile, per side
 constexpr int kGalCells = 64;            // k_mg_galerkin: coarse rows a block, a wave a quarter of each
 constexpr int kVcTile = 16;              // k_mg_pp: level-l cells a block, per side
 constexpr int kRRTile = 7;               // k_mg_rr: level-(l+1) cells a block, per side

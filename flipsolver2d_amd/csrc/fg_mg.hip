@@ -1136,8 +1136,6 @@ __global__ void __launch_bounds__(kBlock) k_mg_post(const SceneDev* scenes, cons
 // neighbours' z0) 8.3 us at 128^2, 10.1 us at 1024^2; an LDS window of whole
 // rows over linear chunks 97 us at 4096^2; this form 4.8, 7.3 and 36 us.
 constexpr int kMaxD1 = 11;               // a code's count (three bits; 4 where materials made it) and four neighbours
-constexpr int kUpR = kUpTile + 2;        // cells a side with the halo
-constexpr int kUpY = kUpTile / 2 + 2;    // level-1 cells a side that the halo's cells prolong from
 static_assert(kUpTile % 2 == 0 && kUpTile * kUpTile % kBlock == 0 && kBlock % kUpTile == 0, "whole rows of a tile a pass");
 
 __global__ void __launch_bounds__(kBlock) k_mg_up0(const SceneDev* scenes, const int2* map, int which)
@@ -1156,9 +1154,8 @@ __global__ void __launch_bounds__(kBlock) k_mg_up0(const SceneDev* scenes, const
     gptr<const float> r = gbl<const float>(which ? s.cr2 : s.cr);
     gptr<const uint8_t> code = gbl<const uint8_t>(s.stencil);
     gptr<float> z = gbl(s.cu);
-    const int tilesJ = (J + kUpTile - 1) / kUpTile, tiles = ((I + kUpTile - 1) / kUpTile) * tilesJ;
-    const int per = (tiles + s.up_blocks - 1) / s.up_blocks;
-    const int t1 = min(tiles, (sb.block + 1) * per);
+    const int tilesJ = up_tiles_j(J);
+    const TileRun run = up_run(up_tiles(I, J), s.up_blocks, sb.block);
     if (threadIdx.x <= kMaxD1) inv[threadIdx.x] = threadIdx.x ? 1.0f / (float)threadIdx.x : 0.f;
     // w x / D1 (0 where D1 is)
     auto over_d = [&](float x, int d) {
@@ -1167,22 +1164,23 @@ __global__ void __launch_bounds__(kBlock) k_mg_up0(const SceneDev* scenes, const
     };
     auto l1 = [](uint8_t k) { return ((k >> 4) & 7) + __popc(k & 15u); };
     double rz = 0.0, rr = 0.0;
-    for (int tile = sb.block * per; tile < t1; tile++) {
-        const int ti = tile / tilesJ, i0 = kUpTile * ti, j0 = kUpTile * (tile - ti * tilesJ);
+    for (int tile = run.first; tile < run.end; tile++) {
+        const TileAt at = up_tile(tile, tilesJ);
         constexpr int Q = (kUpR * kUpR + kBlock - 1) / kBlock, QY = (kUpY * kUpY + kBlock - 1) / kBlock;
         uint8_t kq[Q];
         float vq[Q], yq[QY];
 #pragma unroll
         for (int u = 0; u < Q; u++) {
             const int k = min((int)threadIdx.x + u * kBlock, kUpR * kUpR - 1);
-            const int f = min(max(i0 - 1 + k / kUpR, 0), I - 1) * J + min(max(j0 - 1 + k % kUpR, 0), J - 1);
+            const int f = up_halo(at, k, I, J);
             kq[u] = code[f];
             vq[u] = r[f];
         }
 #pragma unroll
         for (int u = 0; u < QY; u++) {
             const int k = min((int)threadIdx.x + u * kBlock, kUpY * kUpY - 1);
-            const int ci = i0 / 2 - 1 + k / kUpY, cj = j0 / 2 - 1 + k % kUpY;
+            const TileAt y = up_patch(at, k);
+            const int ci = y.i, cj = y.j;
             const bool ok = ci >= 0 && ci < I1 && cj >= 0 && cj < J1;
             yq[u] = y1[min(max(ci, 0), I1 - 1) * J1 + min(max(cj, 0), J1 - 1)] * mask01(ok);
         }
@@ -1205,11 +1203,8 @@ __global__ void __launch_bounds__(kBlock) k_mg_up0(const SceneDev* scenes, const
         for (int u = 0; u < Q; u++) {
             const int k = threadIdx.x + u * kBlock;
             if (k >= kUpR * kUpR) break;
-            const int a = k / kUpR, b = k % kUpR;   // cell (i0 - 1 + a, j0 - 1 + b), i0 and j0 even
-            // prolong_at on the patch, whose first cell is (i0 / 2 - 1, j0 / 2 - 1): an
-            // even cell (odd a) takes its own parent and the one before, an odd one the next
-            const int p0 = (a + 1) >> 1, q0 = (b + 1) >> 1;
-            const int p1 = (a & 1) ? p0 - 1 : p0 + 1, q1 = (b & 1) ? q0 - 1 : q0 + 1;
+            const int a = k / kUpR, b = k % kUpR;
+            const int p0 = up_near(a), q0 = up_near(b), p1 = up_far(a), q1 = up_far(b);   // prolong_at on the patch
             float acc = 0.f;
             acc += (0.75f * 0.75f) * ys[p0][q0];
             acc += (0.75f * 0.25f) * ys[p0][q1];
@@ -1218,10 +1213,10 @@ __global__ void __launch_bounds__(kBlock) k_mg_up0(const SceneDev* scenes, const
             zs[a][b] = over_d(vq[u], l1(kq[u])) + acc;
         }
         __syncthreads();
-        const int b = 1 + (int)threadIdx.x % kUpTile, j = j0 + b - 1;
+        const int b = 1 + (int)threadIdx.x % kUpTile, j = at.j + b - 1;
 #pragma unroll
         for (int u = 0; u < kUpTile * kUpTile / kBlock; u++) {
-            const int a = 1 + (int)threadIdx.x / kUpTile + u * (kBlock / kUpTile), i = i0 + a - 1;
+            const int a = 1 + (int)threadIdx.x / kUpTile + u * (kBlock / kUpTile), i = at.i + a - 1;
             if (i >= I || j >= J) continue;
             const uint8_t k = cs[a][b];
             const float rc = rs[a][b];

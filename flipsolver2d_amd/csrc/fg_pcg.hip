@@ -269,7 +269,7 @@ __device__ __forceinline__ double pcg_row(uint8_t cc, const float (&P)[5])
 // the sums through LDS permutes).
 __global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, const int2* map, int it)
 {
-    constexpr int R = kUpTile + 2;
+    constexpr int R = kUpR;
     __shared__ float ps[R][R + 1];
     const SceneBlock sb = scene_block(map, true);
     const SceneDev& s = scenes[sb.scene];
@@ -284,13 +284,12 @@ __global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, cons
     gptr<float> pnew = gbl((it & 1) ? s.cs1 : s.cp);
     gptr<float> q = gbl<float>(s.cw);
     gptr<const uint8_t> code = gbl<const uint8_t>(s.stencil);
-    const int tilesJ = (J + kUpTile - 1) / kUpTile, tiles = ((I + kUpTile - 1) / kUpTile) * tilesJ;
-    const int per = (tiles + s.up_blocks - 1) / s.up_blocks;
-    const int t0 = sb.block * per, t1 = min(tiles, t0 + per);
+    const int tilesJ = up_tiles_j(J);
+    const TileRun run = up_run(up_tiles(I, J), s.up_blocks, sb.block);
     double pq = 0.0;
     float beta = 0.f;
-    for (int tile = t0; tile < t1; tile++) {
-        const int ti = tile / tilesJ, i0 = kUpTile * ti, j0 = kUpTile * (tile - ti * tilesJ);
+    for (int tile = run.first; tile < run.end; tile++) {
+        const TileAt at = up_tile(tile, tilesJ);
         constexpr int Q = (R * R + kBlock - 1) / kBlock, N = kUpTile * kUpTile / kBlock;
         const int b = (int)threadIdx.x % kUpTile, a0 = (int)threadIdx.x / kUpTile;   // own cells (a0 + u kBlock / kUpTile, b)
         float zq[Q], oq[Q];
@@ -298,14 +297,14 @@ __global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, cons
 #pragma unroll
         for (int u = 0; u < Q; u++) {
             const int k = min((int)threadIdx.x + u * kBlock, R * R - 1);
-            const int f = min(max((i0 - 1 + k / R) * J + (j0 - 1 + k % R), 0), C - 1);
+            const int f = up_halo_linear(at, k, I, J);
             zq[u] = z[f];
             oq[u] = first ? 0.f : pold[f];
         }
 #pragma unroll
         for (int u = 0; u < N; u++)
-            cc[u] = code[min((i0 + a0 + u * (kBlock / kUpTile)) * J + min(j0 + b, J - 1), C - 1)];
-        if (tile == t0) {
+            cc[u] = code[min((at.i + a0 + u * (kBlock / kUpTile)) * J + min(at.j + b, J - 1), C - 1)];
+        if (tile == run.first) {
             // the first tile's loads are on their way before the stop flags are read
 #pragma unroll
             for (int u = 0; u < Q; u++) asm volatile("" : "+v"(zq[u]), "+v"(oq[u]));
@@ -322,7 +321,7 @@ __global__ void __launch_bounds__(kBlock) k_pcg_dir(const SceneDev* scenes, cons
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < N; u++) {
-            const int a = a0 + u * (kBlock / kUpTile), i = i0 + a, j = j0 + b;
+            const int a = a0 + u * (kBlock / kUpTile), i = at.i + a, j = at.j + b;
             if (i >= I || j >= J) continue;
             const float P[5] = {ps[a + 1][b + 1], ps[a][b + 1], ps[a + 2][b + 1], ps[a + 1][b], ps[a + 1][b + 2]};
             const double qd = pcg_row(cc[u], P);
