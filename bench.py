@@ -23,6 +23,10 @@ launch slow the launch pipeline by ~7 %, so the timed frames run without
 them), and `cpu_baseline`: the CPU restatement
 of the reference path (its own PCG, IPP and gated density solve, the
 reference's thread-pool decomposition) on a bounded sample of the workload.
+
+The line holds each leg's results and its dominant kernel (a few KB: a longer
+one would not survive a log's tail); `--details FILE` writes every kernel
+family's table, bytes and launch counts.
 """
 from __future__ import annotations
 
@@ -135,6 +139,7 @@ def parse():
                     help="CPU-baseline budget per solver mode, seconds of timed frames (0: skip)")
     ap.add_argument("--cpu-frames", type=int, default=3, help="frames of each scene in the CPU baseline")
     ap.add_argument("--cpu-threads", type=int, default=0, help="0: min(16, cpu count)")
+    ap.add_argument("--details", default="", help="file for the full results, every kernel family's table included")
     return ap.parse_args()
 
 
@@ -149,6 +154,38 @@ def pctl(v, q):
     pos = q * (len(s) - 1)
     lo, hi = int(pos), min(len(s) - 1, int(pos) + 1)
     return s[lo] + (s[hi] - s[lo]) * (pos - lo)
+
+
+ROOFLINE_KEYS = ("kernel", "bound", "achieved", "peak", "unit", "frac", "traffic_per_algorithmic_byte", "avg_launch_us",
+                 "ms_per_frame")
+DETAIL_KEYS = ("kernels", "algorithmic_bytes_total", "tiling_candidates", "calibration")
+
+
+def brief(x, top=True):
+    """`x` as the line shows it: six digits, no byte totals, of a leg its dominant kernel, and of the headline every kernel
+    family as GB/s and microseconds a launch."""
+    if isinstance(x, float):
+        return float(f"{x:.6g}")
+    if isinstance(x, list):
+        return [brief(v) for v in x]
+    if not isinstance(x, dict):
+        return x
+    out = {}
+    for k, v in x.items():
+        if k == "roofline" and v:
+            out[k] = {q: brief(v[q]) for q in ROOFLINE_KEYS if q in v}
+        elif k == "kernels" and v and top:
+            out[k] = {n: {"gbs": brief(t["achieved"]), "us": brief(t["avg_launch_us"])} for n, t in v.items()}
+        elif k not in DETAIL_KEYS:
+            out[k] = brief(v, False)
+    return out
+
+
+def report(out, a):
+    if a.details:
+        with open(a.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(brief(out), separators=(", ", ": ")), flush=True)
 
 
 class KernelTimer:
@@ -716,8 +753,8 @@ def main():
     if cpu:
         log(f"cpu baseline: {cpu['value']:.3e} particle-substeps/s")
     if b is None:   # a profiling run of other legs: their results alone
-        print(json.dumps({"dam_break_1024": dam, "nbflip_dam_break_1024": nb, "viscous_batch_256": visc,
-                          "isolated_projection": proj, "served": served, "cpu_baseline": cpu}), flush=True)
+        report({"dam_break_1024": dam, "nbflip_dam_break_1024": nb, "viscous_batch_256": visc,
+                "isolated_projection": proj, "served": served, "cpu_baseline": cpu}, a)
         return
 
     dom = b.pop("dominant")
@@ -761,7 +798,7 @@ def main():
         "isolated_projection": proj,
         "served": served,
     }
-    print(json.dumps(out), flush=True)
+    report(out, a)
 
 
 if __name__ == "__main__":
